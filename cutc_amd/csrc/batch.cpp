@@ -32,6 +32,7 @@ struct RankClass {
   ctc_model *model = nullptr;
   uint64_t *seg_train = nullptr, *seg_test = nullptr;  // device, nprob + 1 each
   double *dsum = nullptr;                              // device, 2 * nprob
+  double *dpart = nullptr;                             // device, nprob * kSegBlocks
   bool tuned = false;
   uint32_t tile_len = 0, block = 0;
   hipEvent_t join = nullptr;
@@ -80,6 +81,7 @@ extern "C" void ctc_batch_destroy(ctc_batch *b) {
     if (c.seg_train) (void)hipFree(c.seg_train);
     if (c.seg_test) (void)hipFree(c.seg_test);
     if (c.dsum) (void)hipFree(c.dsum);
+    if (c.dpart) (void)hipFree(c.dpart);
     if (c.join) (void)hipEventDestroy(c.join);
     if (c.ctx) ctc_context_destroy(c.ctx);
   }
@@ -181,7 +183,8 @@ extern "C" ctc_status ctc_batch_create(ctc_context *ctx, uint32_t nproblems, con
     b->total_train += seg_tr[np];
     if (hipMalloc(&c.seg_train, (np + 1) * sizeof(uint64_t)) != hipSuccess ||
         hipMalloc(&c.seg_test, (np + 1) * sizeof(uint64_t)) != hipSuccess ||
-        hipMalloc(&c.dsum, 2 * np * sizeof(double)) != hipSuccess) {
+        hipMalloc(&c.dsum, 2 * np * sizeof(double)) != hipSuccess ||
+        hipMalloc(&c.dpart, np * kSegBlocks * sizeof(double)) != hipSuccess) {
       s = fail(CTC_ERR_NOMEM, "batch segment tables");
       break;
     }
@@ -398,7 +401,10 @@ extern "C" ctc_status ctc_batch_als(ctc_batch *b, const ctc_options *o, uint32_t
 extern "C" ctc_status ctc_batch_rmse(ctc_batch *b, double *rmse_tr, double *rmse_te) {
   if (!b) return fail(CTC_ERR_INVALID_ARG, "ctc_batch_rmse");
   CTC_HIP(hipSetDevice(b->ctx->device));
-  for (auto &c : b->cls) {
+  // every class is enqueued on its own stream before the first is waited for
+  std::vector<std::vector<double>> sums(b->cls.size());
+  for (size_t ci = 0; ci < b->cls.size(); ++ci) {
+    RankClass &c = b->cls[ci];
     ctc_model *m = c.model;
     const uint32_t np = (uint32_t)c.problems.size();
     hipStream_t st = c.ctx->stream;
@@ -410,13 +416,20 @@ extern "C" ctc_status ctc_batch_rmse(ctc_batch *b, double *rmse_tr, double *rmse
     ct.nnz = m->test.nnz;
     FactorArgs fa{};
     for (uint32_t md = 0; md < m->nmodes; ++md) fa.f[md] = m->F[md];
-    CTC_HIP(launch_eval_seg(st, &ca, nullptr, fa, (int)m->nmodes, (int)c.rank, c.seg_train, np, c.dsum));
+    CTC_HIP(launch_eval_seg(st, &ca, nullptr, fa, (int)m->nmodes, (int)c.rank, c.seg_train, np, c.dpart,
+                            c.dsum));
     if (m->test.nnz)
-      CTC_HIP(launch_eval_seg(st, nullptr, &ct, fa, (int)m->nmodes, (int)c.rank, c.seg_test, np, c.dsum + np));
-    std::vector<double> h(2 * (size_t)np, 0.0);
-    CTC_HIP(hipMemcpyAsync(h.data(), c.dsum, (m->test.nnz ? 2 : 1) * np * sizeof(double), hipMemcpyDeviceToHost,
-                           st));
-    CTC_HIP(hipStreamSynchronize(st));
+      CTC_HIP(launch_eval_seg(st, nullptr, &ct, fa, (int)m->nmodes, (int)c.rank, c.seg_test, np, c.dpart,
+                              c.dsum + np));
+    sums[ci].assign(2 * (size_t)np, 0.0);
+  }
+  for (size_t ci = 0; ci < b->cls.size(); ++ci) {
+    RankClass &c = b->cls[ci];
+    const uint32_t np = (uint32_t)c.problems.size();
+    std::vector<double> &h = sums[ci];
+    CTC_HIP(hipMemcpyAsync(h.data(), c.dsum, (c.model->test.nnz ? 2 : 1) * np * sizeof(double),
+                           hipMemcpyDeviceToHost, c.ctx->stream));
+    CTC_HIP(hipStreamSynchronize(c.ctx->stream));
     for (uint32_t k = 0; k < np; ++k) {
       const Placement &pl = b->place[c.problems[k]];
       if (rmse_tr) rmse_tr[c.problems[k]] = pl.ntrain ? std::sqrt(h[k] / (double)pl.ntrain) : 0.0;

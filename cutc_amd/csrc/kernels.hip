@@ -1299,17 +1299,25 @@ __global__ void __launch_bounds__(256) k_eval_coo(CooArgs c, FactorArgs fa, int 
   block_store_sum(acc, part + blockIdx.x);
 }
 
-// squared error per segment [seg[b], seg[b+1]) of the nonzeros, one block per
-// segment (a segment = one problem of a batch); CISS=true reads mode-0 CISS
-// order, false a COO
-template <int N, bool CISS>
-__global__ void __launch_bounds__(256) k_eval_seg(CissArgs c, CooArgs co, FactorArgs fa, int R,
-                                                  const uint64_t *seg, double *out) {
+// Squared error per segment [seg[b], seg[b+1]) of the nonzeros (a segment = one
+// problem of a batch): gridDim.y blocks per segment, each leaving one partial,
+// part[b * gridDim.y + y].  CISS=true reads mode-0 CISS order, false a COO.
+// Bound by the row gathers.  Walkers of R / 4 lanes move a row as one 16-byte
+// load per lane, the walkers of a segment's blocks take its nonzeros in turn,
+// and the FP32 prediction is summed over the walker's lanes.  Few segments are the
+// common case, so a segment is shared by kSegBlocks blocks: with one block per
+// segment and a lane per nonzero, 24 problems of 0.3M nonzeros (six per rank)
+// took 24 ms of an 80 ms pass of ten iterations; this way the pass takes 56 ms.
+template <int R, int N, bool CISS>
+__global__ void __launch_bounds__(256) k_eval_seg(CissArgs c, CooArgs co, FactorArgs fa, const uint64_t *seg,
+                                                  double *part) {
+  constexpr int W = SyncShape<R>::W, CPL = SyncShape<R>::CPL, NW = 256 / W;
+  const int wl = threadIdx.x % W;
   double acc = 0.0;
-  const float *F[4] = {fa.f[0], fa.f[1], fa.f[2], fa.f[3]};
   const uint64_t p1 = seg[blockIdx.x + 1];
-  for (uint64_t p = seg[blockIdx.x] + threadIdx.x; p < p1; p += blockDim.x) {
-    uint32_t ix[4];
+  const uint64_t G = (uint64_t)gridDim.y * NW;
+  for (uint64_t p = seg[blockIdx.x] + (uint64_t)blockIdx.y * NW + threadIdx.x / W; p < p1; p += G) {
+    uint32_t ix[N];
     float x;
     if (CISS) {
       const uint64_t t = p >> 6;
@@ -1322,10 +1330,19 @@ __global__ void __launch_bounds__(256) k_eval_seg(CissArgs c, CooArgs co, Factor
       for (int m = 0; m < N; ++m) ix[m] = co.ind[m][p];
       x = co.vals[p];
     }
-    const double e = (double)x - (double)predict_row<N>(F, ix, R);
-    acc += e * e;
+    float h[CPL];
+    load_row4<CPL>(fa.f[0] + (size_t)ix[0] * R + wl * CPL, h);
+#pragma unroll
+    for (int m = 1; m < N; ++m) {
+      float g[CPL];
+      load_row4<CPL>(fa.f[m] + (size_t)ix[m] * R + wl * CPL, g);
+#pragma unroll
+      for (int j = 0; j < CPL; ++j) h[j] *= g[j];
+    }
+    const double e = (double)x - (double)group_sum<W>((h[0] + h[1]) + (h[2] + h[3]));
+    if (wl == 0) acc += e * e;
   }
-  block_store_sum(acc, out + blockIdx.x);
+  block_store_sum(acc, part + (size_t)blockIdx.x * gridDim.y + blockIdx.y);
 }
 
 __global__ void __launch_bounds__(256) k_sumsq(const float *x, uint64_t n, double *part) {
@@ -1655,16 +1672,19 @@ hipError_t launch_eval_coo(hipStream_t st, const CooArgs &c, const FactorArgs &f
 }
 
 hipError_t launch_eval_seg(hipStream_t st, const CissArgs *c, const CooArgs *co, const FactorArgs &f,
-                           int nmodes, int R, const uint64_t *seg, uint32_t nseg, double *out) {
+                           int nmodes, int R, const uint64_t *seg, uint32_t nseg, double *part, double *out) {
   if (nseg == 0) return hipSuccess;
   const CissArgs ca = c ? *c : CissArgs{};
   const CooArgs cb = co ? *co : CooArgs{};
-#define CTC_SEG(NN)                                                                                    \
-  do {                                                                                                \
-    if (c)                                                                                            \
-      hipLaunchKernelGGL((k_eval_seg<NN, true>), dim3(nseg), dim3(256), 0, st, ca, cb, f, R, seg, out);  \
-    else                                                                                              \
-      hipLaunchKernelGGL((k_eval_seg<NN, false>), dim3(nseg), dim3(256), 0, st, ca, cb, f, R, seg, out); \
+#define CTC_SEG(NN)                                                                                        \
+  do {                                                                                                     \
+    if (c) {                                                                                               \
+      CTC_R_SWITCH(R, hipLaunchKernelGGL((k_eval_seg<RR, NN, true>), dim3(nseg, kSegBlocks), dim3(256), 0, \
+                                         st, ca, cb, f, seg, part));                                       \
+    } else {                                                                                               \
+      CTC_R_SWITCH(R, hipLaunchKernelGGL((k_eval_seg<RR, NN, false>), dim3(nseg, kSegBlocks), dim3(256), 0, \
+                                         st, ca, cb, f, seg, part));                                       \
+    }                                                                                                      \
   } while (0)
   if (nmodes == 3)
     CTC_SEG(3);
@@ -1673,7 +1693,8 @@ hipError_t launch_eval_seg(hipStream_t st, const CissArgs *c, const CooArgs *co,
   else
     return hipErrorInvalidValue;
 #undef CTC_SEG
-  return hipGetLastError();
+  const hipError_t e = hipGetLastError();
+  return e != hipSuccess ? e : launch_reduce_parts(st, part, kSegBlocks, nseg, out);
 }
 
 hipError_t launch_sumsq(hipStream_t st, const float *x, uint64_t n, unsigned nblocks, double *part) {

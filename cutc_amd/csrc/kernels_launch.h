@@ -44,9 +44,12 @@ hipError_t launch_als_solve(hipStream_t st, const double *pieces, const uint32_t
                             double lam, bool refine, bool light, float *A, uint32_t *flag);
 hipError_t launch_eval_coo(hipStream_t st, const CooArgs &c, const FactorArgs &f, int nmodes, int R,
                            unsigned nblocks, double *part);
-// per-segment squared error: exactly one of c (mode-0 CISS order) / co (COO) is non-null
+// per-segment squared error: exactly one of c (mode-0 CISS order) / co (COO) is
+// non-null.  Each segment is shared by kSegBlocks blocks, whose partials
+// (part: nseg x kSegBlocks) are added in order into out[segment].
+constexpr unsigned kSegBlocks = 64;
 hipError_t launch_eval_seg(hipStream_t st, const CissArgs *c, const CooArgs *co, const FactorArgs &f,
-                           int nmodes, int R, const uint64_t *seg, uint32_t nseg, double *out);
+                           int nmodes, int R, const uint64_t *seg, uint32_t nseg, double *part, double *out);
 hipError_t launch_sumsq(hipStream_t st, const float *x, uint64_t n, unsigned nblocks, double *part);
 hipError_t launch_reduce_parts(hipStream_t st, const double *part, uint32_t nb, uint32_t groups,
                                double *out);
