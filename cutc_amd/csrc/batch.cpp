@@ -265,11 +265,10 @@ static ctc_options class_options(const RankClass &c, const ctc_options *o) {
 static ctc_status prepare_class(RankClass &c, const ctc_options *t) {
   ctc_model *m = c.model;
   if (als_uses_rows(t, c.rank)) return als_rows_prepare(m, t, t->precision == CTC_PREC_MIXED);
-  const uint32_t S = span_tiles_of(t);
   size_t need = 0;
   for (uint32_t md = 0; md < m->nmodes; ++md) {
     CTC_TRY(ensure_ciss(m, md));
-    CTC_TRY(ensure_pieces(m, md, S));
+    CTC_TRY(ensure_pieces(m, md, als_span_tiles(t, m->ciss[md].nnz)));
     const DevCiss &d = m->ciss[md];
     need = std::max(need, (size_t)(d.npieces + d.ngroups) * ((size_t)c.rank * c.rank + c.rank) * sizeof(double));
   }

@@ -76,7 +76,7 @@ struct DevCiss {
   uint32_t *span_off = nullptr;  // nspans: piece id = slot + span_off[span]
   uint32_t *slot_pb = nullptr;   // dlength + 1: pieces of slot s
   // heavy slots (more than kHeavyPieces pieces): their pieces are summed in
-  // groups of kGroupPieces consecutive pieces before the ALS solve
+  // groups of consecutive pieces before the ALS solve
   uint64_t ngroups = 0;
   uint32_t *grp_piece = nullptr;  // ngroups: first piece of group g
   uint32_t *grp_n = nullptr;      // ngroups: pieces in group g

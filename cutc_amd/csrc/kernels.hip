@@ -1020,23 +1020,31 @@ __device__ inline int tri_row(int t) {
   return a;
 }
 
-// Heavy slots (more pieces than fit one workgroup's serial sum) are first
-// reduced in fixed groups of consecutive pieces, one workgroup per group, so
-// the solve sums a handful of group sums instead of thousands of pieces.
+// Heavy slots (more pieces than the solve's serial sum should take) are first
+// reduced in fixed groups of consecutive pieces.  A thread owns one element of
+// a group's sum (blockIdx.y: 256 elements of the piece), eight pieces' loads in
+// flight, added in piece order: 20M nonzeros at R = 32, 32 us
+// per mode (218 us with one 64-thread workgroup per group and a load at a time).
 template <int R>
-__global__ void __launch_bounds__(64) k_piece_reduce(const double *pieces, const uint32_t *grp_piece,
-                                                     const uint32_t *grp_n, uint64_t ngroups, double *gsum) {
-  constexpr size_t PSZ = (size_t)R * R + R;
+__global__ void __launch_bounds__(256) k_piece_reduce(const double *pieces, const uint32_t *grp_piece,
+                                                      const uint32_t *grp_n, double *gsum) {
+  constexpr uint32_t PSZ = R * R + R;
+  const uint32_t e = blockIdx.y * 256 + threadIdx.x;
+  if (e >= PSZ) return;
   const uint64_t g = blockIdx.x;
-  if (g >= ngroups) return;
-  const double *P = pieces + (size_t)grp_piece[g] * PSZ;
+  const double *P = pieces + (size_t)grp_piece[g] * PSZ + e;
   const uint32_t n = grp_n[g];
-  double *out = gsum + g * PSZ;
-  for (size_t e = threadIdx.x; e < PSZ; e += 64) {
-    double acc = 0.0;
-    for (uint32_t q = 0; q < n; ++q) acc += P[(size_t)q * PSZ + e];
-    out[e] = acc;
+  double acc = 0.0;
+  uint32_t q = 0;
+  for (; q + 8 <= n; q += 8) {
+    double x[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) x[u] = P[(size_t)(q + u) * PSZ];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) acc += x[u];
   }
+  for (; q < n; ++q) acc += P[(size_t)q * PSZ];
+  gsum[g * PSZ + e] = acc;
 }
 
 template <int R, bool REFINE>
@@ -1194,6 +1202,7 @@ __global__ void __launch_bounds__(256) k_als_solve_h(const double *pieces, const
       p1 = slot_gb[s + 1];
       src = gsum;
     }
+#pragma unroll 1
     for (uint32_t p = p0; p < p1; ++p) {
       const double *P = src + (size_t)p * PSZ;
       // rows i < c are above the diagonal: don't-care (inside the piece, never used)
@@ -1612,25 +1621,28 @@ hipError_t launch_als_gram(hipStream_t st, const CissArgs &c, const FactorArgs &
 hipError_t launch_piece_reduce(hipStream_t st, const double *pieces, const uint32_t *grp_piece,
                                const uint32_t *grp_n, uint64_t ngroups, int R, double *gsum) {
   if (ngroups == 0) return hipSuccess;
-  const unsigned grid = (unsigned)ngroups;
+#define CTC_REDUCE(RR)                                                                                               \
+  case RR:                                                                                                           \
+    hipLaunchKernelGGL((k_piece_reduce<RR>), dim3((unsigned)ngroups, (RR * RR + RR + 255) / 256), dim3(256), 0, st, \
+                       pieces, grp_piece, grp_n, gsum);                                                              \
+    break
   switch (R) {
-    case 8: hipLaunchKernelGGL((k_piece_reduce<8>), dim3(grid), dim3(64), 0, st, pieces, grp_piece, grp_n, ngroups, gsum); break;
-    case 16: hipLaunchKernelGGL((k_piece_reduce<16>), dim3(grid), dim3(64), 0, st, pieces, grp_piece, grp_n, ngroups, gsum); break;
-    case 32: hipLaunchKernelGGL((k_piece_reduce<32>), dim3(grid), dim3(64), 0, st, pieces, grp_piece, grp_n, ngroups, gsum); break;
-    case 64: hipLaunchKernelGGL((k_piece_reduce<64>), dim3(grid), dim3(64), 0, st, pieces, grp_piece, grp_n, ngroups, gsum); break;
+    CTC_REDUCE(8);
+    CTC_REDUCE(16);
+    CTC_REDUCE(32);
+    CTC_REDUCE(64);
     default: return hipErrorInvalidValue;
   }
+#undef CTC_REDUCE
   return hipGetLastError();
 }
 
 hipError_t launch_als_solve(hipStream_t st, const double *pieces, const uint32_t *slot_pb, const double *gsum,
                             const uint32_t *slot_gb, const uint32_t *directory, uint64_t dlength, int R,
-                            double lam, bool refine, bool light, float *A, uint32_t *flag) {
+                            double lam, bool refine, float *A, uint32_t *flag) {
   if (dlength == 0) return hipSuccess;
   const unsigned grid = (unsigned)dlength;
-  // light: few pieces per slot (short rows), where the per-slot factorisation
-  // dominates; slots that sum many pieces keep the 64-lane summation
-  if (!refine && light && R <= 32) {
+  if (!refine && R <= 32) {
     const unsigned g8 = (unsigned)((dlength + 7) / 8);
     switch (R) {
       case 8: hipLaunchKernelGGL((k_als_solve_h<8>), dim3(g8), dim3(256), 0, st, pieces, slot_pb, gsum, slot_gb, directory, dlength, lam, A, flag); break;
@@ -1649,10 +1661,10 @@ hipError_t launch_als_solve(hipStream_t st, const double *pieces, const uint32_t
       hipLaunchKernelGGL((k_als_solve<RR, false>), dim3(grid), dim3(64), 0, st, pieces, slot_pb, gsum,     \
                          slot_gb, directory, dlength, lam, A, flag);                                        \
   } while (0)
-  switch (R) {
-    case 8: CTC_SOLVE(8); break;
-    case 16: CTC_SOLVE(16); break;
-    case 32: CTC_SOLVE(32); break;
+  switch (R) {  // without refinement only rank 64 comes here
+    case 8: hipLaunchKernelGGL((k_als_solve<8, true>), dim3(grid), dim3(64), 0, st, pieces, slot_pb, gsum, slot_gb, directory, dlength, lam, A, flag); break;
+    case 16: hipLaunchKernelGGL((k_als_solve<16, true>), dim3(grid), dim3(64), 0, st, pieces, slot_pb, gsum, slot_gb, directory, dlength, lam, A, flag); break;
+    case 32: hipLaunchKernelGGL((k_als_solve<32, true>), dim3(grid), dim3(64), 0, st, pieces, slot_pb, gsum, slot_gb, directory, dlength, lam, A, flag); break;
     case 64: CTC_SOLVE(64); break;
     default: return hipErrorInvalidValue;
   }

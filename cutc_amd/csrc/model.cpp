@@ -209,16 +209,18 @@ ctc_status ensure_pieces(ctc_model *m, uint32_t mode, uint32_t span_tiles) {
     pb[s] = (uint32_t)(s + off[w]);
   }
   pb[d.dlength] = (uint32_t)base;
-  // group tables for heavy slots
-  constexpr uint32_t kHeavyPieces = 64, kGroupPieces = 32;
+  // group tables for heavy slots: about as many groups as pieces per group, so
+  // that the reduction and the solve each add the square root of the pieces
+  constexpr uint32_t kHeavyPieces = 8;
   std::vector<uint32_t> gpiece, gn, gb(d.dlength + 1);
   for (uint64_t s = 0; s < d.dlength; ++s) {
     gb[s] = (uint32_t)gpiece.size();
     const uint32_t n = pb[s + 1] - pb[s];
     if (n <= kHeavyPieces) continue;
-    for (uint32_t q = 0; q < n; q += kGroupPieces) {
+    const uint32_t per = std::max(kHeavyPieces, (uint32_t)std::ceil(std::sqrt((double)n)));
+    for (uint32_t q = 0; q < n; q += per) {
       gpiece.push_back(pb[s] + q);
-      gn.push_back(std::min(kGroupPieces, n - q));
+      gn.push_back(std::min(per, n - q));
     }
   }
   gb[d.dlength] = (uint32_t)gpiece.size();
@@ -575,7 +577,7 @@ extern "C" ctc_status ctc_model_prepare(ctc_model *m, const ctc_options *o) {
     return als_rows_prepare(m, o, o->precision == CTC_PREC_MIXED);
   for (uint32_t md = 0; md < m->nmodes; ++md) {
     CTC_TRY(ensure_ciss(m, md));
-    if (o->algorithm == CTC_ALS) CTC_TRY(ensure_pieces(m, md, span_tiles_of(o)));
+    if (o->algorithm == CTC_ALS) CTC_TRY(ensure_pieces(m, md, als_span_tiles(o, m->ciss[md].nnz)));
   }
   return CTC_OK;
 }
@@ -587,8 +589,8 @@ static ctc_status als_mode_plain(ctc_model *m, uint32_t mode, const ctc_options 
   const uint32_t R = m->rank;
   if (als_uses_rows(o, R)) return als_mode_rows(m, mode, o, o->precision == CTC_PREC_MIXED);
   if (R > 64) return fail(CTC_ERR_UNSUPPORTED, "the span ALS kernels support ranks up to 64 (got %u)", R);
-  const uint32_t S = span_tiles_of(o);
   CTC_TRY(ensure_ciss(m, mode));
+  const uint32_t S = als_span_tiles(o, m->ciss[mode].nnz);
   CTC_TRY(ensure_pieces(m, mode, S));
   DevCiss &d = m->ciss[mode];
   const size_t psz = (size_t)R * R + R;
@@ -603,8 +605,9 @@ static ctc_status als_mode_plain(ctc_model *m, uint32_t mode, const ctc_options 
     CTC_HIP(launch_als_gram(st, ca, fa, (int)m->nmodes, (int)R, S, d.nspans, d.span_off, pieces,
                             block_of(o)));
   }
-  // rows absent from the directory become 0 (SG/als.cu:699 zeroes the factor)
-  CTC_HIP(launch_fill(st, m->F[mode], m->dims[mode] * R, 0.f));
+  // rows absent from the directory become 0 (SG/als.cu:699 zeroes the factor);
+  // the solve writes every other row
+  if (d.dlength < m->dims[mode]) CTC_HIP(launch_fill(st, m->F[mode], m->dims[mode] * R, 0.f));
   if (d.ngroups) {
     Prof p(m->ctx, "als_reduce");
     CTC_HIP(launch_piece_reduce(st, pieces, d.grp_piece, d.grp_n, d.ngroups, (int)R, gsum));
@@ -612,8 +615,7 @@ static ctc_status als_mode_plain(ctc_model *m, uint32_t mode, const ctc_options 
   {
     Prof p(m->ctx, "als_solve");
     CTC_HIP(launch_als_solve(st, pieces, d.slot_pb, d.ngroups ? gsum : nullptr, d.slot_gb, d.directory,
-                             d.dlength, (int)R, o->lambda, o->refine != 0, d.npieces <= 2 * d.dlength, m->F[mode],
-                             m->dflag));
+                             d.dlength, (int)R, o->lambda, o->refine != 0, m->F[mode], m->dflag));
   }
   m->resid_valid = false;
   return CTC_OK;

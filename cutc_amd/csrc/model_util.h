@@ -36,6 +36,19 @@ inline uint32_t span_tiles_of(const ctc_options *o) {
   return tl / 64;
 }
 
+// tiles per span of the ALS span kernels over nnz nonzeros.  An asked-for
+// tile_len stands; the default shrinks the span until the walk has about
+// kSpanWaves waves, because a span is one wave's serial chain.
+// k_als_gram at R = 16 with spans of 1024 nonzeros and by this rule: 20K
+// nonzeros 78 -> 8 us, 1M nonzeros 74 -> 28 us; from 8.4M nonzeros on the span is 1024.
+constexpr uint64_t kSpanWaves = 8192;
+inline uint32_t als_span_tiles(const ctc_options *o, uint64_t nnz) {
+  const uint32_t most = span_tiles_of(o);
+  if (o && o->tile_len) return most;
+  const uint64_t ntiles = (nnz + kTile - 1) / kTile;
+  return (uint32_t)std::min<uint64_t>(most, std::max<uint64_t>(1, ntiles / kSpanWaves));
+}
+
 inline unsigned block_of(const ctc_options *o) {
   unsigned b = o && o->block ? o->block : 256;
   if (b < 64) b = 64;

@@ -58,3 +58,41 @@ def test_batch_rmse_of_segments(ctx, dims):
     tr, te = b.rmse()
     np.testing.assert_allclose(tr, [w[1] for w in want], rtol=1e-6, atol=4e-6)
     np.testing.assert_allclose(te, [w[2] for w in want], rtol=1e-6, atol=4e-6)
+
+
+def ridge(ind, vals, F, mode, lam):
+    h = np.ones((len(vals), F[0].shape[1]))
+    for m, f in enumerate(F):
+        if m != mode:
+            h *= f.astype(np.float64)[ind[m]]
+    out = np.zeros_like(F[mode], dtype=np.float64)
+    for r in np.unique(ind[mode]):
+        s = ind[mode] == r
+        out[r] = np.linalg.solve(h[s].T @ h[s] + lam * np.eye(h.shape[1]), h[s].T @ vals[s])
+    return out
+
+
+@pytest.mark.parametrize("R,refine", [(8, 0), (16, 0), (32, 0), (16, 1), (64, 0)])
+@pytest.mark.parametrize("dims,nnz", [((1, 40, 30), 1000), ((9, 60, 50), 20000), ((300, 7, 30), 20000),
+                                      ((40, 3, 20, 15), 9000)], ids=["one_row", "long", "mixed", "4way"])
+def test_als_default_spans(ctx, dims, nnz, R, refine):
+    """ALS with the default span over rows of 1 to 300 pieces (eight and fewer
+    are summed by the solve, more in groups), rows without nonzeros in the
+    middle, against the ridge solutions in 64 bits, at the bar of the parity
+    tests (1e-5)."""
+    say(f"[als default spans] dims={dims} nnz={nnz} R={R} refine={refine}")
+    t, ind, vals = coo(dims, nnz - nnz // 10, 3)
+    if dims[0] > 2:  # a row without nonzeros
+        keep = ind[0] != 1
+        ind, vals = [i[keep] for i in ind], vals[keep]
+        t = ct.Coo.from_arrays(ind, vals, dims)
+    rng = np.random.default_rng(8)
+    F = [rng.uniform(-1, 1, (d, R)).astype(np.float32) for d in dims]
+    m = ct.Model(ctx, t, None, None, rank=R)
+    opt = ct.Options(algorithm=ct.ALS, rank=R, lambda_=0.5, refine=refine, als_kernel=ct.ALS_SPANS)
+    for mode in range(len(dims)):
+        m.set_factors(F)
+        m.als_mode_update(mode, opt)
+        want = ridge(ind, vals, F, mode, 0.5)
+        e = np.linalg.norm(m.factor(mode) - want) / np.linalg.norm(want)
+        assert e < 1e-5, (mode, e)
