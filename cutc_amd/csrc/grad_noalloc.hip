@@ -21,7 +21,7 @@ namespace {
 // blocks: 1 MiB
 constexpr uint64_t kGradMaxBlocks = 16384;
 constexpr uint64_t kGradScratchDoubles = 2 * CTC_MAX_MODES * kGradMaxBlocks + 2 * CTC_MAX_MODES;
-constexpr unsigned kRegBlocks = 512;
+constexpr unsigned kRegBlocks = 2048;
 constexpr int kMaxDevices = 64;
 
 static __device__ __align__(256) double scratch[kGradScratchDoubles];
@@ -77,7 +77,7 @@ extern "C" ctc_status ctc_grad_noalloc(ctc_model *m, const float *const *factors
   // walkers of `span` nonzeros, span chosen so that each walk has at most
   // kGradMaxBlocks blocks of partial sums
   const uint64_t per_block = mttkrp_walkers_per_block((int)R, 256);
-  uint64_t span = 256;
+  uint64_t span = walk_span(m->train_nnz, (int)R);
   while ((m->train_nnz + span - 1) / span > kGradMaxBlocks * per_block) span *= 2;
   const uint64_t nb = std::max<uint64_t>(mttkrp_grid(m->train_nnz, (int)R, (uint32_t)span, 256), kRegBlocks);
   if (nb > kGradMaxBlocks || 2 * N * nb + 2 * N > kGradScratchDoubles)
@@ -87,14 +87,14 @@ extern "C" ctc_status ctc_grad_noalloc(ctc_model *m, const float *const *factors
   // unused tails of the walk groups must read as zero: fill kernel, no memset
   CTC_HIP(launch_fill(st, (float *)part, 2 * (2 * N * nb), 0.f));
   for (uint32_t md = 0; md < N; ++md) {
-    CTC_HIP(launch_fill(st, grads[md], m->dims[md] * R, 0.f));
-    unsigned grid = 0;
-    CTC_HIP(launch_mttkrp(st, ciss_args(m->ciss[md]), rel_factors(F, N, md), (int)N, (int)R, (uint32_t)span, true,
-                          grads[md], part + (size_t)md * nb, &grid, 256));
     const DevCiss &d = m->ciss[md];
     const uint64_t nrows = reg_per_occurrence ? d.dlength : m->dims[md];
+    if (reg_per_occurrence && d.dlength < m->dims[md]) CTC_HIP(launch_fill(st, grads[md], m->dims[md] * R, 0.f));
     CTC_HIP(launch_reg_rows(st, d.directory, d.rowptr, nrows, (int)R, (float)lambda, reg_per_occurrence, F[md],
                             grads[md], kRegBlocks, part + (size_t)(N + md) * nb));
+    unsigned grid = 0;
+    CTC_HIP(launch_mttkrp(st, ciss_args(d), rel_factors(F, N, md), (int)N, (int)R, (uint32_t)span, true, grads[md],
+                          part + (size_t)md * nb, &grid, 256, (float)lambda, reg_per_occurrence));
   }
   CTC_HIP(launch_reduce_parts(st, part, (uint32_t)nb, 2 * N, sums));
   if (loss_device) {

@@ -715,19 +715,31 @@ __global__ void __launch_bounds__(256) k_sgd_fold(SettleArgs a) {
 // h = hadamard of the other modes' rows and
 //   w = x                       (kWalkMttkrp: SG/als.cu:295-312 intent), or
 //   w = x - <F_mode(row), h>    (kWalkAdjoint, kWalkJacobi: the residual).
-// Rows may span walkers, so each walker adds its partial row with atomics
-// into a zeroed output.  For the adjoint, out receives -acc and loss_part
-// the per-block sum of squared residuals.  kWalkJacobi is the reference's
-// CCD sums (SG/ccd.cu:157-195): out receives acc = sum e h and den the
-// sum of h * h, per column, all from the factors as they were at launch.
-// kWalkLoss only sums the squared residuals into loss_part (the training
-// loss of tc_loss_sq, SG/completion.c:166-189).
+// A row that starts and ends inside a walker's span is stored.  The rows open
+// at the ends of the spans (a walker's first, where it continues, and its
+// last) are first joined in LDS along the workgroup's walkers, whose spans are
+// consecutive, and each joined row is added with one atomic per entry into the
+// initialised output.  A hot row so costs one atomic row per workgroup: one
+// per walker queued on the row's memory channel for longer than the walk took.
+// For the adjoint, out holds lambda c F (c = the row's nonzeros or 1) and
+// receives -acc, and loss_part the per-block sum of squared residuals.
+// kWalkJacobi is the reference's CCD sums (SG/ccd.cu:157-195): out receives
+// acc = sum e h and den the sum of h * h, per column, all from the factors as
+// they were at launch.  kWalkLoss only sums the squared residuals into
+// loss_part (the training loss of tc_loss_sq, SG/completion.c:166-189).
+// Bound by the gathers of the other modes' rows: the rows of four nonzeros are
+// gathered together, the next chunk's indices one chunk ahead (44 registers at
+// N = 3).  MTTKRP of 8M nonzeros at R = 32 117 us per mode, 2.1 times the
+// indices, values and rows a CU can take from its cache at 64 B per clock; with
+// an atomic row per walker and row 260 us, 283 us with the gathers in fours
+// alone.  Two or eight nonzeros at a time: 123 / 134 us.  The adjoint of 20M
+// nonzeros of a 4-way tensor: 510 us per mode (1100 us).
 // ==========================================================================
 enum : int { kWalkMttkrp = 0, kWalkAdjoint = 1, kWalkJacobi = 2, kWalkLoss = 3 };
 
 template <int R, int N, int KIND>
-__global__ void __launch_bounds__(256) k_mttkrp(CissArgs c, FactorArgs fa, uint32_t span,
-                                                float *out, double *loss_part, float *den) {
+__global__ void __launch_bounds__(256) k_mttkrp(CissArgs c, FactorArgs fa, uint32_t span, float *out,
+                                                double *loss_part, float *den, float lam, int per_occ) {
   constexpr bool ADJ = KIND != kWalkMttkrp;  // w is the residual
   constexpr bool SQ = KIND == kWalkJacobi;
   // a walker is R / 4 lanes, each holding 4 consecutive entries of a row, so
@@ -737,10 +749,15 @@ __global__ void __launch_bounds__(256) k_mttkrp(CissArgs c, FactorArgs fa, uint3
   constexpr int CPL = SyncShape<R>::CPL;
   constexpr int WPW = SyncShape<R>::WPW;
   constexpr uint32_t NONE = 0xFFFFFFFFu;
+  constexpr int NWK = 256 / W;  // walkers of a workgroup, and the open rows they leave: first, last
+  constexpr bool SUMS = KIND != kWalkLoss;
   __shared__ double red[4];
+  __shared__ float open_s[SUMS ? 2 * NWK : 1][R], open_q[SQ ? 2 * NWK : 1][R];
+  __shared__ uint32_t open_id[2 * NWK];
   const int lane = lane_id();
   const int sub = lane / W;
   const int wl = lane % W;
+  const int wk = threadIdx.x / W;
   const uint64_t wave = (uint64_t)blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
   const uint64_t walker = wave * WPW + sub;
   const uint64_t s0 = walker * span;
@@ -749,85 +766,156 @@ __global__ void __launch_bounds__(256) k_mttkrp(CissArgs c, FactorArgs fa, uint3
 
   float acc[CPL], own[CPL], sq[CPL];
   double lsum = 0.0;
-  uint32_t arow = NONE, slot = 0;
+  uint32_t arow = NONE, cnt = 0;
+  bool cont = false;  // the open row began before this span
+  if (SUMS && wl == 0) open_id[2 * wk] = open_id[2 * wk + 1] = NONE;
 #pragma unroll
   for (int q = 0; q < CPL; ++q) acc[q] = 0.f, own[q] = 0.f, sq[q] = 0.f;
   constexpr bool LOSS = KIND == kWalkAdjoint || KIND == kWalkLoss;  // the squared residuals are summed
-  auto flush = [&]() {
-    if (KIND == kWalkLoss) return;
-    float *o = out + (size_t)arow * R + wl * CPL;
-#pragma unroll
-    for (int q2 = 0; q2 < CPL; ++q2) {
-      atomic_add_f32(o + q2, KIND == kWalkAdjoint ? -acc[q2] : acc[q2]);
-      if (SQ) atomic_add_f32(den + (size_t)arow * R + wl * CPL + q2, sq[q2]);
+  constexpr int B = W < 4 ? W : 4;  // nonzeros whose rows are gathered together
+  auto leave_open = [&](int e) {
+    if (wl == 0) open_id[e] = arow;
+    store_row4<CPL>(&open_s[SUMS ? e : 0][wl * CPL], acc);
+    if (SQ) store_row4<CPL>(&open_q[SQ ? e : 0][wl * CPL], sq);
+  };
+  auto end_row = [&]() {  // a row that ends inside the span
+    if (!SUMS) return;
+    if (cont) {
+      leave_open(2 * wk);
+      cont = false;
+      return;
     }
+    float v[CPL];
+    const float reg = lam * (per_occ ? (float)cnt : 1.f);
+#pragma unroll
+    for (int q2 = 0; q2 < CPL; ++q2) v[q2] = KIND == kWalkAdjoint ? reg * own[q2] - acc[q2] : acc[q2];
+    store_row4<CPL>(out + (size_t)arow * R + wl * CPL, v);
+    if (SQ) store_row4<CPL>(den + (size_t)arow * R + wl * CPL, sq);
   };
 
   if (!wave_idle) {
+    // the next chunk's indices, value and tile word of this lane's nonzero
+    uint32_t in[N - 1], tsn = 0;
+    float xn = 0.f;
+    uint64_t mn = 0;
+    auto fetch = [&](uint32_t ch) {
+      const uint64_t el = s0 + ch + wl;
+#pragma unroll
+      for (int s = 0; s < N - 1; ++s) in[s] = 0;
+      if (ch < span && el < s1) {
+#pragma unroll
+        for (int s = 0; s < N - 1; ++s) in[s] = c.oidx[s][el];
+        xn = c.vals[el];
+        mn = c.tile_mask[el >> 6];
+        tsn = c.tile_slot[el >> 6];
+      }
+    };
+    fetch(0);
     for (uint32_t ch = 0; ch < span; ch += W) {
       const uint64_t el = s0 + ch + wl;
-      const bool vl = el < s1;
-      uint32_t il[N - 1];
-      float xl = 0.f;
+      uint32_t il[N - 1], rl = 0;
+#pragma unroll
+      for (int s = 0; s < N - 1; ++s) il[s] = in[s];
+      const float xl = xn;
       bool hl = false;
-      if (vl) {
-#pragma unroll
-        for (int s = 0; s < N - 1; ++s) il[s] = c.oidx[s][el];
-        xl = c.vals[el];
-        hl = (c.tile_mask[el >> 6] >> (el & 63)) & 1ull;
-      } else {
-#pragma unroll
-        for (int s = 0; s < N - 1; ++s) il[s] = 0;
+      if (el < s1) {
+        hl = (mn >> (el & 63)) & 1ull;
+        rl = c.directory[tile_lane_slot(tsn, mn, (int)(el & 63))];
       }
-      const uint64_t hm = __ballot(vl && hl);
+      const uint64_t hm = __ballot(hl);
+      fetch(ch + W);
 #pragma unroll 1
-      for (int q = 0; q < W; ++q) {
-        const int src = sub * W + q;
-        uint32_t idx[N - 1];
+      for (int q0 = 0; q0 < W; q0 += B) {
+        float g[B][N - 1][CPL], og[ADJ ? B : 1][CPL];
+        uint32_t rb[B];
+        bool nw[B];
 #pragma unroll
-        for (int s = 0; s < N - 1; ++s) idx[s] = (uint32_t)__shfl((int)il[s], src, 64);
-        const float x = __shfl(xl, src, 64);
-        const uint64_t e = s0 + ch + q;
-        if (e < s1) {
-          const bool head = (hm >> src) & 1ull;
-          if (arow == NONE || head) {
-            if (arow != NONE) {
-              flush();
-              ++slot;
-            } else {
-              slot = c.tile_slot[s0 >> 6];
+        for (int b = 0; b < B; ++b) {
+          const int src = sub * W + q0 + b;
+          rb[b] = (uint32_t)__shfl((int)rl, src, 64);
+          nw[b] = ((hm >> src) & 1ull) || (ch + q0 + b == 0);  // starts a row or the walker's span
+#pragma unroll
+          for (int s = 0; s < N - 1; ++s)  // past the end: row 0, not used
+            load_row4<CPL>(fa.f[1 + s] + (size_t)(uint32_t)__shfl((int)il[s], src, 64) * R + wl * CPL, g[b][s]);
+          if constexpr (ADJ)
+            if (nw[b]) load_row4<CPL>(fa.f[0] + (size_t)rb[b] * R + wl * CPL, og[b]);
+        }
+#pragma unroll
+        for (int b = 0; b < B; ++b) {
+          const float x = __shfl(xl, sub * W + q0 + b, 64);
+          if (s0 + ch + q0 + b < s1) {
+            if (nw[b]) {
+              if (arow != NONE)
+                end_row();
+              else
+                cont = !((hm >> (sub * W + q0 + b)) & 1ull);
+              arow = rb[b];
+              cnt = 0;
+#pragma unroll
+              for (int q2 = 0; q2 < CPL; ++q2) {
+                acc[q2] = 0.f, sq[q2] = 0.f;
+                if (ADJ) own[q2] = og[b][q2];
+              }
             }
-            arow = c.directory[slot];
+            float h[CPL];
 #pragma unroll
-            for (int q2 = 0; q2 < CPL; ++q2) acc[q2] = 0.f, sq[q2] = 0.f;
-            if (ADJ) load_row4<CPL>(fa.f[0] + (size_t)arow * R + wl * CPL, own);
-          }
-          float h[CPL];
-          load_row4<CPL>(fa.f[1] + (size_t)idx[0] * R + wl * CPL, h);
+            for (int q2 = 0; q2 < CPL; ++q2) h[q2] = g[b][0][q2];
 #pragma unroll
-          for (int s = 1; s < N - 1; ++s) {
-            float g[CPL];
-            load_row4<CPL>(fa.f[1 + s] + (size_t)idx[s] * R + wl * CPL, g);
+            for (int s = 1; s < N - 1; ++s)
 #pragma unroll
-            for (int q2 = 0; q2 < CPL; ++q2) h[q2] *= g[q2];
-          }
-          float w = x;
-          if (ADJ) {
-            float part = 0.f;
+              for (int q2 = 0; q2 < CPL; ++q2) h[q2] *= g[b][s][q2];
+            float w = x;
+            if (ADJ) {
+              float part = 0.f;
 #pragma unroll
-            for (int q2 = 0; q2 < CPL; ++q2) part += own[q2] * h[q2];
-            w = x - group_sum<W>(part);
-            if (LOSS && wl == 0) lsum += (double)w * (double)w;
-          }
+              for (int q2 = 0; q2 < CPL; ++q2) part += own[q2] * h[q2];
+              w = x - group_sum<W>(part);
+              if (LOSS && wl == 0) lsum += (double)w * (double)w;
+            }
+            ++cnt;
 #pragma unroll
-          for (int q2 = 0; q2 < CPL; ++q2) {
-            acc[q2] += w * h[q2];
-            if (SQ) sq[q2] += h[q2] * h[q2];
+            for (int q2 = 0; q2 < CPL; ++q2) {
+              acc[q2] += w * h[q2];
+              if (SQ) sq[q2] += h[q2] * h[q2];
+            }
           }
         }
       }
     }
-    if (arow != NONE) flush();
+    if (SUMS && arow != NONE) leave_open(2 * wk + 1);
+  }
+  if (SUMS) {
+    __syncthreads();
+    // join the open rows of consecutive walkers: a row's first entry takes it
+    auto add = [&](int e, bool more) {
+      float s[CPL], s2[CPL];
+      const uint32_t id = open_id[e];
+      load_row4<CPL>(&open_s[e][wl * CPL], s);
+      if (SQ) load_row4<CPL>(&open_q[SQ ? e : 0][wl * CPL], s2);
+      for (int v = wk + 1; more && v < (int)(blockDim.x / W); ++v) {
+        const uint32_t f = open_id[2 * v];
+        const int from = f == id ? 2 * v : f == NONE && open_id[2 * v + 1] == id ? 2 * v + 1 : -1;
+        if (from < 0) break;
+        float t[CPL];
+        load_row4<CPL>(&open_s[from][wl * CPL], t);
+#pragma unroll
+        for (int q2 = 0; q2 < CPL; ++q2) s[q2] += t[q2];
+        if (SQ) {
+          load_row4<CPL>(&open_q[SQ ? from : 0][wl * CPL], t);
+#pragma unroll
+          for (int q2 = 0; q2 < CPL; ++q2) s2[q2] += t[q2];
+        }
+        if (from == 2 * v) break;  // it ended inside that span
+      }
+#pragma unroll
+      for (int q2 = 0; q2 < CPL; ++q2) {
+        atomic_add_f32(out + (size_t)id * R + wl * CPL + q2, KIND == kWalkAdjoint ? -s[q2] : s[q2]);
+        if (SQ) atomic_add_f32(den + (size_t)id * R + wl * CPL + q2, s2[q2]);
+      }
+    };
+    const uint32_t first = open_id[2 * wk], last = open_id[2 * wk + 1];
+    if (first != NONE && wk == 0) add(0, false);
+    if (last != NONE && (wk == 0 || first != NONE || open_id[2 * wk - 1] != last)) add(2 * wk + 1, true);
   }
   if (LOSS) {
     double t = wave_sum_d(lsum);
@@ -1365,12 +1453,11 @@ __global__ void __launch_bounds__(256) k_sumsq(const float *x, uint64_t n, doubl
 }
 
 // out[k] = sum of part[k * nb .. k * nb + nb) in a fixed order
-__global__ void __launch_bounds__(64) k_reduce_parts(const double *part, uint32_t nb, double *out) {
+__global__ void __launch_bounds__(256) k_reduce_parts(const double *part, uint32_t nb, double *out) {
   const double *p = part + (size_t)blockIdx.x * nb;
   double acc = 0.0;
-  for (uint32_t i = threadIdx.x; i < nb; i += 64) acc += p[i];
-  acc = wave_sum_d(acc);
-  if (threadIdx.x == 0) out[blockIdx.x] = acc;
+  for (uint32_t i = threadIdx.x; i < nb; i += 256) acc += p[i];
+  block_store_sum(acc, out + blockIdx.x);
 }
 
 // ==========================================================================
@@ -1391,26 +1478,36 @@ __global__ void __launch_bounds__(256) k_copy(const uint4 *__restrict__ src, uin
     dst[p] = src[p];
 }
 
-// grad += lambda * c_i * F  for the rows of a CISS directory (c_i = row nnz)
-// or, when per_occurrence == 0, for every row (c_i = 1).
+// The gradient's regulariser, before the adjoint walk adds to it: grad =
+// lambda * c_i * F for the rows of a CISS directory (c_i = row nnz) or, when
+// per_occ == 0, for every row (c_i = 1); part: its share of the loss.  A
+// stream of 16-byte loads and stores: 45 us at 1M rows of R = 32 (20 us of zero
+// fill and 156 us of 4-byte updates after the walk, before).
 __global__ void __launch_bounds__(256) k_reg_rows(const uint32_t *directory, const uint32_t *rowptr,
                                                   uint64_t nrows, int R, float lam, int per_occ,
                                                   const float *F, float *G, double *part) {
   double acc = 0.0;
-  const uint64_t total = nrows * (uint64_t)R;
+  const uint32_t Q = (uint32_t)R / 4;  // 16-byte parts of a row: a power of two
+  const uint64_t total = nrows * (uint64_t)Q;
   for (uint64_t p = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; p < total;
        p += (uint64_t)gridDim.x * blockDim.x) {
-    const uint64_t s = p / R;
-    const int f = (int)(p % R);
-    uint64_t row = s;
+    uint64_t at = p;
     float cnt = 1.f;
     if (per_occ) {
-      row = directory[s];
+      const uint64_t s = p / Q;
+      at = (uint64_t)directory[s] * Q + p % Q;
       cnt = (float)(rowptr[s + 1] - rowptr[s]);
     }
-    const float a = F[row * R + f];
-    G[row * R + f] += lam * cnt * a;
-    acc += 0.5 * (double)lam * (double)cnt * (double)a * (double)a;
+    float a[4], g[4];
+    load_row4<4>(F + at * 4, a);
+    double q = 0.0;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      g[j] = lam * cnt * a[j];
+      q += (double)a[j] * (double)a[j];
+    }
+    store_row4<4>(G + at * 4, g);
+    acc += 0.5 * (double)lam * (double)cnt * q;
   }
   block_store_sum(acc, part + blockIdx.x);
 }
@@ -1518,22 +1615,22 @@ hipError_t launch_sgd_settle(hipStream_t st, SettleArgs a, int R, bool mixed) {
 
 hipError_t launch_mttkrp(hipStream_t st, const CissArgs &c, const FactorArgs &f, int nmodes, int R,
                          uint32_t span, bool adjoint, float *out, double *loss_part,
-                         unsigned *grid_out, unsigned block) {
+                         unsigned *grid_out, unsigned block, float lam, int per_occ) {
   const unsigned grid = (unsigned)mttkrp_grid(c.nnz, R, span, block);
   *grid_out = grid;
   if (c.nnz == 0) return hipSuccess;
   float *none = nullptr;
   if (nmodes == 3) {
     if (adjoint) {
-      CTC_R_SWITCH(R, hipLaunchKernelGGL((k_mttkrp<RR, 3, kWalkAdjoint>), dim3(grid), dim3(block), 0, st, c, f, span, out, loss_part, none));
+      CTC_R_SWITCH(R, hipLaunchKernelGGL((k_mttkrp<RR, 3, kWalkAdjoint>), dim3(grid), dim3(block), 0, st, c, f, span, out, loss_part, none, lam, per_occ));
     } else {
-      CTC_R_SWITCH(R, hipLaunchKernelGGL((k_mttkrp<RR, 3, kWalkMttkrp>), dim3(grid), dim3(block), 0, st, c, f, span, out, loss_part, none));
+      CTC_R_SWITCH(R, hipLaunchKernelGGL((k_mttkrp<RR, 3, kWalkMttkrp>), dim3(grid), dim3(block), 0, st, c, f, span, out, loss_part, none, lam, per_occ));
     }
   } else if (nmodes == 4) {
     if (adjoint) {
-      CTC_R_SWITCH(R, hipLaunchKernelGGL((k_mttkrp<RR, 4, kWalkAdjoint>), dim3(grid), dim3(block), 0, st, c, f, span, out, loss_part, none));
+      CTC_R_SWITCH(R, hipLaunchKernelGGL((k_mttkrp<RR, 4, kWalkAdjoint>), dim3(grid), dim3(block), 0, st, c, f, span, out, loss_part, none, lam, per_occ));
     } else {
-      CTC_R_SWITCH(R, hipLaunchKernelGGL((k_mttkrp<RR, 4, kWalkMttkrp>), dim3(grid), dim3(block), 0, st, c, f, span, out, loss_part, none));
+      CTC_R_SWITCH(R, hipLaunchKernelGGL((k_mttkrp<RR, 4, kWalkMttkrp>), dim3(grid), dim3(block), 0, st, c, f, span, out, loss_part, none, lam, per_occ));
     }
   } else {
     return hipErrorInvalidValue;
@@ -1547,9 +1644,9 @@ hipError_t launch_ccd_jacobi(hipStream_t st, const CissArgs &c, const FactorArgs
   const unsigned grid = (unsigned)mttkrp_grid(c.nnz, R, span, block);
   double *none = nullptr;
   if (nmodes == 3) {
-    CTC_R_SWITCH(R, hipLaunchKernelGGL((k_mttkrp<RR, 3, kWalkJacobi>), dim3(grid), dim3(block), 0, st, c, f, span, num, none, den));
+    CTC_R_SWITCH(R, hipLaunchKernelGGL((k_mttkrp<RR, 3, kWalkJacobi>), dim3(grid), dim3(block), 0, st, c, f, span, num, none, den, 0.f, 0));
   } else if (nmodes == 4) {
-    CTC_R_SWITCH(R, hipLaunchKernelGGL((k_mttkrp<RR, 4, kWalkJacobi>), dim3(grid), dim3(block), 0, st, c, f, span, num, none, den));
+    CTC_R_SWITCH(R, hipLaunchKernelGGL((k_mttkrp<RR, 4, kWalkJacobi>), dim3(grid), dim3(block), 0, st, c, f, span, num, none, den, 0.f, 0));
   } else {
     return hipErrorInvalidValue;
   }
@@ -1562,9 +1659,9 @@ hipError_t launch_loss_walk(hipStream_t st, const CissArgs &c, const FactorArgs 
   const unsigned grid = (unsigned)mttkrp_grid(c.nnz, R, span, block);
   float *none = nullptr;
   if (nmodes == 3) {
-    CTC_R_SWITCH(R, hipLaunchKernelGGL((k_mttkrp<RR, 3, kWalkLoss>), dim3(grid), dim3(block), 0, st, c, f, span, none, part, none));
+    CTC_R_SWITCH(R, hipLaunchKernelGGL((k_mttkrp<RR, 3, kWalkLoss>), dim3(grid), dim3(block), 0, st, c, f, span, none, part, none, 0.f, 0));
   } else if (nmodes == 4) {
-    CTC_R_SWITCH(R, hipLaunchKernelGGL((k_mttkrp<RR, 4, kWalkLoss>), dim3(grid), dim3(block), 0, st, c, f, span, none, part, none));
+    CTC_R_SWITCH(R, hipLaunchKernelGGL((k_mttkrp<RR, 4, kWalkLoss>), dim3(grid), dim3(block), 0, st, c, f, span, none, part, none, 0.f, 0));
   } else {
     return hipErrorInvalidValue;
   }
@@ -1572,6 +1669,14 @@ hipError_t launch_loss_walk(hipStream_t st, const CissArgs &c, const FactorArgs 
 }
 
 uint64_t mttkrp_walkers_per_block(int R, unsigned block) { return (uint64_t)(block / 64) * (64 / (R / 4)); }
+
+// Spans of 256 where they fill the chip (MTTKRP of 8M nonzeros at R = 32: 117 us,
+// 125 / 131 / 131 us with 128 / 64 / 32), down to 32 for smaller tensors: about
+// 4096 waves (the loss of 1M nonzeros at R = 16: 14 us, 89 us with 256).
+uint32_t walk_span(uint64_t nnz, int R) {
+  const uint64_t per = nnz / (4096 * (uint64_t)(256 / R)) / 32 * 32;
+  return (uint32_t)(per < 32 ? 32 : per > 256 ? 256 : per);
+}
 
 uint64_t mttkrp_grid(uint64_t nnz, int R, uint32_t span, unsigned block) {
   const uint64_t walkers = (nnz + span - 1) / span;
@@ -1716,7 +1821,7 @@ hipError_t launch_sumsq(hipStream_t st, const float *x, uint64_t n, unsigned nbl
 
 hipError_t launch_reduce_parts(hipStream_t st, const double *part, uint32_t nb, uint32_t groups,
                                double *out) {
-  hipLaunchKernelGGL(k_reduce_parts, dim3(groups), dim3(64), 0, st, part, nb, out);
+  hipLaunchKernelGGL(k_reduce_parts, dim3(groups), dim3(256), 0, st, part, nb, out);
   return hipGetLastError();
 }
 

@@ -18,9 +18,12 @@ hipError_t launch_sgd_sync(hipStream_t st, const CissArgs &c, const FactorArgs &
                            unsigned block, bool mixed);
 // nb_merge is set here; pb / fb must be prefix sums with pb[0..1] = fb[0..1] = 0
 hipError_t launch_sgd_settle(hipStream_t st, SettleArgs a, int R, bool mixed);
+// out: zeros, or for the adjoint what launch_reg_rows left (lam, per_occ: its arguments)
 hipError_t launch_mttkrp(hipStream_t st, const CissArgs &c, const FactorArgs &f, int nmodes, int R,
                          uint32_t span, bool adjoint, float *out, double *loss_part,
-                         unsigned *grid_out, unsigned block);
+                         unsigned *grid_out, unsigned block, float lam = 0.f, int per_occ = 0);
+// nonzeros per walker of k_mttkrp
+uint32_t walk_span(uint64_t nnz, int R);
 uint64_t mttkrp_grid(uint64_t nnz, int R, uint32_t span, unsigned block);
 // the training loss as a walk of the CISS c (rows kept along their runs):
 // part[b] = the squared residuals of block b, for the mttkrp_grid(c.nnz, R,
@@ -55,6 +58,7 @@ hipError_t launch_reduce_parts(hipStream_t st, const double *part, uint32_t nb, 
                                double *out);
 hipError_t launch_fill(hipStream_t st, float *x, uint64_t n, float v);
 hipError_t launch_copy(hipStream_t st, const void *src, void *dst, uint64_t bytes);  // bytes % 16 == 0
+// G = lam c F over the directory's rows (per_occ; the other rows are not touched) or all nrows rows
 hipError_t launch_reg_rows(hipStream_t st, const uint32_t *directory, const uint32_t *rowptr,
                            uint64_t nrows, int R, float lam, int per_occ, const float *F, float *G,
                            unsigned nblocks, double *part);

@@ -16,6 +16,7 @@ using namespace ctc;
 namespace {
 
 constexpr unsigned kEvalBlocks = 512;  // fixed grid for deterministic reductions
+constexpr unsigned kRegBlocks = 2048;  // of the regulariser's stream over the factors
 // SGD hot rows (updated with plain stores): more than kSgdHotRows training
 // nonzeros and more than kSgdHotRel times the mode's mean.  Measured on the
 // 100M-nonzero tensor (480189 x 17770 x 2182, R = 32), k_sgd ms per epoch:
@@ -1029,7 +1030,7 @@ extern "C" ctc_status ctc_mttkrp(ctc_model *m, uint32_t mode, float *host_out) {
   {
     Prof p(m->ctx, "mttkrp");
     CTC_HIP(launch_mttkrp(st, ciss_args(m->ciss[mode]), rel_factors(m->F, m->nmodes, mode), (int)m->nmodes,
-                          (int)R, 256, false, out, nullptr, &grid, 256));
+                          (int)R, walk_span(m->ciss[mode].nnz, (int)R), false, out, nullptr, &grid, 256));
   }
   CTC_HIP(hipMemcpyAsync(host_out, out, n * sizeof(float), hipMemcpyDeviceToHost, st));
   CTC_HIP(hipStreamSynchronize(st));
@@ -1056,7 +1057,7 @@ extern "C" ctc_status ctc_evaluate(ctc_model *m, double lambda, double *loss, do
   // the training loss as a walk of the mode-0 CISS, each walker keeping its
   // rows along their runs (kWalkLoss); its per-block sums are reduced in order
   // into group 0's first slot, the group's other slots zeroed
-  const uint32_t span = 256;
+  const uint32_t span = walk_span(m->ciss[0].nnz, (int)R);
   const uint64_t nb = mttkrp_grid(m->ciss[0].nnz, (int)R, span, 256);
   if (nb > m->eval_part_n) {
     CTC_HIP(hipStreamSynchronize(st));
@@ -1115,25 +1116,25 @@ extern "C" ctc_status ctc_grad(ctc_model *m, const float *const *factors, float 
     CTC_TRY(ensure_ciss(m, md));
   }
   // partial sums: N walks + N regularisers, each up to `nb` blocks
-  const uint32_t span = 256;
+  const uint32_t span = walk_span(m->train_nnz, (int)R);
   uint64_t nb = 0;
   for (uint32_t md = 0; md < N; ++md) nb = std::max<uint64_t>(nb, mttkrp_grid(m->train_nnz, (int)R, span, 256));
-  nb = std::max<uint64_t>(nb, kEvalBlocks);
+  nb = std::max<uint64_t>(nb, kRegBlocks);
   CTC_TRY(ensure_scratch(m, (size_t)2 * N * nb * sizeof(double)));
   double *part = (double *)m->scratch;
   CTC_HIP(hipMemsetAsync(part, 0, (size_t)2 * N * nb * sizeof(double), st));
   for (uint32_t md = 0; md < N; ++md) {
-    CTC_HIP(launch_fill(st, grads[md], m->dims[md] * R, 0.f));
+    const DevCiss &d = m->ciss[md];
+    const uint64_t nrows = reg_per_occurrence ? d.dlength : m->dims[md];
+    if (reg_per_occurrence && d.dlength < m->dims[md]) CTC_HIP(launch_fill(st, grads[md], m->dims[md] * R, 0.f));
+    CTC_HIP(launch_reg_rows(st, d.directory, d.rowptr, nrows, (int)R, (float)lambda, reg_per_occurrence, F[md],
+                            grads[md], kRegBlocks, part + (size_t)(N + md) * nb));
     unsigned grid = 0;
     {
       Prof p(m->ctx, "adjoint", st);
-      CTC_HIP(launch_mttkrp(st, ciss_args(m->ciss[md]), rel_factors(F, N, md), (int)N, (int)R, span, true,
-                            grads[md], part + (size_t)md * nb, &grid, 256));
+      CTC_HIP(launch_mttkrp(st, ciss_args(d), rel_factors(F, N, md), (int)N, (int)R, span, true, grads[md],
+                            part + (size_t)md * nb, &grid, 256, (float)lambda, reg_per_occurrence));
     }
-    const DevCiss &d = m->ciss[md];
-    const uint64_t nrows = reg_per_occurrence ? d.dlength : m->dims[md];
-    CTC_HIP(launch_reg_rows(st, d.directory, d.rowptr, nrows, (int)R, (float)lambda, reg_per_occurrence, F[md],
-                            grads[md], kEvalBlocks, part + (size_t)(N + md) * nb));
   }
   CTC_HIP(launch_reduce_parts(st, part, (uint32_t)nb, 2 * N, m->dstat));
   CTC_HIP(hipMemcpyAsync(m->hstat, m->dstat, 2 * N * sizeof(double), hipMemcpyDeviceToHost, st));

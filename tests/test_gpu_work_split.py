@@ -96,3 +96,47 @@ def test_als_default_spans(ctx, dims, nnz, R, refine):
         want = ridge(ind, vals, F, mode, 0.5)
         e = np.linalg.norm(m.factor(mode) - want) / np.linalg.norm(want)
         assert e < 1e-5, (mode, e)
+
+
+@pytest.mark.parametrize("R", [8, 16, 32, 64, 128])
+@pytest.mark.parametrize("dims,nnz", [((1, 40, 30), 1100), ((3, 300, 50), 31), ((3, 300, 50), 33),
+                                      ((700, 9, 40), 32 * 131 + 1), ((5, 600, 80), 32 * 1200), ((12, 3, 40, 15), 9000)],
+                         ids=["one_row", "short", "one_span", "rows_in_spans", "rows_over_groups", "4way"])
+def test_walk_row_sums(ctx, dims, nnz, R):
+    """MTTKRP, and the gradient with its two regularisers, of rows inside one
+    walker's span, across walkers and across workgroups, rows that end at a
+    span's end, and rows without nonzeros, against 64 bits at the parity
+    tests' bars (MTTKRP and gradients 1e-5, loss 1e-6)."""
+    import torch
+    say(f"[walk sums] dims={dims} nnz={nnz} R={R}")
+    t, ind, vals = coo(dims, nnz, 11)
+    rng = np.random.default_rng(12)
+    F = [rng.uniform(-1, 1, (d, R)).astype(np.float32) for d in dims]
+    F64 = [f.astype(np.float64) for f in F]
+    m = ct.Model(ctx, t, None, None, rank=R)
+    m.set_factors(F)
+    e = vals - predict(ind, F)
+    hs = []
+    for mode in range(len(dims)):
+        h = np.ones((nnz, R))
+        for k, f in enumerate(F64):
+            if k != mode:
+                h *= f[ind[k]]
+        hs.append(h)
+        want = np.zeros((dims[mode], R))
+        np.add.at(want, ind[mode], vals[:, None] * h)
+        assert np.linalg.norm(m.mttkrp(mode) - want) < 1e-5 * np.linalg.norm(want), mode
+    dev = [torch.from_numpy(f).cuda() for f in F]
+    for per_occ in (False, True):
+        G = [torch.full_like(f, 7.0) for f in dev]
+        torch.cuda.synchronize()
+        loss = m.grad_device([f.data_ptr() for f in dev], [g.data_ptr() for g in G], 0.3, per_occ)
+        wl = 0.5 * np.sum(e * e)
+        for mode in range(len(dims)):
+            c = np.bincount(ind[mode], minlength=dims[mode])[:, None] if per_occ else 1.0
+            want = 0.3 * c * F64[mode]
+            np.add.at(want, ind[mode], -e[:, None] * hs[mode])
+            wl += 0.15 * np.sum(c * F64[mode] ** 2)
+            got = G[mode].cpu().numpy()
+            assert np.linalg.norm(got - want) < 1e-5 * np.linalg.norm(want), (mode, per_occ)
+        assert loss == pytest.approx(wl, rel=1e-6)
