@@ -237,12 +237,10 @@ __global__ void __launch_bounds__(256) k_sgd(CissArgs c, FactorArgs fa, HotRows 
 constexpr double kFixScale = 4294967296.0;        // 2^32
 constexpr double kFixInv = 1.0 / 4294967296.0;    // 2^-32
 
-// A walker is W = R / 4 lanes of a wave; lane l holds the row elements
-// 4l .. 4l + 3, so a row moves with one 16-byte access per lane and a wave
-// carries 256 / R walkers (eight at R = 32).  Each walker is a chain of
-// dependent steps whose row reads miss the L2 (the launch starts with it
-// invalidated), so the more walkers a wave carries, the more of those reads
-// are in flight at once.
+// Lane shape of the merge and of the row walks below: a walker is W = R / 4
+// lanes of a wave; lane l holds the row elements 4l .. 4l + 3, so a row moves
+// with one 16-byte access per lane and a wave carries 256 / R walkers (eight at
+// R = 32).
 template <int R>
 struct SyncShape {
   static constexpr int CPL = 4;
@@ -270,15 +268,6 @@ __device__ inline void store_row4(float *p, const float (&v)[CPL]) {
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 template <int CPL>
-__device__ inline void store_row4_nt(float *p, const float (&v)[CPL]) {
-#pragma unroll
-  for (int j = 0; j < CPL; j += 4) {
-    f32x4 t = {v[j], v[j + 1], v[j + 2], v[j + 3]};
-    __builtin_nontemporal_store(t, reinterpret_cast<f32x4 *>(p + j));
-  }
-}
-
-template <int CPL>
 __device__ inline void load_row4_nt(const float *p, float (&v)[CPL]) {
 #pragma unroll
   for (int j = 0; j < CPL; j += 4) {
@@ -299,81 +288,124 @@ __device__ inline void load_bf4_nt(const uint16_t *p, float (&v)[CPL]) {
   }
 }
 
+// Lane shape of the SGD walk: a lane holds CPL elements of a row.  A walker's
+// time is its chain of instructions per nonzero, which is shorter with two
+// elements, while four take fewer instructions in all: see launch_sgd_sync.
+template <int R, int CPL>
+struct WalkShape {
+  static constexpr int W = R / CPL;
+  static constexpr int WPW = 64 / W;
+};
+
 template <int CPL>
-__device__ inline void store_bf4_nt(uint16_t *p, const float (&v)[CPL]) {
+using Cols = float __attribute__((ext_vector_type(CPL)));
+
+// a staged delta, FP32 or BF16 (round to nearest even)
+template <int CPL, bool MIX>
+__device__ inline void stage_cols(float *stage, size_t at, Cols<CPL> v) {
+  if constexpr (MIX) {
+    uint32_t __attribute__((ext_vector_type(CPL / 2))) t;
 #pragma unroll
-  for (int j = 0; j < CPL; j += 4) {
-    const u32x2 t = {(uint32_t)f2bf(v[j]) | ((uint32_t)f2bf(v[j + 1]) << 16),
-                     (uint32_t)f2bf(v[j + 2]) | ((uint32_t)f2bf(v[j + 3]) << 16)};
-    __builtin_nontemporal_store(t, reinterpret_cast<u32x2 *>(p + j));
+    for (int j = 0; j < CPL / 2; ++j) t[j] = (uint32_t)f2bf(v[2 * j]) | ((uint32_t)f2bf(v[2 * j + 1]) << 16);
+    __builtin_nontemporal_store(t, reinterpret_cast<decltype(t) *>(reinterpret_cast<uint16_t *>(stage) + at));
+  } else {
+    __builtin_nontemporal_store(v, reinterpret_cast<Cols<CPL> *>(stage + at));
   }
 }
 
 // MIX (the mixed-precision path): the run deltas of modes 1.. are staged in
 // BF16 (round to nearest even), halving the staging traffic; the factors, the
 // walker's arithmetic and the sums of the deltas stay FP32 / FP64.
-template <int R, int N, bool MIX>
+//
+// A walker's nonzeros are one dependent chain (each step starts from the
+// rows the last one left), so what a step waits for and the instructions it
+// takes set the time.  Rows of a sub-step do not change while it runs (an
+// in-place mode-0 row has one reader, its own walker), so nothing has to wait
+// but the arithmetic:
+//   * the indices, values, mode-0 rows, run ends and staging positions of
+//     SyncMeta::CH nonzeros are read at once and kept in LDS;
+//   * the rows of nonzero t + 4 are requested when nonzero t has been
+//     consumed, whether a run starts there or not (a row that goes on is a
+//     cache hit, and unconditional loads leave the compiler exact wait counts).
+// Time of a sub-step's walk at R = 32: 12.5M nonzeros 39 -> 21 us, 50M nonzeros
+// 64 -> 53 us (the staged deltas, 200 MB, are written at 3.8 TB/s); R = 64 mixed,
+// 5M nonzeros 41 -> 21 us; R = 16, 20K nonzeros 24 -> 14 us.
+enum : uint32_t { kOwnRow = 1u, kRunEnd = 2u };  // kRunEnd << k: the run in mode k ends with this nonzero
+
+template <int R, int N, bool MIX, int CPL>
+struct SyncMeta {
+  static constexpr int W = WalkShape<R, CPL>::W;
+  static constexpr int CH = 4 * W < 32 ? 4 * W : 32;      // nonzeros of a walker per round: at most 4 per lane
+  static constexpr int WORDS = N + 2 + (MIX ? N - 1 : 0);  // other modes' rows, value, mode-0 row, flags, positions
+  // one nonzero more than are kept (read ahead, not used); odd: the walkers'
+  // broadcasts fall on different banks
+  static constexpr int STRIDE = ((CH + 1) * WORDS) | 1;
+  static constexpr size_t kWaveBytes = (size_t)WalkShape<R, CPL>::WPW * STRIDE * sizeof(uint32_t);
+};
+
+template <int R, int N, bool MIX, int CPL>
 __global__ void __launch_bounds__(256) k_sgd_sync(CissArgs c, FactorArgs fa, SyncArgs sy, uint32_t span,
                                                   uint32_t sub, uint32_t s, uint64_t nspans, uint32_t long_min,
                                                   float step, float lam) {
-  constexpr int W = SyncShape<R>::W;
-  constexpr int CPL = SyncShape<R>::CPL;
-  constexpr int WPW = SyncShape<R>::WPW;
-  constexpr uint32_t NONE = 0xFFFFFFFFu;
+  constexpr int W = WalkShape<R, CPL>::W;
+  constexpr int WPW = WalkShape<R, CPL>::WPW;
+  using Meta = SyncMeta<R, N, MIX, CPL>;
+  constexpr int CH = Meta::CH, NW = Meta::WORDS, J = CH / W;
+  constexpr int B = 4;  // nonzeros whose rows are in flight
+  extern __shared__ uint32_t meta_s[];
   const int lane = lane_id();
-  const int sub_w = lane / W;
   const int wl = lane % W;
   const uint64_t wave = (uint64_t)blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
-  const uint64_t walker = wave * WPW + sub_w;
+  const uint64_t walker = wave * WPW + lane / W;
   if (wave * WPW >= nspans) return;  // whole wave idle (uniform)
-  uint64_t e0 = 0, e1 = 0;
+  uint32_t *meta = meta_s + (threadIdx.x / W) * Meta::STRIDE;
+  uint64_t e0 = 0;
+  uint32_t len = 0;  // this walker's nonzeros in the sub-step
   if (walker < nspans) {
     const uint64_t send = (walker + 1) * span < c.nnz ? (walker + 1) * span : c.nnz;
     e0 = walker * span + (uint64_t)s * sub;
-    e1 = e0 + sub < send ? e0 + sub : send;
-    if (e0 > e1) e0 = e1;
+    if (e0 < send) len = (uint32_t)(send - e0 < sub ? send - e0 : sub);
   }
-  float *Fm[N];
-#pragma unroll
-  for (int q = 0; q < N; ++q) Fm[q] = fa.f[q];
-  float v[N][CPL], del[N][CPL];
-  uint32_t cur[N];
-#pragma unroll
-  for (int q = 0; q < N; ++q) {
-    cur[q] = NONE;
-#pragma unroll
-    for (int k = 0; k < CPL; ++k) v[q][k] = 0.f, del[q][k] = 0.f;
-  }
-  uint32_t slot = 0;
-  bool own0 = false;  // the current mode-0 row is stored in place (no other walker meets it)
-  // modes 1..: the next slot of this chunk's runs and, on the mixed path, its
-  // staging position, read one run ahead (the table has one entry of padding)
-  uint32_t rslot[N], rpos[N];
+  using V = Cols<CPL>;
+  V v[N], del[N];
+  bool fresh[N];  // the next nonzero starts a run in mode k
+  uint32_t rslot[N];  // modes 1..: the next staging slot
 #pragma unroll
   for (int k = 0; k < N; ++k) {
-    rslot[k] = (k >= 1 && walker < nspans) ? sy.sbase[k][(size_t)s * nspans + walker] : 0u;
-    rpos[k] = (MIX && k >= 1) ? sy.dest[k][rslot[k]] : 0u;
+    fresh[k] = true;
+    rslot[k] = k >= 1 ? sy.sbase[k][(size_t)s * nspans + (walker < nspans ? walker : nspans - 1)] : 0u;
+    v[k] = del[k] = 0.f;
   }
-  auto hand_in = [&](int q) {
-    if (q >= 1) {  // the run's delta goes to its staging slot / position
-      if constexpr (MIX) {
-        const uint32_t pos = rpos[q];
-        rpos[q] = sy.dest[q][++rslot[q]];
-        store_bf4_nt<CPL>(reinterpret_cast<uint16_t *>(sy.stage[q]) + (size_t)pos * R + wl * CPL, del[q]);
-      } else {
-        store_row4_nt<CPL>(sy.stage[q] + (size_t)rslot[q]++ * R + wl * CPL, del[q]);
-      }
+
+  // the rows in flight of nonzero t (in slot t % B), and what is known of it;
+  // what LDS holds of a nonzero is read one nonzero before its rows are requested
+  V g[B][N];
+  float xb[B], xm = 0.f;
+  uint32_t row0[B], fl[B], rm[N], fm = 0;
+  auto peek = [&](int t) {
+    const uint32_t *w = meta + t * NW;
+#pragma unroll
+    for (int k = 0; k < N; ++k) rm[k] = w[k == 0 ? N : k - 1];
+    xm = __uint_as_float(w[N - 1]);
+    fm = w[N + 1];
+  };
+  auto request = [&](int b) {
+    xb[b] = xm, row0[b] = rm[0], fl[b] = fm;
+#pragma unroll
+    for (int k = 0; k < N; ++k)
+      g[b][k] = *reinterpret_cast<const V *>(fa.f[k] + (size_t)rm[k] * R + wl * CPL);
+  };
+  // a mode-0 run ends: its row is stored in place where no other walker meets
+  // it; the deltas of a longer row are added as fixed-point integers
+  auto end_row0 = [&](uint32_t row, bool own) {
+    if (own) {
+      *reinterpret_cast<V *>(fa.f[0] + (size_t)row * R + wl * CPL) = v[0];
       return;
     }
-    if (own0) {
-      store_row4<CPL>(Fm[0] + (size_t)cur[0] * R + wl * CPL, v[0]);
-      return;
-    }
-    // a long mode-0 row: fixed-point sums
-    const uint32_t h = sy.hidx[0][cur[0]];
+    const uint32_t h = sy.hidx[0][row];
     unsigned long long *d;
     if (h == 0xFFFFFFFFu) {
-      d = (unsigned long long *)sy.D[0] + (size_t)cur[0] * R;
+      d = (unsigned long long *)sy.D[0] + (size_t)row * R;
     } else {
       // a hot row's mean needs its count of runs; a cold row adds its delta
       // sum, so the merge needs no count (an untouched row's sum is 0)
@@ -382,92 +414,132 @@ __global__ void __launch_bounds__(256) k_sgd_sync(CissArgs c, FactorArgs fa, Syn
       if (wl == 0) atomicAdd(sy.ch[0] + r, 1u);
     }
 #pragma unroll
-    for (int k = 0; k < CPL; ++k)
-      atomicAdd(d + wl * CPL + k, (unsigned long long)__double2ll_rn((double)del[q][k] * kFixScale));
+    for (int j = 0; j < CPL; ++j)
+      atomicAdd(d + wl * CPL + j, (unsigned long long)__double2ll_rn((double)del[0][j] * kFixScale));
   };
-
-  for (uint32_t ch = 0; ch < sub; ch += W) {
-    const uint64_t el = e0 + ch + wl;
-    const bool vl = el < e1;
-    uint32_t il[N - 1];
-    float xl = 0.f;
-    bool hl = false;
-    if (vl) {
+  auto consume = [&](int t, int b) {
 #pragma unroll
-      for (int q = 0; q < N - 1; ++q) il[q] = c.oidx[q][el];
-      xl = c.vals[el];
-      hl = (c.tile_mask[el >> 6] >> (el & 63)) & 1ull;
-    } else {
-#pragma unroll
-      for (int q = 0; q < N - 1; ++q) il[q] = 0;
+    for (int k = 0; k < N; ++k) {
+      v[k] = fresh[k] ? g[b][k] : v[k];
+      del[k] = fresh[k] ? V(0.f) : del[k];
     }
-    const uint64_t hm = __ballot(vl && hl);
-#pragma unroll 1  // rolled: 76 VGPRs, six waves per SIMD
-    for (int q = 0; q < W; ++q) {
-      const int src = sub_w * W + q;
-      uint32_t idx[N];
+    float part = 0.f;
 #pragma unroll
-      for (int k = 0; k < N - 1; ++k) idx[1 + k] = (uint32_t)__shfl((int)il[k], src, 64);
-      const float x = __shfl(xl, src, 64);
-      const uint64_t e = e0 + ch + q;
-      if (e < e1) {
-        const bool head = (hm >> src) & 1ull;
-        bool new0 = false;
-        if (cur[0] == NONE) {
-          slot = tile_lane_slot(c.tile_slot[e >> 6], c.tile_mask[e >> 6], (int)(e & 63));
-          new0 = true;
-        } else if (head) {
-          slot = slot + 1;
-          new0 = true;
-        }
-        if (new0) {
-          idx[0] = c.directory[slot];
-        } else {
-          idx[0] = cur[0];
-        }
+    for (int j = 0; j < CPL; ++j) {
+      float pv = v[0][j];
 #pragma unroll
-        for (int k = 0; k < N; ++k) {
-          if (idx[k] != cur[k]) {
-            if (cur[k] != NONE) hand_in(k);
-            if (k == 0) own0 = c.rowptr[slot + 1] - c.rowptr[slot] < long_min;
-            cur[k] = idx[k];
-            load_row4<CPL>(Fm[k] + (size_t)idx[k] * R + wl * CPL, v[k]);
+      for (int k = 1; k < N - 1; ++k) pv *= v[k][j];
+      part = fmaf(pv, v[N - 1][j], part);
+    }
+    const float err = xb[b] - group_sum<W>(part);
 #pragma unroll
-            for (int j = 0; j < CPL; ++j) del[k][j] = 0.f;
-          }
-        }
-        float part = 0.f;
+    for (int j = 0; j < CPL; ++j) {
+      float d[N];  // the step over its rate
 #pragma unroll
-        for (int j = 0; j < CPL; ++j) {
-          float pv = v[0][j];
+      for (int k = 0; k < N; ++k) {
+        float o = 1.f;
 #pragma unroll
-          for (int k = 1; k < N; ++k) pv *= v[k][j];
-          part += pv;
-        }
-        const float err = x - group_sum<W>(part);
+        for (int k2 = 0; k2 < N; ++k2)
+          if (k2 != k) o *= v[k2][j];
+        d[k] = fmaf(err, o, -(lam * v[k][j]));
+      }
 #pragma unroll
-        for (int j = 0; j < CPL; ++j) {
-          float d[N];
-#pragma unroll
-          for (int k = 0; k < N; ++k) {
-            float o = 1.f;
-#pragma unroll
-            for (int k2 = 0; k2 < N; ++k2)
-              if (k2 != k) o *= v[k2][j];
-            d[k] = step * (err * o - lam * v[k][j]);
-          }
-#pragma unroll
-          for (int k = 0; k < N; ++k) {
-            v[k][j] += d[k];
-            del[k][j] += d[k];
-          }
-        }
+      for (int k = 0; k < N; ++k) {
+        v[k][j] = fmaf(step, d[k], v[k][j]);
+        del[k][j] = fmaf(step, d[k], del[k][j]);
       }
     }
-  }
 #pragma unroll
-  for (int k = 0; k < N; ++k)
-    if (cur[k] != NONE) hand_in(k);
+    for (int k = 0; k < N; ++k) fresh[k] = (fl[b] & (kRunEnd << k)) != 0;
+#pragma unroll
+    for (int k = 1; k < N; ++k)
+      if (fresh[k]) {  // the run's delta goes to its staging slot / position
+        const uint32_t at = MIX ? meta[t * NW + N + 1 + k] : rslot[k]++;
+        stage_cols<CPL, MIX>(sy.stage[k], (size_t)at * R + wl * CPL, del[k]);
+      }
+    if (fresh[0]) end_row0(row0[b], (fl[b] & kOwnRow) != 0);
+  };
+
+  for (uint32_t ch = 0; ch < sub; ch += CH) {
+    wave_sync();  // the last round's reads are done
+    const uint32_t n = ch < len ? (len - ch < (uint32_t)CH ? len - ch : (uint32_t)CH) : 0u;
+    if (__ballot(n > 0) == 0) break;
+    // unconditional, so that all the loads of a step are in flight together
+    // (past the walker's end: its last nonzero again, or nonzero 0)
+    const uint64_t last = len ? e0 + len - 1 : 0;
+    uint32_t ix[J][N - 1], nx[J][N - 1], slot[J], row[J], r0[J], r1[J];
+    uint64_t mask[J];
+    float x[J];
+#pragma unroll
+    for (int j = 0; j < J; ++j) {
+      const uint64_t at = e0 + ch + j * W + wl, e = at < last ? at : last, f = e < last ? e + 1 : e;
+      slot[j] = c.tile_slot[e >> 6], mask[j] = c.tile_mask[e >> 6];
+#pragma unroll
+      for (int k = 0; k < N - 1; ++k) ix[j][k] = c.oidx[k][e], nx[j][k] = c.oidx[k][f];
+      x[j] = c.vals[e];
+    }
+#pragma unroll
+    for (int j = 0; j < J; ++j) {
+      const uint64_t at = e0 + ch + j * W + wl, e = at < last ? at : last;
+      slot[j] = tile_lane_slot(slot[j], mask[j], (int)(e & 63));
+      row[j] = c.directory[slot[j]];
+      r0[j] = c.rowptr[slot[j]], r1[j] = c.rowptr[slot[j] + 1];
+    }
+    uint32_t fl_t[J];
+#pragma unroll
+    for (int j = 0; j < J; ++j) {
+      const uint64_t at = e0 + ch + j * W + wl;
+      fl_t[j] = r1[j] - r0[j] < long_min ? kOwnRow : 0u;
+      if (at >= last || (uint64_t)r1[j] == at + 1) fl_t[j] |= kRunEnd;
+#pragma unroll
+      for (int k = 1; k < N; ++k)
+        if (at >= last || nx[j][k - 1] != ix[j][k - 1]) fl_t[j] |= kRunEnd << k;
+    }
+    uint32_t pos[J][N];
+    if constexpr (MIX) {
+      // staging positions of the runs that end here: the slots counted on from
+      // the walker's next one, in walk order
+#pragma unroll
+      for (int k = 1; k < N; ++k)
+#pragma unroll
+        for (int j = 0; j < J; ++j) {
+          const bool ends = (uint32_t)(j * W + wl) < n && (fl_t[j] & (kRunEnd << k));
+          const uint64_t mine = (__ballot(ends) >> (lane - wl)) & (W == 64 ? ~0ull : (1ull << W) - 1);
+          pos[j][k] = ends ? sy.dest[k][rslot[k] + __popcll(mine & ((1ull << wl) - 1))] : 0u;
+          rslot[k] += __popcll(mine);
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < J; ++j) {
+      uint32_t *w = meta + (j * W + wl) * NW;
+#pragma unroll
+      for (int k = 0; k < N - 1; ++k) w[k] = ix[j][k];
+      w[N - 1] = __float_as_uint(x[j]);
+      w[N] = row[j];
+      w[N + 1] = fl_t[j];
+      if constexpr (MIX)
+#pragma unroll
+        for (int k = 1; k < N; ++k) w[N + 1 + k] = pos[j][k];
+    }
+    wave_sync();
+#pragma unroll
+    for (int b = 0; b < B; ++b) {
+      peek(b);
+      request(b);
+    }
+    peek(B);
+#pragma unroll 1
+    for (int q = 0; q < CH - B; q += B)
+#pragma unroll
+      for (int b = 0; b < B; ++b) {
+        if ((uint32_t)(q + b) < n) consume(q + b, b);
+        request(b);
+        peek(q + B + b + 1);  // of the last: one past the round's nonzeros, not used
+      }
+#pragma unroll
+    for (int b = 0; b < B; ++b)
+      if ((uint32_t)(CH - B + b) < n) consume(CH - B + b, b);
+  }
 }
 
 // Mode 0's long rows (k_sgd_sync's fixed-point sums) as block `blk` of a
@@ -1515,13 +1587,13 @@ __global__ void __launch_bounds__(256) k_reg_rows(const uint32_t *directory, con
 // ==========================================================================
 // launchers
 // ==========================================================================
-#define CTC_R_SWITCH(R, BODY)                                       \
+#define CTC_R_SWITCH(R, ...)                                        \
   switch (R) {                                                      \
-    case 8: { constexpr int RR = 8; BODY; } break;                  \
-    case 16: { constexpr int RR = 16; BODY; } break;                \
-    case 32: { constexpr int RR = 32; BODY; } break;                \
-    case 64: { constexpr int RR = 64; BODY; } break;                \
-    case 128: { constexpr int RR = 128; BODY; } break;              \
+    case 8: { constexpr int RR = 8; __VA_ARGS__; } break;           \
+    case 16: { constexpr int RR = 16; __VA_ARGS__; } break;         \
+    case 32: { constexpr int RR = 32; __VA_ARGS__; } break;         \
+    case 64: { constexpr int RR = 64; __VA_ARGS__; } break;         \
+    case 128: { constexpr int RR = 128; __VA_ARGS__; } break;       \
     default: return hipErrorInvalidValue;                           \
   }
 
@@ -1565,32 +1637,40 @@ hipError_t launch_sgd(hipStream_t st, const CissArgs &c, const FactorArgs &f, co
   return hipErrorInvalidValue;
 }
 
+template <int R, int N, bool MIX, int CPL>
+static void launch_sync_as(hipStream_t st, const CissArgs &c, const FactorArgs &f, const SyncArgs &sy, uint32_t span,
+                           uint32_t sub, uint32_t s, uint64_t nspans, uint32_t long_min, float step, float lam,
+                           unsigned block) {
+  constexpr uint64_t wpw = WalkShape<R, CPL>::WPW;
+  const size_t lds = (block / 64) * SyncMeta<R, N, MIX, CPL>::kWaveBytes;
+  hipLaunchKernelGGL((k_sgd_sync<R, N, MIX, CPL>), dim3(grid_for((nspans + wpw - 1) / wpw, block)), dim3(block), lds, st,
+                     c, f, sy, span, sub, s, nspans, long_min, step, lam);
+}
+
 hipError_t launch_sgd_sync(hipStream_t st, const CissArgs &c, const FactorArgs &f, const SyncArgs &sy, int nmodes,
                            int R, uint32_t span, uint32_t sub, uint32_t s, uint32_t long_min, float step, float lam,
                            unsigned block, bool mixed) {
   if (c.nnz == 0) return hipSuccess;
+  if (nmodes != 3 && nmodes != 4) return hipErrorInvalidValue;
   const uint64_t nspans = (c.nnz + span - 1) / span;
-  const int wpw = 256 / R;  // walkers per wave (SyncShape)
-  const uint64_t waves = (nspans + wpw - 1) / wpw;
-  const unsigned grid = grid_for(waves, block);
-#define CTC_SYNC_LAUNCH(NN, MM) \
-  CTC_R_SWITCH(R, hipLaunchKernelGGL((k_sgd_sync<RR, NN, MM>), dim3(grid), dim3(block), 0, st, c, f, sy, span, sub, s, nspans, long_min, step, lam))
+  // Two elements per lane while four would leave a SIMD with less than two
+  // waves (R = 32: 12.5M nonzeros 3113 us an epoch against 3230, 50M nonzeros 6104
+  // against 5957; R = 16, 20K nonzeros 1424 against 1628).  From R = 64 on the sum
+  // over a walker of more than 16 lanes would cost more.  Mixed: always four,
+  // the order of that sum decides how the staged deltas round.
+  constexpr uint64_t kTwoPerSimd = 2048;
+  const bool two = R <= 32 && nspans / (256 / (uint64_t)R) < kTwoPerSimd;
+#define CTC_SYNC(NN)                                                                                             \
+  CTC_R_SWITCH(R, constexpr int kFew = RR <= 32 ? 2 : 4;                                                         \
+               (mixed ? launch_sync_as<RR, NN, true, 4> : two ? launch_sync_as<RR, NN, false, kFew>              \
+                                                              : launch_sync_as<RR, NN, false, 4>)(               \
+                   st, c, f, sy, span, sub, s, nspans, long_min, step, lam, block))
   if (nmodes == 3) {
-    if (mixed) {
-      CTC_SYNC_LAUNCH(3, true);
-    } else {
-      CTC_SYNC_LAUNCH(3, false);
-    }
-  } else if (nmodes == 4) {
-    if (mixed) {
-      CTC_SYNC_LAUNCH(4, true);
-    } else {
-      CTC_SYNC_LAUNCH(4, false);
-    }
+    CTC_SYNC(3);
   } else {
-    return hipErrorInvalidValue;
+    CTC_SYNC(4);
   }
-#undef CTC_SYNC_LAUNCH
+#undef CTC_SYNC
   return hipGetLastError();
 }
 

@@ -62,7 +62,7 @@ struct SyncArgs {
   uint32_t *ch[4];    // hot rows x kSyncReplicas
   float *stage[4];    // modes 1..: runs of one sub-step x R (BF16 entries on the mixed path)
   const uint32_t *sbase[4];  // modes 1..: first slot of each (sub-step, walker) chunk
-  const uint32_t *dest[4];   // modes 1.., mixed path: the sub-step's staging position of each slot (padded by one)
+  const uint32_t *dest[4];   // modes 1.., mixed path: the sub-step's staging position of each slot
 };
 
 // Staged merge of one sub-step (k_sgd_settle + k_sgd_fold).  Per staged
@@ -150,16 +150,19 @@ __device__ inline void wave_sync() {
 }
 
 // Sum across groups of W consecutive lanes (W in {1,2,...,64}); every lane of
-// the group receives the total.  DPP quad permutes for distances 1 and 2,
-// ds_swizzle (xor mode, within 32 lanes) for 4..16, ds_bpermute across halves.
+// the group receives the total.  DPP quad permutes for distances 1 and 2, DPP
+// mirrors of 8 and 16 lanes for 4 and 8 (the lanes of a quad, then of an
+// eight, hold the same sum by then), ds_swizzle for 16, ds_bpermute across halves.
 template <int W>
 __device__ inline float group_sum(float v) {
   if constexpr (W >= 2)
     v += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0xB1, 0xF, 0xF, false));
   if constexpr (W >= 4)
     v += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x4E, 0xF, 0xF, false));
-  if constexpr (W >= 8) v += __int_as_float(__builtin_amdgcn_ds_swizzle(__float_as_int(v), 0x101F));
-  if constexpr (W >= 16) v += __int_as_float(__builtin_amdgcn_ds_swizzle(__float_as_int(v), 0x201F));
+  if constexpr (W >= 8)
+    v += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x141, 0xF, 0xF, false));
+  if constexpr (W >= 16)
+    v += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x140, 0xF, 0xF, false));
   if constexpr (W >= 32) v += __int_as_float(__builtin_amdgcn_ds_swizzle(__float_as_int(v), 0x401F));
   if constexpr (W >= 64) v += __shfl_xor(v, 32, 64);
   return v;

@@ -798,7 +798,7 @@ static ctc_status ensure_sync(ctc_model *m, uint32_t span, uint32_t sub) {
     // every row's slots of a sub-step cut into pieces of at most kStagePiece
     // slots; a row of one piece is settled by it, the others are folded
     std::vector<uint32_t> piece_start, piece_row, slots(key.size());
-    std::vector<uint32_t> dest(key.size() + 1, 0);  // + 1: the walk reads one ahead
+    std::vector<uint32_t> dest(key.size());
     std::vector<FoldSeg> fold;
     std::vector<uint64_t> &poff = m->sgd_piece_off[k], &foff = m->sgd_fold_off[k];
     poff.assign(nsub + 1, 0);

@@ -140,3 +140,31 @@ def test_walk_row_sums(ctx, dims, nnz, R):
             got = G[mode].cpu().numpy()
             assert np.linalg.norm(got - want) < 1e-5 * np.linalg.norm(want), (mode, per_occ)
         assert loss == pytest.approx(wl, rel=1e-6)
+
+
+@pytest.mark.parametrize("R,mixed", [(8, False), (16, False), (16, True), (32, False), (32, True), (64, True), (128, False)])
+@pytest.mark.parametrize("dims,nnz,span,sub", [((1, 40, 30), 1, 2048, 32), ((40, 12, 9), 31, 2048, 32),
+                                               ((40, 12, 9), 700, 100, 33), ((9, 30, 6, 7), 3001, 256, 70),
+                                               ((3, 500, 400), 140_003, 8, 3), ((4000, 300, 80), 150_001, 64, 32)],
+                         ids=["one", "short", "odd_substep", "4way_rounds", "many_walkers", "short_rows"])
+def test_sgd_walk_rounds(ctx, dims, nnz, span, sub, R, mixed):
+    """The SGD walk with sub-steps of less than a round of nonzeros, of one
+    round and of several, with the walkers of part of a wave and of more waves than
+    two per SIMD (both lane shapes), runs that go on across rounds, and mode-0
+    rows in place and over walkers, against the oracle's schedule in 64 bits at the
+    parity tests' bars (1e-5; mixed 2e-4: a delta near a BF16 tie may round
+    the other way)."""
+    import oracle as O
+    say(f"[sgd walk] dims={dims} nnz={nnz} span={span} sub={sub} R={R} mixed={mixed}")
+    t, ind, vals = coo(dims, nnz, 21)
+    rng = np.random.default_rng(22)
+    F = [(0.5 * rng.uniform(-1, 1, (d, R))).astype(np.float32) for d in dims]
+    F64 = [f.astype(np.float64) for f in F]
+    oc = O.Coo(ind, vals, dims)
+    O.sgd_sync_epoch(oc, F64, 1e-3, 0.05, span, sub, 400, order=O.mode_order(oc, 0)[0], nthreads=4, mixed=mixed)
+    m = ct.Model(ctx, t, None, None, rank=R)
+    m.set_factors(F)
+    m.sgd_epoch(ct.Options(algorithm=ct.SGD, rank=R, lambda_=0.05, sgd_scale=1.0, tile_len=span, sgd_substep=sub,
+                           sgd_hot_rows=400, precision=ct.PREC_MIXED if mixed else ct.PREC_FP32), lr=1e-3)
+    for k, f in enumerate(F64):
+        assert np.linalg.norm(m.factor(k) - f) < (2e-4 if mixed else 1e-5) * np.linalg.norm(f), k
