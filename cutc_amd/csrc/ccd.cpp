@@ -7,7 +7,8 @@
 // subtraction of column f is deferred into the pass of column f+1 (or the next
 // epoch's column 0) so each (column, mode) costs one pass over the tensor.
 // At the start of column f every mode's per-row records are packed from the
-// column-major mirror: (pending column's new value, f saved, f current).
+// column-major mirror: (pending column's new value, f saved, f current); the
+// column's mirror is cleared there, so rows without nonzeros become 0.
 //
 // ccd_epoch_jacobi is the reference's own CCD form, run on request only.
 #include <algorithm>
@@ -52,8 +53,15 @@ ctc_status ccd_epoch_impl(ctc_model *m, const ctc_options *o) {
 
   const unsigned block = block_of(o);
   for (uint32_t f = 0; f < R; ++f) {
-    for (uint32_t md = 0; md < N; ++md)
-      CTC_HIP(launch_ccd_pack(st, m->FT[md], m->dims[md], (int)f, m->ccd_pending, (float4 *)m->ccdx[md]));
+    CcdPackArgs pk{};
+    for (uint32_t md = 0; md < 4; ++md) {
+      pk.ft[md] = md < N ? m->FT[md] : nullptr;
+      pk.x[md] = md < N ? (float4 *)m->ccdx[md] : nullptr;
+      pk.off[md + 1] = pk.off[md] + (md < N ? m->dims[md] : 0);
+    }
+    pk.col = (int)f;
+    pk.sub_col = m->ccd_pending;
+    CTC_HIP(launch_ccd_pack(st, pk));
     for (uint32_t it = 0; it < inner; ++it) {
       for (uint32_t md = 0; md < N; ++md) {
         const DevCiss &d = m->ciss[md];
@@ -80,11 +88,10 @@ ctc_status ccd_epoch_impl(ctc_model *m, const ctc_options *o) {
           Prof p(m->ctx, "ccd_col");
           CTC_HIP(launch_ccd_col(st, a, (int)N, block));
         }
-        CTC_HIP(launch_fill(st, col, m->dims[md], 0.f));  // rows with no nonzero -> 0
         {
           Prof p(m->ctx, "ccd_finish");
-          CTC_HIP(launch_ccd_finish(st, pieces, d.slot_pb, d.directory, d.dlength, d.npieces, o->lambda, col,
-                                    (float4 *)m->ccdx[md]));
+          CTC_HIP(launch_ccd_finish(st, pieces, d.slot_pb, d.heavy_slot, d.nheavy_slot, d.directory, d.dlength,
+                                    o->lambda, col, (float4 *)m->ccdx[md]));
         }
       }
     }

@@ -75,6 +75,8 @@ struct DevCiss {
   uint64_t nspans = 0, npieces = 0;
   uint32_t *span_off = nullptr;  // nspans: piece id = slot + span_off[span]
   uint32_t *slot_pb = nullptr;   // dlength + 1: pieces of slot s
+  uint32_t *heavy_slot = nullptr;  // slots of more than kHeavyPieces pieces
+  uint64_t nheavy_slot = 0;
   // heavy slots (more than kHeavyPieces pieces): their pieces are summed in
   // groups of consecutive pieces before the ALS solve
   uint64_t ngroups = 0;

@@ -23,11 +23,18 @@ struct CcdColArgs {
 constexpr uint32_t kCcdLdsRows = 2304;  // 36 KB of 16-byte records
 
 hipError_t launch_ccd_col(hipStream_t st, const CcdColArgs &a, int nmodes, unsigned block);
-// npieces: the mode's piece count (picks one lane or one wave per slot)
-hipError_t launch_ccd_finish(hipStream_t st, const double *pieces, const uint32_t *slot_pb,
-                             const uint32_t *directory, uint64_t dlength, uint64_t npieces, double lam,
-                             float *col, float4 *x);
-hipError_t launch_ccd_pack(hipStream_t st, const float *ft, uint64_t rows, int col, int sub_col, float4 *x);
+// heavy: the slots of more than kHeavyPieces pieces
+hipError_t launch_ccd_finish(hipStream_t st, const double *pieces, const uint32_t *slot_pb, const uint32_t *heavy,
+                             uint64_t nheavy, const uint32_t *directory, uint64_t dlength, double lam, float *col,
+                             float4 *x);
+// every mode's records at the start of a column's update
+struct CcdPackArgs {
+  float *ft[4];      // column-major mirrors
+  float4 *x[4];
+  uint64_t off[5];   // mode m: rows off[m] .. off[m + 1]
+  int col, sub_col;  // sub_col: the pending column (-1: none)
+};
+hipError_t launch_ccd_pack(hipStream_t st, const CcdPackArgs &a);
 hipError_t launch_ccd_resid(hipStream_t st, const CissArgs &c, const FactorArgs &f, int nmodes, int R,
                             float *resid);
 // F(row, :) <- num(row, :) / (lambda + den(row, :)) for the rows of a

@@ -19,11 +19,15 @@
 //
 // Reductions.  One wave walks a span of tiles, one lane per nonzero.  Row
 // sums inside a tile use a segmented inclusive scan (DPP row shifts and
-// ds_bpermute for the cross-row steps) with the row starts of the tile
-// mask as flags; the row still open at the end of a tile is carried in a
-// wave-uniform register into the next tile.  Completed rows are written as
-// (num, den) pieces with the same piece numbering as the ALS Gram pieces, so
-// the per-row sums have a fixed order (deterministic, no atomics).
+// broadcasts) that takes each lane's distance to its row's start from the tile
+// mask; the row still open at the end of a tile is carried in a wave-uniform
+// value into the next tile.  Completed rows are written as (num, den) pieces
+// with the same piece numbering as the ALS Gram pieces, so the per-row sums
+// have a fixed order (deterministic, no atomics).
+//
+// The three passes of a column over 20M nonzeros (480K x 18K x 2K): 135 / 172 /
+// 195 us (169 / 182 / 219 us with the scan on the LDS pipe and no tile in
+// flight); the 16 bytes per nonzero that a pass streams take 68 us.
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
@@ -33,27 +37,38 @@
 
 namespace ctc {
 
-// inclusive segmented scan over the wave: f = segment-start flag
-__device__ inline void seg_scan(float &a, float &b, bool f) {
-  const int lane = lane_id();
-#pragma unroll
-  for (int d = 1; d < 64; d <<= 1) {
-    const float ua = __shfl_up(a, d, 64);
-    const float ub = __shfl_up(b, d, 64);
-    const int uf = __shfl_up((int)f, d, 64);
-    if (lane >= d) {
-      if (!f) {
-        a += ua;
-        b += ub;
-      }
-      f = f || uf;
-    }
-  }
+// one step of the scan: x + the DPP source where the lane's segment reaches it
+// (a select, not a product: the other segments' sums may be infinite)
+template <int CTRL, int ROWS>
+__device__ inline float scan_step(float x, bool reach) {
+  const float u = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), CTRL, ROWS, 0xF, false));
+  return x + (reach ? u : 0.f);
 }
 
-// The pass of wave w over its span.  LS >= 0: the records of other mode LS
-// (a mode of at most kCcdLdsRows rows) are read from the workgroup's copy xs
-// in LDS instead of gathered from memory.
+// Inclusive segmented scan over the wave; dist = lanes from the start of the
+// lane's segment to it.  Row shifts within 16 lanes, then the row ends
+// broadcast to the next row and the half's end to the upper half: no LDS pipe
+// (18 ds_bpermute per tile before) and no flag to carry along.
+__device__ inline void seg_scan(float &a, float &b, int dist) {
+  const int lane = lane_id();
+  a = scan_step<0x111, 0xF>(a, dist >= 1), b = scan_step<0x111, 0xF>(b, dist >= 1);
+  a = scan_step<0x112, 0xF>(a, dist >= 2), b = scan_step<0x112, 0xF>(b, dist >= 2);
+  a = scan_step<0x114, 0xF>(a, dist >= 4), b = scan_step<0x114, 0xF>(b, dist >= 4);
+  a = scan_step<0x118, 0xF>(a, dist >= 8), b = scan_step<0x118, 0xF>(b, dist >= 8);
+  const bool r1 = dist > (lane & 15), r2 = dist > (lane & 31);
+  a = scan_step<0x142, 0xA>(a, r1), b = scan_step<0x142, 0xA>(b, r1);
+  a = scan_step<0x143, 0xC>(a, r2), b = scan_step<0x143, 0xC>(b, r2);
+}
+
+__device__ inline float lane_value(float x, uint32_t lane) {
+  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), (int)lane));
+}
+
+// The pass of wave w (uniform) over its span.  LS >= 0: the records of other
+// mode LS (a mode of at most kCcdLdsRows rows) are read from the workgroup's
+// copy xs in LDS instead of gathered from memory.  The indices and the
+// residual of tile t + 2 and the records of tile t + 1 are in flight while
+// tile t is summed.
 template <int N, int LS>
 __device__ __forceinline__ void ccd_col_wave(const CcdColArgs &a, uint64_t w, const float4 *xs) {
   const int lane = lane_id();
@@ -65,78 +80,90 @@ __device__ __forceinline__ void ccd_col_wave(const CcdColArgs &a, uint64_t w, co
   double carry_n = 0.0, carry_d = 0.0;
   uint32_t carry_slot = 0;
   bool have_carry = false;
+  double2 *pieces = reinterpret_cast<double2 *>(a.pieces);
 
+  uint32_t ix[N - 1], row = 0;  // of the tile after the next
+  float en;
+  auto indices = [&](uint64_t t) {
+    t = t < t1 ? t : t1 - 1;  // past the span: its last tile again, not used
+    const uint64_t at = t * kTile + lane, p = at < c.nnz ? at : c.nnz - 1;
+#pragma unroll
+    for (int s = 0; s < N - 1; ++s) ix[s] = c.oidx[s][p];
+    en = a.resid[p];
+    // lanes past the end take a valid row's slot too
+    if (fix) row = c.directory[tile_lane_slot(c.tile_slot[t], c.tile_mask[t], (int)(p & 63))];
+  };
+  float4 qn[N];
+  float e1;
+  uint32_t ln = 0;  // the record in LDS is read when its tile is summed
+  auto records = [&]() {
+#pragma unroll
+    for (int s = 0; s < N - 1; ++s)
+      if (s == LS)
+        ln = ix[s];
+      else
+        qn[1 + s] = a.x[1 + s][ix[s]];
+    if (fix) qn[0] = a.x[0][row];  // the own mode's row: pending and saved values
+    e1 = en;
+  };
+  indices(t0);
+  records();
+  indices(t0 + 1);
   for (uint64_t t = t0; t < t1; ++t) {
+    float4 q[N];
+#pragma unroll
+    for (int s = 0; s < N; ++s) q[s] = s == 1 + LS && LS >= 0 ? xs[ln] : qn[s];
+    float e = e1;
+    records();
+    indices(t + 2);
     const uint64_t base = t * kTile;
     const uint32_t cnt = (uint32_t)((c.nnz - base) < (uint64_t)kTile ? (c.nnz - base) : kTile);
     uint64_t mask = c.tile_mask[t];
     if (cnt < 64) mask &= (1ull << cnt) - 1ull;
     const uint32_t first_slot = c.tile_slot[t];
     const bool valid = (uint32_t)lane < cnt;
-    float num = 0.f, den = 0.f;
-    uint32_t myslot = first_slot;
-    if (valid) {
-      const uint64_t p = base + lane;
-      myslot = tile_lane_slot(first_slot, mask, lane);
-      float4 q[N];
+    if (fix) {
+      if (a.sub_col >= 0) {
+        float v = q[0].x;
 #pragma unroll
-      for (int s = 0; s < N - 1; ++s) q[1 + s] = s == LS ? xs[c.oidx[s][p]] : a.x[1 + s][c.oidx[s][p]];
-      float e = a.resid[p];
-      if (fix) {
-        q[0] = a.x[0][c.directory[myslot]];  // the own mode's row: pending and saved values
-        if (a.sub_col >= 0) {
-          float v = q[0].x;
-#pragma unroll
-          for (int s = 1; s < N; ++s) v *= q[s].x;
-          e -= v;
-        }
-        if (a.add_back) {
-          float v = q[0].y;
-#pragma unroll
-          for (int s = 1; s < N; ++s) v *= q[s].y;
-          e += v;
-        }
-        a.resid[p] = e;
+        for (int s = 1; s < N; ++s) v *= q[s].x;
+        e -= v;
       }
-      float h = q[1].z;
+      if (a.add_back) {
+        float v = q[0].y;
 #pragma unroll
-      for (int s = 2; s < N; ++s) h *= q[s].z;
-      num = e * h;
-      den = h * h;
+        for (int s = 1; s < N; ++s) v *= q[s].y;
+        e += v;
+      }
+      if (valid) a.resid[base + lane] = e;
     }
-    const bool head = valid && ((mask >> lane) & 1ull);
-    seg_scan(num, den, lane == 0 || head);
+    float h = q[1].z;
+#pragma unroll
+    for (int s = 2; s < N; ++s) h *= q[s].z;
+    float num = valid ? e * h : 0.f, den = valid ? h * h : 0.f;
+    const uint64_t upto = (mask | 1ull) & (lane == 63 ? ~0ull : (2ull << lane) - 1ull);
+    seg_scan(num, den, lane - (63 - __clzll((long long)upto)));
 
     // first segment: lanes [0, fh); fh = first row start after lane 0
     const uint64_t later = mask & ~1ull;
     const uint32_t fh = later ? (uint32_t)__ffsll((unsigned long long)later) - 1u : cnt;
     const bool join = (t > t0) && !(mask & 1ull);  // lane 0 continues the carried row
     if (have_carry && !join) {
-      if (lane == 0) {
-        a.pieces[(size_t)(carry_slot + poff) * 2] = carry_n;
-        a.pieces[(size_t)(carry_slot + poff) * 2 + 1] = carry_d;
-      }
+      if (lane == 0) pieces[carry_slot + poff] = make_double2(carry_n, carry_d);
       have_carry = false;
       carry_n = carry_d = 0.0;
     }
-    const double fn = (double)__shfl(num, (int)fh - 1, 64) + (join ? carry_n : 0.0);
-    const double fd = (double)__shfl(den, (int)fh - 1, 64) + (join ? carry_d : 0.0);
+    const double fn = (double)lane_value(num, fh - 1) + (join ? carry_n : 0.0);
+    const double fd = (double)lane_value(den, fh - 1) + (join ? carry_d : 0.0);
     if (fh < cnt) {
-      if (lane == 0) {
-        a.pieces[(size_t)(first_slot + poff) * 2] = fn;
-        a.pieces[(size_t)(first_slot + poff) * 2 + 1] = fd;
-      }
+      if (lane == 0) pieces[first_slot + poff] = make_double2(fn, fd);
       // complete middle segments end at lanes i in [fh, cnt-1) whose next lane
       // starts a row; the last segment (ending at cnt-1) becomes the carry
-      const bool tail = valid && (uint32_t)lane >= fh && (uint32_t)lane + 1 < cnt &&
-                        ((mask >> (lane + 1)) & 1ull);
-      if (tail) {
-        a.pieces[(size_t)(myslot + poff) * 2] = (double)num;
-        a.pieces[(size_t)(myslot + poff) * 2 + 1] = (double)den;
-      }
-      carry_n = (double)__shfl(num, (int)cnt - 1, 64);
-      carry_d = (double)__shfl(den, (int)cnt - 1, 64);
-      carry_slot = (uint32_t)__shfl((int)myslot, (int)cnt - 1, 64);
+      const bool tail = (uint32_t)lane >= fh && (uint32_t)lane + 1 < cnt && ((mask >> (lane + 1)) & 1ull);
+      if (tail) pieces[tile_lane_slot(first_slot, mask, lane) + poff] = make_double2((double)num, (double)den);
+      carry_n = (double)lane_value(num, cnt - 1);
+      carry_d = (double)lane_value(den, cnt - 1);
+      carry_slot = tile_lane_slot(first_slot, mask, (int)cnt - 1);
     } else {
       carry_n = fn;
       carry_d = fd;
@@ -144,15 +171,17 @@ __device__ __forceinline__ void ccd_col_wave(const CcdColArgs &a, uint64_t w, co
     }
     have_carry = true;
   }
-  if (have_carry && lane == 0) {
-    a.pieces[(size_t)(carry_slot + poff) * 2] = carry_n;
-    a.pieces[(size_t)(carry_slot + poff) * 2 + 1] = carry_d;
-  }
+  if (have_carry && lane == 0) pieces[carry_slot + poff] = make_double2(carry_n, carry_d);
+}
+
+// the wave's span, as the uniform value it is: the tile words are scalar loads
+__device__ inline uint64_t wave_index() {
+  return (uint64_t)blockIdx.x * (blockDim.x >> 6) + (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
 }
 
 template <int N>
 __global__ void __launch_bounds__(256) k_ccd_col(CcdColArgs a) {
-  const uint64_t w = (uint64_t)blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
+  const uint64_t w = wave_index();
   if (w >= a.nspans) return;
   ccd_col_wave<N, -1>(a, w, nullptr);
 }
@@ -160,12 +189,12 @@ __global__ void __launch_bounds__(256) k_ccd_col(CcdColArgs a) {
 // 1024-thread workgroups (16 spans) sharing one LDS copy of the records of a
 // small other mode: its gathers no longer go through the texture addresser.
 template <int N, int LS>
-__global__ void __launch_bounds__(1024) k_ccd_col_lds(CcdColArgs a) {
+__global__ void __launch_bounds__(1024, 8) k_ccd_col_lds(CcdColArgs a) {
   __shared__ float4 xs[kCcdLdsRows];
   const float4 *src = a.x[1 + LS];
   for (uint32_t i = threadIdx.x; i < a.lds_rows; i += blockDim.x) xs[i] = src[i];
   __syncthreads();
-  const uint64_t w = (uint64_t)blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
+  const uint64_t w = wave_index();
   if (w >= a.nspans) return;
   ccd_col_wave<N, LS>(a, w, xs);
 }
@@ -209,61 +238,46 @@ __device__ inline void ccd_finish_wave(uint64_t slot, const double *pieces, cons
   if (lane == 0) ccd_finish_slot(slot, n, d, directory, lam, col, x);
 }
 
+// Blocks 0 .. hb - 1 take the slots of more than kHeavyPieces pieces (listed by
+// the host), a wave each as above; the blocks after them 256 consecutive slots
+// each, a lane per slot, whose few pieces are added in piece order.  The slots,
+// their rows and their records are consecutive, so the kernel is a stream; with
+// the slots dealt to the blocks in a stride, which kept the long rows (the
+// hottest are numbered first) apart, 480K slots took 25 us; now 9 us.
 __global__ void __launch_bounds__(256) k_ccd_finish(const double *pieces, const uint32_t *slot_pb,
-                                                    const uint32_t *directory, uint64_t dlength,
-                                                    double lam, float *col, float4 *x) {
-  const uint64_t s = (uint64_t)blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
-  if (s < dlength) ccd_finish_wave(s, pieces, slot_pb, directory, lam, col, x);
-}
-
-// For modes whose slots hold about one piece (mode 0 of the benchmark tensor:
-// 480K rows, each meeting a span boundary rarely): a block takes 256 slots;
-// a slot of at most kFinishLight pieces is summed by its own lane in piece
-// order, the heavier ones are listed in LDS and summed by a wave each as
-// above.  Measured per pass on the benchmark tensor: mode 0 35.5 us (129 us
-// with a wave for every slot, 119 us with 256 consecutive slots per block,
-// where the hottest rows, numbered first, queued in the first blocks); the
-// other modes, whose slots hold tens to thousands of pieces, 9 us with a wave
-// per slot and longer with lanes.
-constexpr uint32_t kFinishLight = 8;
-
-__global__ void __launch_bounds__(256) k_ccd_finish_light(const double *pieces, const uint32_t *slot_pb,
-                                                          const uint32_t *directory, uint64_t dlength,
-                                                          double lam, float *col, float4 *x) {
-  __shared__ uint32_t heavy[256];
-  __shared__ uint32_t nheavy;
-  // slots are dealt to the blocks in a stride (block b takes b, b + G, ...):
-  // the long rows are the hottest, numbered first, and land in different
-  // blocks instead of queueing in the first ones
-  const uint64_t s = (uint64_t)blockIdx.x + (uint64_t)threadIdx.x * gridDim.x;
-  if (threadIdx.x == 0) nheavy = 0;
-  __syncthreads();
-  if (s < dlength) {
-    const uint32_t p0 = slot_pb[s], p1 = slot_pb[s + 1];
-    if (p1 - p0 <= kFinishLight) {
-      double n = 0.0, d = 0.0;
-      for (uint32_t p = p0; p < p1; ++p) {
-        const double2 q = reinterpret_cast<const double2 *>(pieces)[p];
-        n += q.x;
-        d += q.y;
-      }
-      ccd_finish_slot(s, n, d, directory, lam, col, x);
-    } else {
-      heavy[atomicAdd(&nheavy, 1u)] = threadIdx.x;
-    }
+                                                    const uint32_t *heavy, uint64_t nheavy, uint32_t hb,
+                                                    const uint32_t *directory, uint64_t dlength, double lam,
+                                                    float *col, float4 *x) {
+  if (blockIdx.x < hb) {
+    const uint64_t h = (uint64_t)blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
+    if (h < nheavy) ccd_finish_wave(heavy[h], pieces, slot_pb, directory, lam, col, x);
+    return;
   }
-  __syncthreads();
-  for (uint32_t h = threadIdx.x >> 6; h < nheavy; h += blockDim.x >> 6)
-    ccd_finish_wave((uint64_t)blockIdx.x + (uint64_t)heavy[h] * gridDim.x, pieces, slot_pb, directory, lam, col, x);
+  const uint64_t s = (uint64_t)(blockIdx.x - hb) * 256 + threadIdx.x;
+  if (s >= dlength) return;
+  const uint32_t p0 = slot_pb[s], p1 = slot_pb[s + 1];
+  if (p1 - p0 > kHeavyPieces) return;
+  double n = 0.0, d = 0.0;
+  for (uint32_t p = p0; p < p1; ++p) {
+    const double2 q = reinterpret_cast<const double2 *>(pieces)[p];
+    n += q.x;
+    d += q.y;
+  }
+  ccd_finish_slot(s, n, d, directory, lam, col, x);
 }
 
-// per-row records of column `col` at the start of its update
-__global__ void __launch_bounds__(256) k_ccd_pack(const float *ft, uint64_t rows, int col, int sub_col, float4 *x) {
-  const float *cur = ft + (size_t)col * rows;
-  const float *sub = sub_col >= 0 ? ft + (size_t)sub_col * rows : nullptr;
-  for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < rows; i += (uint64_t)gridDim.x * blockDim.x) {
-    const float v = cur[i];
-    x[i] = make_float4(sub ? sub[i] : 0.f, v, v, 0.f);
+// per-row records of every mode at the start of a column's update; the column's
+// mirror is cleared for the rows without nonzeros, the finish writes the others
+__global__ void __launch_bounds__(256) k_ccd_pack(CcdPackArgs a) {
+  const uint64_t n = a.off[4];
+  for (uint64_t p = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; p < n; p += (uint64_t)gridDim.x * blockDim.x) {
+    int m = 0;
+    while (m < 3 && p >= a.off[m + 1]) ++m;
+    const uint64_t i = p - a.off[m], rows = a.off[m + 1] - a.off[m];
+    float *cur = a.ft[m] + (size_t)a.col * rows + i;
+    const float v = *cur;
+    a.x[m][i] = make_float4(a.sub_col >= 0 ? a.ft[m][(size_t)a.sub_col * rows + i] : 0.f, v, v, 0.f);
+    *cur = 0.f;
   }
 }
 
@@ -350,24 +364,21 @@ hipError_t launch_ccd_col(hipStream_t st, const CcdColArgs &a, int nmodes, unsig
   return hipGetLastError();
 }
 
-hipError_t launch_ccd_finish(hipStream_t st, const double *pieces, const uint32_t *slot_pb,
-                             const uint32_t *directory, uint64_t dlength, uint64_t npieces, double lam,
-                             float *col, float4 *x) {
+hipError_t launch_ccd_finish(hipStream_t st, const double *pieces, const uint32_t *slot_pb, const uint32_t *heavy,
+                             uint64_t nheavy, const uint32_t *directory, uint64_t dlength, double lam, float *col,
+                             float4 *x) {
   if (dlength == 0) return hipSuccess;
-  if (npieces <= 2 * dlength)  // about one piece per slot
-    hipLaunchKernelGGL(k_ccd_finish_light, dim3((unsigned)((dlength + 255) / 256)), dim3(256), 0, st, pieces,
-                       slot_pb, directory, dlength, lam, col, x);
-  else
-    hipLaunchKernelGGL(k_ccd_finish, dim3((unsigned)((dlength + 3) / 4)), dim3(256), 0, st, pieces, slot_pb,
-                       directory, dlength, lam, col, x);
+  const uint32_t hb = (uint32_t)((nheavy + 3) / 4);
+  hipLaunchKernelGGL(k_ccd_finish, dim3(hb + (unsigned)((dlength + 255) / 256)), dim3(256), 0, st, pieces, slot_pb,
+                     heavy, nheavy, hb, directory, dlength, lam, col, x);
   return hipGetLastError();
 }
 
-hipError_t launch_ccd_pack(hipStream_t st, const float *ft, uint64_t rows, int col, int sub_col, float4 *x) {
-  if (rows == 0) return hipSuccess;
-  uint64_t blocks = (rows + 255) / 256;
+hipError_t launch_ccd_pack(hipStream_t st, const CcdPackArgs &a) {
+  if (a.off[4] == 0) return hipSuccess;
+  uint64_t blocks = (a.off[4] + 255) / 256;
   if (blocks > 4096) blocks = 4096;
-  hipLaunchKernelGGL(k_ccd_pack, dim3((unsigned)blocks), dim3(256), 0, st, ft, rows, col, sub_col, x);
+  hipLaunchKernelGGL(k_ccd_pack, dim3((unsigned)blocks), dim3(256), 0, st, a);
   return hipGetLastError();
 }
 

@@ -84,6 +84,8 @@ constexpr uint32_t kStagePiece = 1024;
 // rows of at most this many runs in a sub-step are settled by one walker each
 // (most rows of a skewed mode); longer ones by a workgroup per piece
 constexpr uint32_t kSettleLight = 32;
+// slots of more span pieces than this are summed by more than one lane or wave
+constexpr uint32_t kHeavyPieces = 8;
 struct FoldSeg {
   uint32_t row, piece, npiece, runs;  // piece: first piece, sub-step relative
 };

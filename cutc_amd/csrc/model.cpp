@@ -155,7 +155,7 @@ ctc_status ensure_ciss(ctc_model *m, uint32_t mode) {
 static void free_dev_ciss(DevCiss &d) {
   for (int s = 0; s < 3; ++s) dev_free(d.oidx[s]);
   for (void *p : {(void *)d.vals, (void *)d.tile_slot, (void *)d.tile_mask, (void *)d.directory, (void *)d.rowptr,
-                  (void *)d.span_off, (void *)d.slot_pb, (void *)d.grp_piece, (void *)d.grp_n, (void *)d.slot_gb,
+                  (void *)d.span_off, (void *)d.slot_pb, (void *)d.grp_piece, (void *)d.grp_n, (void *)d.slot_gb, (void *)d.heavy_slot,
                   (void *)d.mix_items, (void *)d.mix_heavy_slot, (void *)d.mix_heavy_pb, (void *)d.mix_grp,
                   (void *)d.mix_heavy_gb})
     dev_free(p);
@@ -212,12 +212,12 @@ ctc_status ensure_pieces(ctc_model *m, uint32_t mode, uint32_t span_tiles) {
   pb[d.dlength] = (uint32_t)base;
   // group tables for heavy slots: about as many groups as pieces per group, so
   // that the reduction and the solve each add the square root of the pieces
-  constexpr uint32_t kHeavyPieces = 8;
-  std::vector<uint32_t> gpiece, gn, gb(d.dlength + 1);
+  std::vector<uint32_t> gpiece, gn, gb(d.dlength + 1), heavy;
   for (uint64_t s = 0; s < d.dlength; ++s) {
     gb[s] = (uint32_t)gpiece.size();
     const uint32_t n = pb[s + 1] - pb[s];
     if (n <= kHeavyPieces) continue;
+    heavy.push_back((uint32_t)s);
     const uint32_t per = std::max(kHeavyPieces, (uint32_t)std::ceil(std::sqrt((double)n)));
     for (uint32_t q = 0; q < n; q += per) {
       gpiece.push_back(pb[s] + q);
@@ -230,10 +230,13 @@ ctc_status ensure_pieces(ctc_model *m, uint32_t mode, uint32_t span_tiles) {
   dev_free(d.grp_piece);
   dev_free(d.grp_n);
   dev_free(d.slot_gb);
-  d.span_off = d.slot_pb = d.grp_piece = d.grp_n = d.slot_gb = nullptr;
+  dev_free(d.heavy_slot);
+  d.span_off = d.slot_pb = d.grp_piece = d.grp_n = d.slot_gb = d.heavy_slot = nullptr;
   hipStream_t st = m->ctx->stream;
   CTC_TRY(upload(&d.span_off, off.data(), nspans, st));
   CTC_TRY(upload(&d.slot_pb, pb.data(), d.dlength + 1, st));
+  d.nheavy_slot = heavy.size();
+  CTC_TRY(upload(&d.heavy_slot, heavy.data(), heavy.size(), st));
   d.ngroups = gpiece.size();
   if (d.ngroups) {
     CTC_TRY(upload(&d.grp_piece, gpiece.data(), d.ngroups, st));
