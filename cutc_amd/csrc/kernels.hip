@@ -232,7 +232,7 @@ __global__ void __launch_bounds__(256) k_sgd(CissArgs c, FactorArgs fa, HotRows 
 //     integers (2^-32 units) into its delta sum D (integer addition is
 //     associative, so the sum does not depend on the order the walkers finish
 //     in), a hot row's into kSyncReplicas replicas with a count of runs, and
-//     k_sgd_fold adds the sum (cold) or the mean (hot) and clears them.
+//     k_sgd_settle adds the sum (cold) or the mean (hot) and clears them.
 // ==========================================================================
 constexpr double kFixScale = 4294967296.0;        // 2^32
 constexpr double kFixInv = 1.0 / 4294967296.0;    // 2^-32
@@ -267,26 +267,8 @@ __device__ inline void store_row4(float *p, const float (&v)[CPL]) {
 // past the caches.
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
-template <int CPL>
-__device__ inline void load_row4_nt(const float *p, float (&v)[CPL]) {
-#pragma unroll
-  for (int j = 0; j < CPL; j += 4) {
-    const f32x4 t = __builtin_nontemporal_load(reinterpret_cast<const f32x4 *>(p + j));
-    v[j] = t.x, v[j + 1] = t.y, v[j + 2] = t.z, v[j + 3] = t.w;
-  }
-}
-
 // Four BF16 entries per lane (8 bytes): the mixed path's staged deltas.
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
-
-template <int CPL>
-__device__ inline void load_bf4_nt(const uint16_t *p, float (&v)[CPL]) {
-#pragma unroll
-  for (int j = 0; j < CPL; j += 4) {
-    const u32x2 t = __builtin_nontemporal_load(reinterpret_cast<const u32x2 *>(p + j));
-    v[j] = bf_lo(t.x), v[j + 1] = bf_hi(t.x), v[j + 2] = bf_lo(t.y), v[j + 3] = bf_hi(t.y);
-  }
-}
 
 // Lane shape of the SGD walk: a lane holds CPL elements of a row.  A walker's
 // time is its chain of instructions per nonzero, which is shorter with two
@@ -560,9 +542,16 @@ __device__ inline void sgd_merge_block(const MergeArgs &a, uint64_t blk) {
   const int m = a.mode[g];
   const uint64_t k = i - a.off[g];
   if (a.is_hot[g]) {
-    // hot row k of mode m: sum its replicas, add the mean of its runs' deltas
+    // hot row k of mode m: sum its replicas, add the mean of its runs' deltas;
+    // the loads of eight replicas at a time, the clearing after them
+    static_assert(kSyncReplicas % 8 == 0, "replicas are read in eights");
     uint32_t cnt = 0;
-    for (int r = 0; r < kSyncReplicas; ++r) cnt += a.ch[m][k * kSyncReplicas + r];
+    const uint4 *ch = reinterpret_cast<const uint4 *>(a.ch[m] + k * kSyncReplicas);
+#pragma unroll
+    for (int r = 0; r < kSyncReplicas / 4; ++r) {
+      const uint4 t = ch[r];
+      cnt += (t.x + t.y) + (t.z + t.w);
+    }
     if (cnt == 0) return;
     const uint32_t row = a.hrow[m][k];
     float *gr = a.F[m] + (size_t)row * R;
@@ -572,10 +561,16 @@ __device__ inline void sgd_merge_block(const MergeArgs &a, uint64_t blk) {
     for (int j = 0; j < CPL; ++j) {
       const int col = wl + j * W;
       long long sum = 0;
-      for (int r = 0; r < kSyncReplicas; ++r) {
-        sum += d[(size_t)r * R + col];
-        d[(size_t)r * R + col] = 0;
+#pragma unroll
+      for (int r = 0; r < kSyncReplicas; r += 8) {
+        long long x[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) x[u] = d[(size_t)(r + u) * R + col];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) sum += x[u];
       }
+#pragma unroll
+      for (int r = 0; r < kSyncReplicas; ++r) d[(size_t)r * R + col] = 0;
       gr[col] = (float)((double)gr[col] + (double)sum * kFixInv * sc);
     }
     if (wl < kSyncReplicas) a.ch[m][k * kSyncReplicas + wl] = 0u;
@@ -598,12 +593,48 @@ __device__ inline void sgd_merge_block(const MergeArgs &a, uint64_t blk) {
   }
 }
 
-// One launch per sub-step settles every piece of the staged modes: a
-// workgroup per piece, whose walkers take the piece's positions in turn
-// (FP64 partial sums) and add their partials in
-// walker order.  A piece that holds a whole row applies it; the others leave
-// their sums for k_sgd_fold.  The order is fixed, so the result is
-// reproducible.
+// acc += the staged deltas at positions p, p + stride, ... before e, in that
+// order, in FP64.  FP32 deltas sit at their slot, BF16 ones at the position
+// itself (positions are numbered over the epoch, s0 is the sub-step's first).
+// What a long list waits for is its round trips, so eight deltas are in flight,
+// and their slots are read while the eight before them are.
+template <int R, bool MIX>
+__device__ inline void sum_staged(const float *stage, const uint32_t *slots, uint32_t s0, uint32_t p, uint32_t e,
+                                  uint32_t stride, int col, double (&acc)[SyncShape<R>::CPL]) {
+  constexpr int CPL = SyncShape<R>::CPL, U = 8;
+  static_assert(CPL == 4, "a lane's share of a delta is one 16-byte (BF16: 8-byte) load");
+  uint32_t at[U];
+  auto slot = [&](uint32_t q) -> uint32_t { return q >= e ? 0u : MIX ? q - s0 : slots[q]; };
+#pragma unroll
+  for (int u = 0; u < U; ++u) at[u] = slot(p + u * stride);
+  for (; p < e; p += U * stride) {
+    u32x2 xb[U];  // BF16 deltas as they are stored
+    f32x4 xf[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      if (p + u * stride < e) {
+        const size_t i = (size_t)at[u] * R + col;
+        if constexpr (MIX)
+          xb[u] = __builtin_nontemporal_load(reinterpret_cast<const u32x2 *>(reinterpret_cast<const uint16_t *>(stage) + i));
+        else
+          xf[u] = __builtin_nontemporal_load(reinterpret_cast<const f32x4 *>(stage + i));
+      }
+#pragma unroll
+    for (int u = 0; u < U; ++u) at[u] = slot(p + (U + u) * stride);
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      if (p + u * stride < e) {
+        if constexpr (MIX) {
+          acc[0] += (double)bf_lo(xb[u].x), acc[1] += (double)bf_hi(xb[u].x);
+          acc[2] += (double)bf_lo(xb[u].y), acc[3] += (double)bf_hi(xb[u].y);
+        } else {
+#pragma unroll
+          for (int j = 0; j < CPL; ++j) acc[j] += (double)xf[u][j];
+        }
+      }
+  }
+}
+
 // A row of at most kSettleLight runs, settled by one walker (W lanes) of
 // light block lblk: its runs' deltas summed in position order in FP64, the
 // sum (cold row) or the mean (hot row) added to the row.
@@ -620,10 +651,6 @@ __device__ inline void sgd_settle_light(const SettleArgs &a, uint64_t lblk) {
   const uint32_t gp = a.light[k][li - a.lb[k]];
   const uint32_t b = a.piece_start[k][gp], e = a.piece_start[k][gp + 1];
   const uint32_t row = a.piece_row[k][gp];
-  const float *stage = a.stage[k];
-  const uint32_t s0 = (uint32_t)a.slot0[k];
-  const uint32_t *slots = a.slots[k];
-  auto at = [&](uint32_t q) -> size_t { return MIX ? (size_t)(q - s0) : (size_t)slots[q]; };
   float *fr = a.F[k] + (size_t)row * R + wl * CPL;
   float fv[CPL];
   load_row4<CPL>(fr, fv);
@@ -631,30 +658,7 @@ __device__ inline void sgd_settle_light(const SettleArgs &a, uint64_t lblk) {
   double acc[CPL];
 #pragma unroll
   for (int j = 0; j < CPL; ++j) acc[j] = 0.0;
-  uint32_t p = b;
-  for (; p + 3 < e; p += 4) {  // four slots in flight, added in position order
-    float x[4][CPL];
-#pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      if constexpr (MIX)
-        load_bf4_nt<CPL>(reinterpret_cast<const uint16_t *>(stage) + at(p + u) * R + wl * CPL, x[u]);
-      else
-        load_row4_nt<CPL>(stage + at(p + u) * R + wl * CPL, x[u]);
-    }
-#pragma unroll
-    for (int u = 0; u < 4; ++u)
-#pragma unroll
-      for (int j = 0; j < CPL; ++j) acc[j] += (double)x[u][j];
-  }
-  for (; p < e; ++p) {
-    float x[CPL];
-    if constexpr (MIX)
-      load_bf4_nt<CPL>(reinterpret_cast<const uint16_t *>(stage) + at(p) * R + wl * CPL, x);
-    else
-      load_row4_nt<CPL>(stage + at(p) * R + wl * CPL, x);
-#pragma unroll
-    for (int j = 0; j < CPL; ++j) acc[j] += (double)x[j];
-  }
+  sum_staged<R, MIX>(a.stage[k], a.slots[k], (uint32_t)a.slot0[k], b, e, 1, wl * CPL, acc);
   const double sc = ((hw >> (row & 31)) & 1u) ? 1.0 / (double)(e - b) : 1.0;
   float out[CPL];
 #pragma unroll
@@ -662,10 +666,21 @@ __device__ inline void sgd_settle_light(const SettleArgs &a, uint64_t lblk) {
   store_row4<CPL>(fr, out);
 }
 
-// Blocks 0 .. pb[4] - 1: one heavy piece each (a workgroup sums its slots);
-// the blocks after them: NW light rows each (sgd_settle_light).
+// One launch per sub-step settles every piece of the staged modes and mode 0's
+// long rows.  Blocks 0 .. pb[4] - 1: one heavy piece each, whose walkers take
+// the piece's positions in turn (FP64 partial sums) and add their partials in
+// walker order; a piece that holds a whole row applies it, the others leave
+// their sums for k_sgd_fold.  The next nb_light blocks: NW light rows each
+// (sgd_settle_light).  The rest: mode 0 (sgd_merge_block).  Every order is
+// fixed, so the result is reproducible.  Both lists are sorted by their runs,
+// longest first: the walkers of a wave have like counts, and the long pieces
+// do not start last.  Bound by the round trips of the longest lists, then by the
+// staged deltas (12.5M nonzeros at R = 32: 50 MB): 15.8 us a sub-step (21.4 us
+// unsorted, with four deltas in flight; 16.9 us with four and eight waves per
+// SIMD), 50M nonzeros 30.9 us (34.4 us), 200 MB at 6.5 TB/s.  With mode 0 here,
+// k_sgd_fold (5 us) runs only where a row has several pieces.
 template <int R, bool MIX>
-__global__ void __launch_bounds__(256) k_sgd_settle(SettleArgs a) {
+__global__ void __launch_bounds__(256, MIX ? 8 : 6) k_sgd_settle(SettleArgs a) {
   constexpr int CPL = SyncShape<R>::CPL;  // a slot's row moves as 16-byte pieces
   constexpr int W = SyncShape<R>::W;
   constexpr int NW = 256 / W;  // walkers per workgroup
@@ -673,8 +688,11 @@ __global__ void __launch_bounds__(256) k_sgd_settle(SettleArgs a) {
   __shared__ double part[NW][R];
   __shared__ double red[G][R];
   const uint64_t pblk = blockIdx.x;
-  if (pblk >= a.pb[4]) {  // uniform per block: the light path has no barrier
-    sgd_settle_light<R, MIX>(a, pblk - a.pb[4]);
+  if (pblk >= a.pb[4]) {  // uniform per block: these paths have no barrier
+    if (pblk < a.pb[4] + a.nb_light)
+      sgd_settle_light<R, MIX>(a, pblk - a.pb[4]);
+    else
+      sgd_merge_block<R>(a.mg, pblk - a.pb[4] - a.nb_light);
     return;
   }
   int k = 1;
@@ -683,11 +701,6 @@ __global__ void __launch_bounds__(256) k_sgd_settle(SettleArgs a) {
   const int wid = threadIdx.x / W;
   const int wl = threadIdx.x % W;
   const uint32_t b = a.piece_start[k][gp], e = a.piece_start[k][gp + 1];
-  const float *stage = a.stage[k];
-  const uint32_t s0 = (uint32_t)a.slot0[k];  // positions are numbered over the epoch
-  const uint32_t *slots = a.slots[k];
-  // the staged delta at position q: FP32 at its slot, BF16 at q itself
-  auto at = [&](uint32_t q) -> size_t { return MIX ? (size_t)(q - s0) : (size_t)slots[q]; };
   // a whole row's factor entry and hot bit, read while the slots are summed
   const uint32_t row = a.piece_row[k][gp];
   float fv = 0.f;
@@ -699,30 +712,7 @@ __global__ void __launch_bounds__(256) k_sgd_settle(SettleArgs a) {
   double acc[CPL];
 #pragma unroll
   for (int j = 0; j < CPL; ++j) acc[j] = 0.0;
-  uint32_t p = b + wid;
-  for (; p + 3 * NW < e; p += 4 * NW) {  // four independent slots in flight
-    float x[4][CPL];
-#pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      if constexpr (MIX)
-        load_bf4_nt<CPL>(reinterpret_cast<const uint16_t *>(stage) + at(p + u * NW) * R + wl * CPL, x[u]);
-      else
-        load_row4_nt<CPL>(stage + at(p + u * NW) * R + wl * CPL, x[u]);
-    }
-#pragma unroll
-    for (int u = 0; u < 4; ++u)
-#pragma unroll
-      for (int j = 0; j < CPL; ++j) acc[j] += (double)x[u][j];
-  }
-  for (; p < e; p += NW) {
-    float x[CPL];
-    if constexpr (MIX)
-      load_bf4_nt<CPL>(reinterpret_cast<const uint16_t *>(stage) + at(p) * R + wl * CPL, x);
-    else
-      load_row4_nt<CPL>(stage + at(p) * R + wl * CPL, x);
-#pragma unroll
-    for (int j = 0; j < CPL; ++j) acc[j] += (double)x[j];
-  }
+  sum_staged<R, MIX>(a.stage[k], a.slots[k], (uint32_t)a.slot0[k], b + wid, e, NW, wl * CPL, acc);
 #pragma unroll
   for (int j = 0; j < CPL; ++j) part[wid][wl * CPL + j] = acc[j];
   __syncthreads();
@@ -749,21 +739,16 @@ __global__ void __launch_bounds__(256) k_sgd_settle(SettleArgs a) {
   }
 }
 
-// Blocks 0 .. nb_merge - 1 merge mode 0's long rows (sgd_merge_block); after
-// them one walker per staged row of more than one piece adds its pieces'
-// partial sums in order, then the total (a cold row) or the total over its
-// count of runs (a hot row) to the row.
+// One walker per staged row of more than one piece adds its pieces' partial
+// sums in order, then the total (a cold row) or the total over its count of
+// runs (a hot row) to the row.
 template <int R>
 __global__ void __launch_bounds__(256) k_sgd_fold(SettleArgs a) {
   constexpr int W = R < 64 ? R : 64;
   constexpr int CPL = R / W;
   constexpr int WPW = 64 / W;
-  if (blockIdx.x < a.nb_merge) {
-    sgd_merge_block<R>(a.mg, blockIdx.x);
-    return;
-  }
   const int wl = lane_id() % W;
-  const uint64_t i = ((uint64_t)(blockIdx.x - a.nb_merge) * (blockDim.x >> 6) + (threadIdx.x >> 6)) * WPW + lane_id() / W;
+  const uint64_t i = ((uint64_t)blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6)) * WPW + lane_id() / W;
   int k = 1;
   while (k < 3 && i >= a.fb[k + 1]) ++k;
   if (i >= a.fb[k + 1]) return;
@@ -772,6 +757,7 @@ __global__ void __launch_bounds__(256) k_sgd_fold(SettleArgs a) {
   double t[CPL];
 #pragma unroll
   for (int j = 0; j < CPL; ++j) t[j] = 0.0;
+#pragma unroll 4
   for (uint32_t q = 0; q < sg.npiece; ++q)
 #pragma unroll
     for (int j = 0; j < CPL; ++j) t[j] += pt[(size_t)(sg.piece + q) * R + wl + j * W];
@@ -1677,9 +1663,9 @@ hipError_t launch_sgd_sync(hipStream_t st, const CissArgs &c, const FactorArgs &
 hipError_t launch_sgd_settle(hipStream_t st, SettleArgs a, int R, bool mixed) {
   const int W = R < 64 ? R : 64;
   const uint64_t items = a.mg.off[a.mg.nseg];
-  a.nb_merge = grid_for((items + (64 / W) - 1) / (64 / W), 256);
   const uint64_t nw = 1024 / (uint64_t)R;  // light rows per block: 256 / (R / 4) walkers
-  const uint64_t sb = a.pb[4] + (a.lb[4] + nw - 1) / nw;
+  a.nb_light = (a.lb[4] + nw - 1) / nw;
+  const uint64_t sb = a.pb[4] + a.nb_light + grid_for((items + (64 / W) - 1) / (64 / W), 256);
   if (sb > 0x7FFFFFFFull) return hipErrorInvalidValue;
   if (sb > 0) {
     if (mixed) {
@@ -1688,7 +1674,7 @@ hipError_t launch_sgd_settle(hipStream_t st, SettleArgs a, int R, bool mixed) {
       CTC_R_SWITCH(R, hipLaunchKernelGGL((k_sgd_settle<RR, false>), dim3((unsigned)sb), dim3(256), 0, st, a));
     }
   }
-  const uint64_t fg = a.nb_merge + grid_for((a.fb[4] + (64 / W) - 1) / (64 / W), 256);
+  const uint64_t fg = grid_for((a.fb[4] + (64 / W) - 1) / (64 / W), 256);
   if (fg > 0) CTC_R_SWITCH(R, hipLaunchKernelGGL((k_sgd_fold<RR>), dim3((unsigned)fg), dim3(256), 0, st, a));
   return hipGetLastError();
 }

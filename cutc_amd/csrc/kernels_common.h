@@ -108,7 +108,7 @@ struct MergeArgs {
 
 struct SettleArgs {
   MergeArgs mg;        // mode 0's long and hot rows
-  uint64_t nb_merge;   // k_sgd_fold's first blocks, which take mg's items
+  uint64_t nb_light;   // k_sgd_settle's blocks of light rows, before those of mg's items
   float *F[4];
   const uint32_t *hot[4];  // hot-row bitmaps
   const float *stage[4];
@@ -123,7 +123,7 @@ struct SettleArgs {
   const uint32_t *light[4];  // the sub-step's rows of at most kSettleLight runs, a walker each
   uint64_t pb[5];          // mode k's heavy pieces: k_sgd_settle's blocks pb[k] .. pb[k + 1]
   uint64_t lb[5];          // mode k's light rows: walkers lb[k] .. lb[k + 1] of the blocks after pb[4]
-  uint64_t fb[5];          // mode k's multi-piece rows: k_sgd_fold's walkers fb[k] .. fb[k + 1] after the merge
+  uint64_t fb[5];          // mode k's multi-piece rows: k_sgd_fold's walkers fb[k] .. fb[k + 1]
 };
 
 __device__ inline int lane_id() { return (int)(threadIdx.x & 63); }

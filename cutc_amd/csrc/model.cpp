@@ -838,12 +838,17 @@ static ctc_status ensure_sync(ctc_model *m, uint32_t span, uint32_t sub) {
     std::vector<uint64_t> &hoff = m->sgd_heavy_off[k], &loff = m->sgd_light_off[k];
     hoff.assign(nsub + 1, 0);
     loff.assign(nsub + 1, 0);
+    // each list by its pieces' runs, most first (the order of equals is kept)
+    std::vector<std::vector<uint32_t>> by_runs(kStagePiece + 1);
     for (uint64_t s2 = 0; s2 < nsub; ++s2) {
       hoff[s2] = heavy.size();
       loff[s2] = light.size();
-      for (uint64_t gp = poff[s2]; gp < poff[s2 + 1]; ++gp) {
-        const bool lt = piece_row[gp] != 0xFFFFFFFFu && piece_start[gp + 1] - piece_start[gp] <= ctc::kSettleLight;
-        (lt ? light : heavy).push_back((uint32_t)gp);
+      for (uint64_t gp = poff[s2]; gp < poff[s2 + 1]; ++gp)
+        by_runs[piece_start[gp + 1] - piece_start[gp]].push_back((uint32_t)gp);
+      for (uint32_t n = kStagePiece + 1; n-- > 0;) {
+        for (const uint32_t gp : by_runs[n])
+          (n <= kSettleLight && piece_row[gp] != 0xFFFFFFFFu ? light : heavy).push_back(gp);
+        by_runs[n].clear();
       }
     }
     hoff[nsub] = heavy.size();
@@ -880,8 +885,8 @@ static ctc_status ensure_sync(ctc_model *m, uint32_t span, uint32_t sub) {
 
 // One epoch of the bulk-synchronous schedule: per sub-step, k_sgd_sync over
 // every walker, then k_sgd_settle over the pieces of the other modes' rows and
-// k_sgd_fold over mode 0's long rows and the other modes' rows of several
-// pieces.
+// mode 0's long rows, and k_sgd_fold over the other modes' rows of several pieces,
+// where there are any.
 // Enqueued only (no synchronisation).
 static ctc_status sgd_epoch_sync(ctc_model *m, const ctc_options *o, double lr) {
   uint32_t span = 0, sub = 0;
