@@ -693,19 +693,21 @@ __device__ inline void store_row(const MixedArgs &a, MixedSmem<R> &sm, uint32_t 
 // cores, K + lambda I eliminated in place (L D L^T, no square roots), two
 // triangular solves, a = H^T z.  All in FP64 (the BF16 path stages the
 // BF16-rounded h), so no refinement step is needed.
-// NT = 16 serves rows of at most 16 nonzeros, NT = 32 the rest; the LDS of a
-// workgroup is sized for its NT, and the BF16 path keeps h as BF16 bits, so
-// the common short rows take ~6 KB of LDS at R = 128 (several waves per SIMD)
-// instead of the 25 KB a 32-row FP32 stage needs.
+// NT = 16 serves rows of at most 16 nonzeros, NT = 32 the rest.
+//
+// The system stays in the matrix cores' accumulator layout (lane (q, c) of a
+// 16 x 16 block holds rows 4v + q of column c; both triangles are kept): at step
+// k a column's entries come by a DPP broadcast within 16 lanes and row k by one
+// shuffle, where a system in LDS cost 50 LDS accesses a step.  Only the row's
+// own nonzeros are staged; what the other rows of H hold reaches entries of K
+// that are padding and replaced.  R = 128, BF16, 393K rows of at most 16
+// nonzeros 709 us (987 us), 19K rows of 17 to 32 186 us (411 us).
 template <int R, int P, int NT>
 struct ThinSmem {
   typedef typename std::conditional<P == kPrecBF16, uint16_t, double>::type HT;
-  static constexpr int HS = R + 1;  // staged h stride (odd: spreads LDS banks)
-  static constexpr int KS = NT + 1;
+  static constexpr int EPL = P == kPrecBF16 || R == 128 ? 2 : 1;  // features per lane and load
+  static constexpr int HS = R + (P == kPrecBF16 ? 2 : 1);         // staged h stride: odd in LDS words (BF16) or doubles
   HT H[NT * HS];
-  double K[NT * KS];
-  double x[NT];
-  int bad;
   __device__ static double hval(HT v) {
     if constexpr (P == kPrecBF16)
       return (double)__uint_as_float((uint32_t)v << 16);
@@ -714,131 +716,197 @@ struct ThinSmem {
   }
 };
 
+// x of lane K of every 16 lanes
+template <int K>
+__device__ inline double row_lane(double x) {
+  const uint64_t u = __builtin_bit_cast(uint64_t, x);
+  const uint32_t lo = (uint32_t)__builtin_amdgcn_mov_dpp((int)(uint32_t)u, 0x150 + K, 0xF, 0xF, true);
+  const uint32_t hi = (uint32_t)__builtin_amdgcn_mov_dpp((int)(uint32_t)(u >> 32), 0x150 + K, 0xF, 0xF, true);
+  return __builtin_bit_cast(double, (uint64_t)hi << 32 | lo);
+}
+
+// x of (uniform) lane p
+__device__ inline double lane_value_d(double x, int p) {
+  const uint64_t u = __builtin_bit_cast(uint64_t, x);
+  const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)u, p);
+  const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(u >> 32), p);
+  return __builtin_bit_cast(double, (uint64_t)hi << 32 | lo);
+}
+
+// One step of L D L^T on the NB x NB blocks A of 16 x 16 (n rows in use), the
+// right-hand side b (lane c: entry 16 j + c, in every q) alongside: after it,
+// column K below the diagonal holds l_iK d_K.
+template <int NB, int K>
+__device__ inline void thin_eliminate(f64x4 (&A)[NB][NB], double (&b)[NB], double (&rd)[NB], int n, bool &ok) {
+  if constexpr (K < 16 * NB) {
+    if (K >= n) return;  // uniform: the padding is the identity, without coupling
+    constexpr int KB = K / 16, KC = K % 16;
+    const int l = threadIdx.x & 63, c = l & 15;
+    double r[NB];  // row K
+#pragma unroll
+    for (int j = KB; j < NB; ++j) r[j] = __shfl(A[KB][j][KC / 4], (KC & 3) * 16 + c, 64);
+    const double d = row_lane<KC>(r[KB]);
+    ok = ok && d > 0.0;
+    const double rk = rcp_f64(d > 0.0 ? d : 1.0);
+    const double bk = row_lane<KC>(b[KB]);
+    if (c == KC) rd[KB] = rk;
+    double lc[NB];  // l_cK of the columns still to eliminate, else 0
+#pragma unroll
+    for (int j = KB; j < NB; ++j) {
+      lc[j] = j > KB || c > KC ? r[j] * rk : 0.0;
+      b[j] = __builtin_fma(-lc[j], bk, b[j]);
+    }
+#pragma unroll
+    for (int i = KB; i < NB; ++i)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        const double aik = row_lane<KC>(A[i][KB][v]);
+#pragma unroll
+        for (int j = KB; j < NB; ++j) A[i][j][v] = __builtin_fma(-aik, lc[j], A[i][j][v]);
+      }
+    thin_eliminate<NB, K + 1>(A, b, rd, n, ok);
+  }
+}
+
+// back solve L^T z = w, z in place of w (lane c: entry 16 j + c)
+template <int NB, int K>
+__device__ inline void thin_back(const f64x4 (&A)[NB][NB], double (&b)[NB], const double (&rd)[NB], int n) {
+  if constexpr (K > 0) {
+    if (K < n) {  // uniform
+      constexpr int KB = K / 16, KC = K % 16;
+      const int l = threadIdx.x & 63, c = l & 15;
+      const double zk = row_lane<KC>(b[KB]);
+#pragma unroll
+      for (int j = 0; j <= KB; ++j) {
+        const double r = __shfl(A[KB][j][KC / 4], (KC & 3) * 16 + c, 64);  // l_Kc d_c where c is before K
+        if (j < KB || c < KC) b[j] = __builtin_fma(-r * rd[j], zk, b[j]);
+      }
+    }
+    thin_back<NB, K - 1>(A, b, rd, n);
+  }
+}
+
 template <int R, int N, int P, int NT>
-__global__ void __launch_bounds__(64) k_rows_thin(MixedArgs a, uint64_t base) {
+__global__ void __launch_bounds__(256) k_rows_thin(MixedArgs a, uint64_t base, uint64_t count) {
   typedef ThinSmem<R, P, NT> TS;
-  __shared__ TS sm;
-  const uint4 it = a.thin[base + blockIdx.x];
-  const int l = threadIdx.x;
+  constexpr int EPL = TS::EPL, LPR = R / EPL, RPS = 64 / LPR, NB = NT / 16, U = 8;
+  __shared__ TS sms[4];
+  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const uint64_t item = (uint64_t)blockIdx.x * 4 + wave;
+  if (item >= count) return;  // no barrier below
+  TS &sm = sms[wave];
+  const uint4 it = a.thin[base + item];
+  const int l = threadIdx.x & 63, c = l & 15;
   const int n = (int)(it.z - it.y);
-  constexpr int nt = NT;  // system size handled (zero-padded)
-  // 1. stage h for the row's nonzeros (rows >= n zero) and x.  Lane p < n
-  // loads nonzero p's ids once; the gathers of all nonzeros are then issued
-  // back to back (independent loads, one memory latency for the row).
-  constexpr int FPL = R / 64 > 0 ? R / 64 : 1;  // features per lane
+  // 1. stage h of the row's nonzeros: lane p < n loads nonzero p's ids once,
+  // the gathers of U groups of nonzeros are then in flight together
   uint32_t myid[N - 1];
 #pragma unroll
   for (int s = 0; s < N - 1; ++s) myid[s] = l < n ? a.oidx[s][it.y + l] : 0u;
-  if (l < NT) sm.x[l] = l < n ? (double)a.vals[it.y + l] : 0.0;
-#pragma unroll 8
-  for (int p = 0; p < nt; ++p) {
-    uint32_t id[N - 1];
+  const float xl = l < n ? a.vals[it.y + l] : 0.f;
+  const int fl = (l % LPR) * EPL;
+  for (int p0 = 0; p0 < n; p0 += U * RPS) {
+    uint32_t ub[U][N - 1];       // BF16 pairs
+    float uf[U][N - 1][EPL];
 #pragma unroll
-    for (int s = 0; s < N - 1; ++s) id[s] = (uint32_t)__shfl((int)myid[s], p, 64);
+    for (int u = 0; u < U; ++u) {
+      const int p = p0 + u * RPS + l / LPR;
 #pragma unroll
-    for (int j = 0; j < FPL; ++j) {
-      const int f = l + 64 * j;
-      if (f >= R) continue;
-      typename TS::HT h = 0;
-      if (p < n) {
+      for (int s = 0; s < N - 1; ++s) {
+        const uint32_t id = (uint32_t)__shfl((int)myid[s], p & 63, 64);
+        if (p >= n) continue;
         if constexpr (P == kPrecBF16) {
-          float hf = 1.f;
-#pragma unroll
-          for (int s = 0; s < N - 1; ++s) hf *= __uint_as_float((uint32_t)a.fb[s][(size_t)id[s] * R + f] << 16);
-          h = f2bf(hf);
+          ub[u][s] = *reinterpret_cast<const uint32_t *>(a.fb[s] + (size_t)id * R + fl);
+        } else if constexpr (EPL == 2) {
+          const float2 t = *reinterpret_cast<const float2 *>(a.fr[s] + (size_t)id * R + fl);
+          uf[u][s][0] = t.x, uf[u][s][1] = t.y;
         } else {
-          double hd = 1.0;
-#pragma unroll
-          for (int s = 0; s < N - 1; ++s) hd *= (double)a.fr[s][(size_t)id[s] * R + f];
-          h = hd;
+          uf[u][s][0] = a.fr[s][(size_t)id * R + fl];
         }
       }
-      sm.H[p * TS::HS + f] = h;
     }
-  }
-  if (l == 0) sm.bad = 0;
-  wave_sync();
-  // 2. K = H H^T (lower 16x16 tiles) on v_mfma_f64_16x16x4f64
-  f64x4 k00 = {0.0, 0.0, 0.0, 0.0}, k10 = k00, k11 = k00;
-  for (int f0 = 0; f0 < R; f0 += 4) {
-    const int f = f0 + (l >> 4);
-    const double h0 = TS::hval(sm.H[(l & 15) * TS::HS + f]);
-    k00 = __builtin_amdgcn_mfma_f64_16x16x4f64(h0, h0, k00, 0, 0, 0);
-    if constexpr (NT == 32) {
-      const double h1 = TS::hval(sm.H[(16 + (l & 15)) * TS::HS + f]);
-      k10 = __builtin_amdgcn_mfma_f64_16x16x4f64(h1, h0, k10, 0, 0, 0);
-      k11 = __builtin_amdgcn_mfma_f64_16x16x4f64(h1, h1, k11, 0, 0, 0);
-    }
-  }
-  const double lam = a.lam;
 #pragma unroll
-  for (int v = 0; v < 4; ++v) {
-    const int r = row16(v, l), c = l & 15;
-    // padded rows/columns (>= n) become the identity
-    auto put = [&](int rr, int cc, double val) {
-      const bool pad = rr >= n || cc >= n;
-      sm.K[rr * TS::KS + cc] = pad ? (rr == cc ? 1.0 : 0.0) : val + (rr == cc ? lam : 0.0);
-    };
-    put(r, c, k00[v]);
-    if constexpr (NT == 32) {
-      put(16 + r, c, k10[v]);
-      put(16 + r, 16 + c, k11[v]);
-    }
-  }
-  wave_sync();
-  // 3. K = L D L^T in place: after step k, K[i][j] (i > j) = l_ij d_j and
-  // K[j][j] = d_j.  Lane l updates column c = l % 32 for rows of its half.
-  // The padding (rows and columns >= n) is the identity with no coupling, so
-  // steps k >= n - 1 change nothing: the elimination and both solves stop at
-  // the row's own size.
-  {
-    const int c = l & 31, half = l >> 5;
-    bool ok = true;
-    for (int k = 0; k < n - 1; ++k) {
-      const double dk = sm.K[k * TS::KS + k];
-      ok = ok && dk > 0.0;
-      const double lck = (c < NT ? sm.K[c * TS::KS + k] : 0.0) * rcp_f64(dk > 0.0 ? dk : 1.0);
-      double aik[16];
+    for (int u = 0; u < U; ++u) {
+      const int p = p0 + u * RPS + l / LPR;
+      if (p >= n) continue;
+      typename TS::HT *dst = sm.H + p * TS::HS + fl;
+      if constexpr (P == kPrecBF16) {
+        float h0 = bf_lo(ub[u][0]), h1 = bf_hi(ub[u][0]);
 #pragma unroll
-      for (int e = 0; e < 16; ++e) aik[e] = (16 * half + e < NT) ? sm.K[(16 * half + e) * TS::KS + k] : 0.0;
-      wave_sync();
-      if (c > k && c < nt) {
+        for (int s = 1; s < N - 1; ++s) h0 *= bf_lo(ub[u][s]), h1 *= bf_hi(ub[u][s]);
+        *reinterpret_cast<uint32_t *>(dst) = (uint32_t)f2bf(h0) | (uint32_t)f2bf(h1) << 16;
+      } else {
 #pragma unroll
-        for (int e = 0; e < 16; ++e) {
-          const int i = 16 * half + e;
-          if (i >= c && i < nt) sm.K[i * TS::KS + c] = __builtin_fma(-aik[e], lck, sm.K[i * TS::KS + c]);
+        for (int e = 0; e < EPL; ++e) {
+          double h = (double)uf[u][0][e];
+#pragma unroll
+          for (int s = 1; s < N - 1; ++s) h *= (double)uf[u][s][e];
+          dst[e] = h;
         }
       }
-      wave_sync();
     }
-    ok = ok && sm.K[(n - 1) * TS::KS + n - 1] > 0.0;
-    if (!ok && l == 0) sm.bad = 1;
   }
   wave_sync();
-  // 4. z = (L D L^T)^-1 x: lane i < nt holds x_i
-  double xi = l < nt ? sm.x[l] : 0.0;
-  const double di = l < nt ? sm.K[l * TS::KS + l] : 1.0;
-  const double rdi = rcp_f64(di > 0.0 ? di : 1.0);
-  for (int j = 0; j < n - 1; ++j) {  // forward, unit lower L: l_ij = K[i][j] / d_j
-    const double yj = __shfl(xi * rdi, j, 64);  // y_j / d_j
-    if (l > j && l < nt) xi = __builtin_fma(-sm.K[l * TS::KS + j], yj, xi);
+  // 2. K = H H^T on v_mfma_f64_16x16x4f64; one block alone would be one
+  // dependent chain, so it is summed in two
+  constexpr int NC = NB == 1 ? 2 : 1;
+  f64x4 A[NB][NB], A2 = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+  for (int i = 0; i < NB; ++i)
+#pragma unroll
+    for (int j = 0; j < NB; ++j) A[i][j] = f64x4{0.0, 0.0, 0.0, 0.0};
+#pragma unroll 2
+  for (int f0 = 0; f0 < R; f0 += 4 * NC) {
+    double h[NC][NB];
+#pragma unroll
+    for (int e = 0; e < NC; ++e)
+#pragma unroll
+      for (int i = 0; i < NB; ++i) h[e][i] = TS::hval(sm.H[(16 * i + c) * TS::HS + f0 + 4 * e + (l >> 4)]);
+#pragma unroll
+    for (int i = 0; i < NB; ++i)
+#pragma unroll
+      for (int j = 0; j < NB; ++j)
+        A[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(h[0][i], h[0][j], A[i][j], 0, 0, 0);
+    if constexpr (NC == 2) A2 = __builtin_amdgcn_mfma_f64_16x16x4f64(h[1][0], h[1][0], A2, 0, 0, 0);
   }
-  xi *= rdi;
-  for (int j = n - 1; j > 0; --j) {  // backward, L^T: l_ji = K[j][i] / d_i
-    const double zj = __shfl(xi, j, 64);
-    if (l < j) xi = __builtin_fma(-sm.K[j * TS::KS + l] * rdi, zj, xi);
+  if constexpr (NC == 2) A[0][0] += A2;
+  double b[NB], rd[NB];
+#pragma unroll
+  for (int i = 0; i < NB; ++i) {
+#pragma unroll
+    for (int j = 0; j < NB; ++j)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {  // padded rows and columns (>= n) become the identity
+        const int rr = 16 * i + row16(v, l), cc = 16 * j + c;
+        const double k = A[i][j][v] + (rr == cc ? a.lam : 0.0);
+        A[i][j][v] = rr >= n || cc >= n ? (rr == cc ? 1.0 : 0.0) : k;
+      }
+    b[i] = (double)__shfl(xl, 16 * i + c, 64);
+    rd[i] = 1.0;
   }
-  wave_sync();
-  if (l < NT) sm.x[l] = xi;
-  wave_sync();
+  // 3., 4. K = L D L^T, z = K^-1 x
+  bool ok = true;
+  thin_eliminate<NB, 0>(A, b, rd, n, ok);
+#pragma unroll
+  for (int i = 0; i < NB; ++i) b[i] *= rd[i];
+  thin_back<NB, NT - 1>(A, b, rd, n);
   // 5. a = H^T z
   float *dst = a.out + (size_t)a.directory[it.x] * R;
-  const bool ok = sm.bad == 0;
-  for (int f = l; f < R; f += 64) {
-    double acc = 0.0;
-    for (int p = 0; p < n; ++p) acc = __builtin_fma(TS::hval(sm.H[p * TS::HS + f]), sm.x[p], acc);
-    dst[f] = ok ? (float)acc : 0.f;
+  constexpr int FPL = (R + 63) / 64;
+  double acc[FPL];
+#pragma unroll
+  for (int j = 0; j < FPL; ++j) acc[j] = 0.0;
+  const int lf = R < 64 ? l % R : l;
+  for (int p = 0; p < n; ++p) {
+    double z = lane_value_d(b[0], p & 15);
+    if constexpr (NB > 1)
+      if (p >= 16) z = lane_value_d(b[NB - 1], p & 15);
+#pragma unroll
+    for (int j = 0; j < FPL; ++j) acc[j] = __builtin_fma(TS::hval(sm.H[p * TS::HS + lf + 64 * j]), z, acc[j]);
   }
+#pragma unroll
+  for (int j = 0; j < FPL; ++j)
+    if (l < R) dst[l + 64 * j] = ok ? (float)acc[j] : 0.f;
   if (!ok && l == 0) atomicOr(a.flag, 1u);
 }
 
@@ -1220,11 +1288,11 @@ hipError_t launch_mixed_heavy(hipStream_t st, const MixedArgs &a, int nmodes, in
   do {                                                                                                            \
     const uint64_t n16 = a.nthin16, n32 = a.nthin - a.nthin16;                                                    \
     if (a.prec == kPrecBF16) {                                                                                    \
-      if (n16) hipLaunchKernelGGL((k_rows_thin<RR, NN, kPrecBF16, 16>), dim3((unsigned)n16), dim3(64), 0, st, a, 0ull); \
-      if (n32) hipLaunchKernelGGL((k_rows_thin<RR, NN, kPrecBF16, 32>), dim3((unsigned)n32), dim3(64), 0, st, a, n16);  \
+      if (n16) hipLaunchKernelGGL((k_rows_thin<RR, NN, kPrecBF16, 16>), dim3((unsigned)((n16 + 3) / 4)), dim3(256), 0, st, a, 0ull, n16); \
+      if (n32) hipLaunchKernelGGL((k_rows_thin<RR, NN, kPrecBF16, 32>), dim3((unsigned)((n32 + 3) / 4)), dim3(256), 0, st, a, n16, n32);  \
     } else {                                                                                                      \
-      if (n16) hipLaunchKernelGGL((k_rows_thin<RR, NN, kPrecF64, 16>), dim3((unsigned)n16), dim3(64), 0, st, a, 0ull);  \
-      if (n32) hipLaunchKernelGGL((k_rows_thin<RR, NN, kPrecF64, 32>), dim3((unsigned)n32), dim3(64), 0, st, a, n16);   \
+      if (n16) hipLaunchKernelGGL((k_rows_thin<RR, NN, kPrecF64, 16>), dim3((unsigned)((n16 + 3) / 4)), dim3(256), 0, st, a, 0ull, n16);  \
+      if (n32) hipLaunchKernelGGL((k_rows_thin<RR, NN, kPrecF64, 32>), dim3((unsigned)((n32 + 3) / 4)), dim3(256), 0, st, a, n16, n32);   \
     }                                                                                                             \
   } while (0)
 

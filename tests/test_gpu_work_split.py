@@ -168,3 +168,37 @@ def test_sgd_walk_rounds(ctx, dims, nnz, span, sub, R, mixed):
                            sgd_hot_rows=400, precision=ct.PREC_MIXED if mixed else ct.PREC_FP32), lr=1e-3)
     for k, f in enumerate(F64):
         assert np.linalg.norm(m.factor(k) - f) < (2e-4 if mixed else 1e-5) * np.linalg.norm(f), k
+
+
+@pytest.mark.parametrize("R", [32, 64, 128])
+@pytest.mark.parametrize("mixed", [False, True], ids=["fp32", "mixed"])
+@pytest.mark.parametrize("rest", [(47, 39), (23, 19, 17)], ids=["3way", "4way"])
+def test_als_row_lengths(ctx, rest, mixed, R):
+    """The row-fused ALS update of rows of 1 to 67 nonzeros, one of each length and
+    one of several Gram steps, and rows without nonzeros, each row against the
+    ridge solution in 64 bits (mixed: the oracle's BF16-operand update) at the
+    parity tests' bars, row by row (1e-5, 1e-4)."""
+    import oracle as O
+    say(f"[als row lengths] rest={rest} R={R} mixed={mixed}")
+    rng = np.random.default_rng(31)
+    lens = [*range(1, 68), 0, 301, 0]
+    rng.shuffle(lens)
+    rows = np.repeat(np.arange(len(lens)), lens)
+    flat = np.concatenate([rng.choice(int(np.prod(rest)), size=n, replace=False) for n in lens])
+    ind = [rows.astype(np.uint32), *(a.astype(np.uint32) for a in np.unravel_index(flat, rest))]
+    vals = rng.uniform(1.0, 5.0, len(rows))
+    dims = (len(lens), *rest)
+    F = [rng.uniform(-1, 1, (d, R)).astype(np.float32) for d in dims]
+    m = ct.Model(ctx, ct.Coo.from_arrays(ind, vals, dims), None, None, rank=R)
+    m.set_factors(F)
+    m.als_mode_update(0, ct.Options(algorithm=ct.ALS, rank=R, lambda_=0.5, als_kernel=ct.ALS_ROWS,
+                                    precision=ct.PREC_MIXED if mixed else ct.PREC_FP32))
+    if mixed:
+        want = [f.copy() for f in F]
+        assert O.als_mode_bf16(O.Coo(ind, vals, dims), 0, want, 0.5) == 0
+        want = want[0].astype(np.float64)
+    else:
+        want = ridge(ind, vals, F, 0, 0.5)
+    got = m.factor(0).astype(np.float64)
+    for r, n in enumerate(lens):
+        assert np.linalg.norm(got[r] - want[r]) <= (1e-4 if mixed else 1e-5) * np.linalg.norm(want[r]), (r, n)
