@@ -49,7 +49,7 @@ template <int R>
 struct MixedSmem {
   static constexpr int NW = R / 32, RT = R / 16, NTILE = RT * (RT + 1) / 2;
   static constexpr int TPW = (NTILE + NW - 1) / NW;  // FP64 path: lower tiles per wave
-  static constexpr int HS = R + 2;                   // FP64 path: staged row stride (doubles)
+  static constexpr int HS = R + 16;                  // FP64 path: staged row stride (doubles)
   static constexpr int NT64 = NTILE * 256 > 32 * HS ? NTILE * 256 : 32 * HS;
   double tiles[NT64];  // FP64 lower tiles; the Gram phase stages h here
   double vm[R], vx[R], vy[R];
@@ -164,22 +164,53 @@ __device__ inline void gram_chunk(const MixedArgs &a, uint32_t p0, uint32_t p1, 
 // FP64 variant: h = product of the FP32 rows formed in FP64, staged in LDS
 // as FP64 (32 nonzeros x R), and every lower 16x16 tile of G accumulated on
 // v_mfma_f64_16x16x4f64, tiles dealt round-robin to the waves (wave w owns
-// tiles w, w + NW, ...); m accumulated in FP64.
+// tiles w, w + NW, ...); m accumulated in FP64.  LDS bandwidth bounds the
+// Gram, so a wave reads each 16-column operand once per step for all its tiles
+// (the tile list is fixed at compile time per wave), and the layout keeps the
+// banks busy: rows are 16 doubles more than a multiple of the banks apart, so
+// two rows of an operand fill them, and a thread stages the pairs of features
+// 2 fg + R / 4 i of nonzeros qp and qp + 16.
+// Batch class of rank 64 (19K rows of 0.3M-nonzero problems): 605 us per mode
+// update, 1010 us with both operands read per tile, 8 consecutive features per
+// thread and two waves per SIMD in k_mixed_items (its bounds hold it to three;
+// the batch pass 41.3 ms, 43.4 ms with two).
+template <int R, int W, int NW>
+__device__ inline void gram_tiles(const double *hs, f64x4 *acc) {
+  constexpr int HS = MixedSmem<R>::HS, RT = R / 16;
+  const int l = threadIdx.x & 63;
+#pragma unroll 2
+  for (int s = 0; s < 8; ++s) {
+    const double *hq = hs + (4 * s + (l >> 4)) * HS + (l & 15);
+    double h[RT];
+#pragma unroll
+    for (int i = 0; i < RT; ++i) h[i] = hq[16 * i];
+    int j = 0;
+#pragma unroll
+    for (int I = 0; I < RT; ++I)
+#pragma unroll
+      for (int J = 0; J <= I; ++J)
+        if (tileno(I, J) % NW == W) {
+          acc[j] = __builtin_amdgcn_mfma_f64_16x16x4f64(h[I], h[J], acc[j], 0, 0, 0);
+          ++j;
+        }
+  }
+}
+
 template <int R, int N>
 __device__ inline void gram_f64(const MixedArgs &a, uint32_t p0, uint32_t p1, f64x4 *acc, double *mp,
                                 double *hs) {
   constexpr int NW = R / 32, FG8 = R / 8, HS = MixedSmem<R>::HS;
-  constexpr int NTILE = MixedSmem<R>::NTILE, TPW = MixedSmem<R>::TPW;
-  const int tid = threadIdx.x, w = tid >> 6, l = tid & 63;
+  const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int fg = tid % FG8, qp = tid / FG8;
-  // software pipeline as in gram_chunk: ids two steps ahead, rows one ahead
+  // software pipeline: ids two steps ahead; the next step's rows are requested
+  // once this step's are staged and arrive under its matrix products
   uint32_t id_n[2][N - 1];
   float x_n[2], x_r[2];
-  float4 u_n[2][N - 1][2], u_c[2][N - 1][2];
+  float2 u_n[2][N - 1][4];
   auto load_ids = [&](uint32_t base) {
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
-      const uint32_t p = base + 2 * qp + h;
+      const uint32_t p = base + qp + 16 * h;
       const bool ok = p < p1;
 #pragma unroll
       for (int s = 0; s < N - 1; ++s) id_n[h][s] = ok ? a.oidx[s][p] : 0u;
@@ -191,9 +222,9 @@ __device__ inline void gram_f64(const MixedArgs &a, uint32_t p0, uint32_t p1, f6
     for (int h = 0; h < 2; ++h)
 #pragma unroll
       for (int s = 0; s < N - 1; ++s) {
-        const float *row = a.fr[s] + (size_t)id_n[h][s] * R + 8 * fg;
-        u_n[h][s][0] = *(const float4 *)row;
-        u_n[h][s][1] = *(const float4 *)(row + 4);
+        const float *row = a.fr[s] + (size_t)id_n[h][s] * R + 2 * fg;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) u_n[h][s][i] = *(const float2 *)(row + 2 * FG8 * i);
       }
   };
   load_ids(p0);
@@ -202,62 +233,49 @@ __device__ inline void gram_f64(const MixedArgs &a, uint32_t p0, uint32_t p1, f6
   x_r[1] = x_n[1];
   load_ids(p0 + 32);
   for (uint32_t base = p0; base < p1; base += 32) {
-    float x_c[2];
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
-      x_c[h] = x_r[h];
-      x_r[h] = x_n[h];
+      const bool ok = base + qp + 16 * h < p1;
+      double *dst = hs + (qp + 16 * h) * HS + 2 * fg;
 #pragma unroll
-      for (int s = 0; s < N - 1; ++s) u_c[h][s][0] = u_n[h][s][0], u_c[h][s][1] = u_n[h][s][1];
+      for (int i = 0; i < 4; ++i) {
+        double h0 = (double)u_n[h][0][i].x, h1 = (double)u_n[h][0][i].y;
+#pragma unroll
+        for (int s = 1; s < N - 1; ++s) h0 *= (double)u_n[h][s][i].x, h1 *= (double)u_n[h][s][i].y;
+        h0 = ok ? h0 : 0.0, h1 = ok ? h1 : 0.0;  // past the row's end: other rows' entries were read
+        mp[2 * i] += (double)x_r[h] * h0;
+        mp[2 * i + 1] += (double)x_r[h] * h1;
+        *(double2 *)(dst + 2 * FG8 * i) = make_double2(h0, h1);
+      }
+      x_r[h] = x_n[h];
     }
     load_rows();           // rows of step base + 32
     load_ids(base + 64);   // ids of step base + 64
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      const uint32_t p = base + 2 * qp + h;
-      double hd[8];
-      if (p < p1) {
-#pragma unroll
-        for (int f = 0; f < 8; ++f) hd[f] = 1.0;
-#pragma unroll
-        for (int s = 0; s < N - 1; ++s) {
-          const float4 u0 = u_c[h][s][0], u1 = u_c[h][s][1];
-          hd[0] *= u0.x;
-          hd[1] *= u0.y;
-          hd[2] *= u0.z;
-          hd[3] *= u0.w;
-          hd[4] *= u1.x;
-          hd[5] *= u1.y;
-          hd[6] *= u1.z;
-          hd[7] *= u1.w;
-        }
-        const double x = x_c[h];
-#pragma unroll
-        for (int f = 0; f < 8; ++f) mp[f] += x * hd[f];
-      } else {
-#pragma unroll
-        for (int f = 0; f < 8; ++f) hd[f] = 0.0;
-      }
-      double *dst = hs + (2 * qp + h) * HS + 8 * fg;
-#pragma unroll
-      for (int f = 0; f < 8; f += 2) *(double2 *)(dst + f) = make_double2(hd[f], hd[f + 1]);
-    }
     __syncthreads();
-#pragma unroll
-    for (int s = 0; s < 8; ++s) {
-      const double *hq = hs + (4 * s + (l >> 4)) * HS + (l & 15);
-#pragma unroll
-      for (int j = 0; j < TPW; ++j) {
-        const int u = w + NW * j;
-        if (u >= NTILE) continue;  // wave-uniform
-        int I, J;
-        tile_ij(u, I, J);
-        acc[j] = __builtin_amdgcn_mfma_f64_16x16x4f64(hq[16 * I], hq[16 * J], acc[j], 0, 0, 0);
+    if constexpr (NW == 1) {
+      gram_tiles<R, 0, 1>(hs, acc);
+    } else if constexpr (NW == 2) {
+      if (w == 0)
+        gram_tiles<R, 0, 2>(hs, acc);
+      else
+        gram_tiles<R, 1, 2>(hs, acc);
+    } else {
+      switch (w) {
+        case 0: gram_tiles<R, 0, 4>(hs, acc); break;
+        case 1: gram_tiles<R, 1, 4>(hs, acc); break;
+        case 2: gram_tiles<R, 2, 4>(hs, acc); break;
+        default: gram_tiles<R, 3, 4>(hs, acc); break;
       }
     }
     __syncthreads();
   }
 }
+
+// feature of a thread's f-th partial of m (the staging's share of a thread)
+template <int R>
+__device__ inline int m_feature(int fg, int f, float) { return 8 * fg + f; }
+template <int R>
+__device__ inline int m_feature(int fg, int f, double) { return R / 4 * (f >> 1) + 2 * fg + (f & 1); }
 
 // sums the per-thread m partials of the workgroup into sm.vm (FP64); ends
 // with a barrier
@@ -271,7 +289,7 @@ __device__ inline void reduce_m(T *mp, SM &sm) {
     for (int f = 0; f < 8; ++f) mp[f] += __shfl_xor(mp[f], o, 64);
   if (l < FG8)
 #pragma unroll
-    for (int f = 0; f < 8; ++f) sm.contrib[w][8 * fg + f] = (double)mp[f];
+    for (int f = 0; f < 8; ++f) sm.contrib[w][m_feature<R>(fg, f, T())] = (double)mp[f];
   __syncthreads();
   if (tid < R) {
     double s = 0.0;
@@ -1110,7 +1128,7 @@ struct AccShape<R, kPrecF64> {  // round-robin 16x16 tiles, 4 doubles per lane e
 };
 
 template <int R, int N, int P>
-__global__ void __launch_bounds__(2 * R, 2) k_mixed_items(MixedArgs a) {
+__global__ void __launch_bounds__(2 * R, P == kPrecF64 && R <= 64 ? 3 : 2) k_mixed_items(MixedArgs a) {
   typedef AccShape<R, P> S;
   __shared__ MixedSmem<R> sm;
   const uint4 it = a.items[blockIdx.x];
