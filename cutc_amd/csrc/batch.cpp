@@ -269,6 +269,7 @@ static ctc_status prepare_class(RankClass &c, const ctc_options *t) {
   for (uint32_t md = 0; md < m->nmodes; ++md) {
     CTC_TRY(ensure_ciss(m, md));
     CTC_TRY(ensure_pieces(m, md, als_span_tiles(t, m->ciss[md].nnz)));
+    if (als_uses_thin(t, c.rank)) CTC_TRY(ensure_thin(m, md));
     const DevCiss &d = m->ciss[md];
     need = std::max(need, (size_t)(d.npieces + d.ngroups) * ((size_t)c.rank * c.rank + c.rank) * sizeof(double));
   }
@@ -335,6 +336,7 @@ static std::vector<uintptr_t> graph_key_of(ctc_batch *b, const ctc_options *o, u
       k.push_back((uintptr_t)d.slot_pb);
       k.push_back((uintptr_t)d.span_off);
       k.push_back((uintptr_t)d.slot_gb);
+      k.push_back((uintptr_t)(als_uses_thin(&t, c.rank) ? d.thin_items : nullptr));
       k.push_back((uintptr_t)d.mix_items);
       k.push_back((uintptr_t)d.mix_chunk);
       k.push_back((uintptr_t)c.model->F[md]);

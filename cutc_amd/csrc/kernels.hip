@@ -1006,9 +1006,13 @@ __global__ void __launch_bounds__(256) k_mttkrp(CissArgs c, FactorArgs fa, uint3
 // ==========================================================================
 typedef double doublex4 __attribute__((ext_vector_type(4)));
 
+//
+// tile_thin (null: none) marks the nonzeros of rows that are solved in their
+// dual form: the walk passes over them and writes no piece for their rows.
 template <int R, int N>
 __device__ __forceinline__ void als_gram_walk(const CissArgs &c, const FactorArgs &fa, uint32_t span_tiles,
-                                              uint64_t nspans, const uint32_t *span_off, double *pieces) {
+                                              uint64_t nspans, const uint32_t *span_off, const uint64_t *tile_thin,
+                                              double *pieces) {
   constexpr int CG = (R + 15) / 16;      // 16-column groups
   constexpr int NB = CG * (CG + 1) / 2;  // lower-triangle 16x16 blocks
   constexpr int NPS = 4;                 // nonzeros per MFMA step
@@ -1020,6 +1024,7 @@ __device__ __forceinline__ void als_gram_walk(const CissArgs &c, const FactorArg
   const uint64_t t1 = t0 + span_tiles < c.ntiles ? t0 + span_tiles : c.ntiles;
   const uint32_t poff = span_off[w];
   uint32_t slot = c.tile_slot[t0];
+  bool skip = false;  // the open row is marked in tile_thin
   const int col = lane & 15;
   const int nsub = lane >> 4;
 
@@ -1069,13 +1074,24 @@ __device__ __forceinline__ void als_gram_walk(const CissArgs &c, const FactorArg
     }
     uint64_t mask = c.tile_mask[t];
     if (cnt < 64) mask &= (1ull << cnt) - 1ull;
+    const uint64_t thin = tile_thin ? tile_thin[t] : 0ull;
     uint32_t pos = 0;
     while (pos < cnt) {
       if ((mask >> pos) & 1ull) {
         if (!(t == t0 && pos == 0)) {
-          flush(slot + poff);
+          if (!skip) flush(slot + poff);
           ++slot;
         }
+      }
+      skip = (thin >> pos) & 1ull;
+      if (skip) {  // on to the next nonzero that is not marked, past the rows that start on the way
+        const uint64_t stop = ~thin >> pos;
+        uint32_t to = stop ? pos + (uint32_t)__ffsll((unsigned long long)stop) - 1u : cnt;
+        if (to > cnt) to = cnt;
+        const uint64_t upto = to >= 64 ? ~0ull : (1ull << to) - 1ull;
+        slot += (uint32_t)__popcll(mask & upto & ~((2ull << pos) - 1ull));
+        pos = to;
+        continue;
       }
       const uint64_t rest = (pos >= 63) ? 0ull : ((mask >> (pos + 1)) << (pos + 1));
       uint32_t nxt = rest ? (uint32_t)__ffsll((unsigned long long)rest) - 1u : cnt;
@@ -1132,7 +1148,7 @@ __device__ __forceinline__ void als_gram_walk(const CissArgs &c, const FactorArg
       pos = nxt;
     }
   }
-  flush(slot + poff);
+  if (!skip) flush(slot + poff);
 }
 
 // Occupancy: at R <= 32 the walk (with its one-step gather lookahead) is held
@@ -1142,13 +1158,15 @@ __device__ __forceinline__ void als_gram_walk(const CissArgs &c, const FactorArg
 // waves, 4.00 ms with lookahead at 6.
 template <int R, int N>
 __global__ void __launch_bounds__(256, 6) k_als_gram(CissArgs c, FactorArgs fa, uint32_t span_tiles,
-                                                     uint64_t nspans, const uint32_t *span_off, double *pieces) {
-  als_gram_walk<R, N>(c, fa, span_tiles, nspans, span_off, pieces);
+                                                     uint64_t nspans, const uint32_t *span_off,
+                                                     const uint64_t *tile_thin, double *pieces) {
+  als_gram_walk<R, N>(c, fa, span_tiles, nspans, span_off, tile_thin, pieces);
 }
 template <int R, int N>
 __global__ void __launch_bounds__(256) k_als_gram_wide(CissArgs c, FactorArgs fa, uint32_t span_tiles,
-                                                       uint64_t nspans, const uint32_t *span_off, double *pieces) {
-  als_gram_walk<R, N>(c, fa, span_tiles, nspans, span_off, pieces);
+                                                       uint64_t nspans, const uint32_t *span_off,
+                                                     const uint64_t *tile_thin, double *pieces) {
+  als_gram_walk<R, N>(c, fa, span_tiles, nspans, span_off, tile_thin, pieces);
 }
 
 // ==========================================================================
@@ -1322,8 +1340,8 @@ __global__ void __launch_bounds__(64) k_als_solve(const double *pieces, const ui
 template <int R>
 __global__ void __launch_bounds__(256) k_als_solve_h(const double *pieces, const uint32_t *slot_pb,
                                                      const double *gsum, const uint32_t *slot_gb,
-                                                     const uint32_t *directory, uint64_t dlength, double lam,
-                                                     float *A, uint32_t *flag) {
+                                                     const uint32_t *directory, const uint32_t *list, uint64_t count,
+                                                     double lam, float *A, uint32_t *flag) {
   static_assert(R <= 32, "one half-wave per slot");
   constexpr size_t PSZ = (size_t)R * R + R;
   constexpr int CB = R + 2;  // column k, then z_k / x_k; even, so every half's buffer is 16-byte aligned
@@ -1332,8 +1350,9 @@ __global__ void __launch_bounds__(256) k_als_solve_h(const double *pieces, const
   const int c = lane & 31;
   const int cc = c < R ? c : R - 1;  // clamped column for lanes past the rank
   const int hw = (int)(threadIdx.x >> 5);
-  const uint64_t s = (uint64_t)blockIdx.x * 8 + (uint64_t)hw;
-  const bool live = s < dlength;
+  const uint64_t i0 = (uint64_t)blockIdx.x * 8 + (uint64_t)hw;
+  const bool live = i0 < count;
+  const uint64_t s = live && list ? list[i0] : i0;
   double *buf = cbuf[hw];
 
   double g[R];
@@ -1752,7 +1771,7 @@ uint64_t mttkrp_grid(uint64_t nnz, int R, uint32_t span, unsigned block) {
 }
 
 hipError_t launch_als_gram(hipStream_t st, const CissArgs &c, const FactorArgs &f, int nmodes, int R,
-                           uint32_t span_tiles, uint64_t nspans, const uint32_t *span_off,
+                           uint32_t span_tiles, uint64_t nspans, const uint32_t *span_off, const uint64_t *tile_thin,
                            double *pieces, unsigned block) {
   if (c.nnz == 0) return hipSuccess;
   const unsigned grid = grid_for(nspans, block);
@@ -1760,10 +1779,10 @@ hipError_t launch_als_gram(hipStream_t st, const CissArgs &c, const FactorArgs &
   do {                                                                                                    \
     if (nmodes == 3)                                                                                      \
       hipLaunchKernelGGL((k_als_gram<RR, 3>), dim3(grid), dim3(block), 0, st, c, f, span_tiles, nspans, \
-                         span_off, pieces);                                                               \
+                         span_off, tile_thin, pieces);                                                               \
     else                                                                                                  \
       hipLaunchKernelGGL((k_als_gram<RR, 4>), dim3(grid), dim3(block), 0, st, c, f, span_tiles, nspans, \
-                         span_off, pieces);                                                               \
+                         span_off, tile_thin, pieces);                                                               \
   } while (0)
   switch (R) {
     case 8: CTC_GRAM(8); break;
@@ -1773,15 +1792,15 @@ hipError_t launch_als_gram(hipStream_t st, const CissArgs &c, const FactorArgs &
         CTC_GRAM(32);
       else  // four modes need more than the 80 registers of 6 waves per SIMD (it would spill)
         hipLaunchKernelGGL((k_als_gram_wide<32, 4>), dim3(grid), dim3(block), 0, st, c, f, span_tiles, nspans,
-                           span_off, pieces);
+                           span_off, tile_thin, pieces);
       break;
     case 64:
       if (nmodes == 3)
         hipLaunchKernelGGL((k_als_gram_wide<64, 3>), dim3(grid), dim3(block), 0, st, c, f, span_tiles, nspans,
-                           span_off, pieces);
+                           span_off, tile_thin, pieces);
       else
         hipLaunchKernelGGL((k_als_gram_wide<64, 4>), dim3(grid), dim3(block), 0, st, c, f, span_tiles, nspans,
-                           span_off, pieces);
+                           span_off, tile_thin, pieces);
       break;
     default: return hipErrorInvalidValue;
   }
@@ -1809,16 +1828,18 @@ hipError_t launch_piece_reduce(hipStream_t st, const double *pieces, const uint3
 }
 
 hipError_t launch_als_solve(hipStream_t st, const double *pieces, const uint32_t *slot_pb, const double *gsum,
-                            const uint32_t *slot_gb, const uint32_t *directory, uint64_t dlength, int R,
-                            double lam, bool refine, float *A, uint32_t *flag) {
-  if (dlength == 0) return hipSuccess;
+                            const uint32_t *slot_gb, const uint32_t *directory, const uint32_t *list, uint64_t count,
+                            int R, double lam, bool refine, float *A, uint32_t *flag) {
+  if (count == 0) return hipSuccess;
+  if (list && (refine || R > 32)) return hipErrorInvalidValue;
+  const uint64_t dlength = count;
   const unsigned grid = (unsigned)dlength;
   if (!refine && R <= 32) {
     const unsigned g8 = (unsigned)((dlength + 7) / 8);
     switch (R) {
-      case 8: hipLaunchKernelGGL((k_als_solve_h<8>), dim3(g8), dim3(256), 0, st, pieces, slot_pb, gsum, slot_gb, directory, dlength, lam, A, flag); break;
-      case 16: hipLaunchKernelGGL((k_als_solve_h<16>), dim3(g8), dim3(256), 0, st, pieces, slot_pb, gsum, slot_gb, directory, dlength, lam, A, flag); break;
-      case 32: hipLaunchKernelGGL((k_als_solve_h<32>), dim3(g8), dim3(256), 0, st, pieces, slot_pb, gsum, slot_gb, directory, dlength, lam, A, flag); break;
+      case 8: hipLaunchKernelGGL((k_als_solve_h<8>), dim3(g8), dim3(256), 0, st, pieces, slot_pb, gsum, slot_gb, directory, list, count, lam, A, flag); break;
+      case 16: hipLaunchKernelGGL((k_als_solve_h<16>), dim3(g8), dim3(256), 0, st, pieces, slot_pb, gsum, slot_gb, directory, list, count, lam, A, flag); break;
+      case 32: hipLaunchKernelGGL((k_als_solve_h<32>), dim3(g8), dim3(256), 0, st, pieces, slot_pb, gsum, slot_gb, directory, list, count, lam, A, flag); break;
       default: return hipErrorInvalidValue;
     }
     return hipGetLastError();

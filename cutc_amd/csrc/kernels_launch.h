@@ -37,14 +37,16 @@ uint64_t mttkrp_walkers_per_block(int R, unsigned block);
 // of the factors as they are; num / den are zeroed dims x R arrays
 hipError_t launch_ccd_jacobi(hipStream_t st, const CissArgs &c, const FactorArgs &f, int nmodes, int R,
                              uint32_t span, float *num, float *den, unsigned block);
+// tile_thin (or null): the nonzeros whose rows are left to launch_rows_thin
 hipError_t launch_als_gram(hipStream_t st, const CissArgs &c, const FactorArgs &f, int nmodes, int R,
-                           uint32_t span_tiles, uint64_t nspans, const uint32_t *span_off,
+                           uint32_t span_tiles, uint64_t nspans, const uint32_t *span_off, const uint64_t *tile_thin,
                            double *pieces, unsigned block);
 hipError_t launch_piece_reduce(hipStream_t st, const double *pieces, const uint32_t *grp_piece,
                                const uint32_t *grp_n, uint64_t ngroups, int R, double *gsum);
+// slots list[0 .. count), or 0 .. count where list is null (with refine or R = 64 it is)
 hipError_t launch_als_solve(hipStream_t st, const double *pieces, const uint32_t *slot_pb, const double *gsum,
-                            const uint32_t *slot_gb, const uint32_t *directory, uint64_t dlength, int R,
-                            double lam, bool refine, float *A, uint32_t *flag);
+                            const uint32_t *slot_gb, const uint32_t *directory, const uint32_t *list, uint64_t count,
+                            int R, double lam, bool refine, float *A, uint32_t *flag);
 hipError_t launch_eval_coo(hipStream_t st, const CooArgs &c, const FactorArgs &f, int nmodes, int R,
                            unsigned nblocks, double *part);
 // per-segment squared error: exactly one of c (mode-0 CISS order) / co (COO) is

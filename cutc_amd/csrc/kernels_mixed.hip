@@ -807,7 +807,7 @@ __device__ inline void thin_back(const f64x4 (&A)[NB][NB], double (&b)[NB], cons
 template <int R, int N, int P, int NT>
 __global__ void __launch_bounds__(256) k_rows_thin(MixedArgs a, uint64_t base, uint64_t count) {
   typedef ThinSmem<R, P, NT> TS;
-  constexpr int EPL = TS::EPL, LPR = R / EPL, RPS = 64 / LPR, NB = NT / 16, U = 8;
+  constexpr int EPL = TS::EPL, LPR = R / EPL, RPS = 64 / LPR, NB = NT / 16, U = 4;
   __shared__ TS sms[4];
   const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   const uint64_t item = (uint64_t)blockIdx.x * 4 + wave;

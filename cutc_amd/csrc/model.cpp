@@ -9,6 +9,7 @@
 #include "ctc_internal.h"
 #include "host_parallel.h"
 #include "kernels_launch.h"
+#include "kernels_mixed.h"
 #include "model_util.h"
 
 using namespace ctc;
@@ -155,7 +156,8 @@ ctc_status ensure_ciss(ctc_model *m, uint32_t mode) {
 static void free_dev_ciss(DevCiss &d) {
   for (int s = 0; s < 3; ++s) dev_free(d.oidx[s]);
   for (void *p : {(void *)d.vals, (void *)d.tile_slot, (void *)d.tile_mask, (void *)d.directory, (void *)d.rowptr,
-                  (void *)d.span_off, (void *)d.slot_pb, (void *)d.grp_piece, (void *)d.grp_n, (void *)d.slot_gb, (void *)d.heavy_slot,
+                  (void *)d.span_off, (void *)d.slot_pb, (void *)d.grp_piece, (void *)d.grp_n, (void *)d.slot_gb,
+                  (void *)d.heavy_slot, (void *)d.thin_items, (void *)d.tile_thin, (void *)d.long_slot,
                   (void *)d.mix_items, (void *)d.mix_heavy_slot, (void *)d.mix_heavy_pb, (void *)d.mix_grp,
                   (void *)d.mix_heavy_gb})
     dev_free(p);
@@ -247,6 +249,38 @@ ctc_status ensure_pieces(ctc_model *m, uint32_t mode, uint32_t span_tiles) {
   d.span_tiles = span_tiles;
   d.nspans = nspans;
   d.npieces = base;
+  return CTC_OK;
+}
+
+// Tables of the rows of at most kSpanThin nonzeros (als_uses_thin).  Few of them
+// stay with the other rows (nthin = 0): a launch of their own pays from about
+// 4096 rows on, a wave each for the chip's slots.
+ctc_status ensure_thin(ctc_model *m, uint32_t mode) {
+  constexpr uint32_t kSpanThin = 16, kThinMin = 4096;
+  DevCiss &d = m->ciss[mode];
+  if (d.thin_ready) return CTC_OK;
+  std::vector<uint4> items;
+  std::vector<uint32_t> rest;
+  std::vector<uint64_t> mask(d.ntiles, 0);
+  for (uint64_t s = 0; s < d.dlength; ++s) {
+    const uint32_t p0 = d.h_rowptr[s], p1 = d.h_rowptr[s + 1];
+    if (p1 - p0 > kSpanThin) {
+      rest.push_back((uint32_t)s);
+      continue;
+    }
+    items.push_back(make_uint4((uint32_t)s, p0, p1, 0u));
+    for (uint32_t p = p0; p < p1; ++p) mask[p >> 6] |= 1ull << (p & 63);
+  }
+  if (items.size() >= kThinMin) {
+    hipStream_t st = m->ctx->stream;
+    CTC_TRY(upload(&d.thin_items, items.data(), items.size(), st));
+    CTC_TRY(upload(&d.tile_thin, mask.data(), mask.size(), st));
+    CTC_TRY(upload(&d.long_slot, rest.data(), rest.size(), st));
+    CTC_HIP(hipStreamSynchronize(st));
+    d.nthin = items.size();
+    d.nlong_slot = rest.size();
+  }
+  d.thin_ready = true;
   return CTC_OK;
 }
 
@@ -581,7 +615,10 @@ extern "C" ctc_status ctc_model_prepare(ctc_model *m, const ctc_options *o) {
     return als_rows_prepare(m, o, o->precision == CTC_PREC_MIXED);
   for (uint32_t md = 0; md < m->nmodes; ++md) {
     CTC_TRY(ensure_ciss(m, md));
-    if (o->algorithm == CTC_ALS) CTC_TRY(ensure_pieces(m, md, als_span_tiles(o, m->ciss[md].nnz)));
+    if (o->algorithm == CTC_ALS) {
+      CTC_TRY(ensure_pieces(m, md, als_span_tiles(o, m->ciss[md].nnz)));
+      if (als_uses_thin(o, m->rank)) CTC_TRY(ensure_thin(m, md));
+    }
   }
   return CTC_OK;
 }
@@ -596,7 +633,10 @@ static ctc_status als_mode_plain(ctc_model *m, uint32_t mode, const ctc_options 
   CTC_TRY(ensure_ciss(m, mode));
   const uint32_t S = als_span_tiles(o, m->ciss[mode].nnz);
   CTC_TRY(ensure_pieces(m, mode, S));
+  const bool use_thin = als_uses_thin(o, R);
+  if (use_thin) CTC_TRY(ensure_thin(m, mode));
   DevCiss &d = m->ciss[mode];
+  const bool thin = use_thin && d.nthin > 0;
   const size_t psz = (size_t)R * R + R;
   CTC_TRY(ensure_scratch(m, (d.npieces + d.ngroups) * psz * sizeof(double)));
   hipStream_t st = m->ctx->stream;
@@ -606,8 +646,8 @@ static ctc_status als_mode_plain(ctc_model *m, uint32_t mode, const ctc_options 
   FactorArgs fa = rel_factors(m->F, m->nmodes, mode);
   {
     Prof p(m->ctx, "als_gram");
-    CTC_HIP(launch_als_gram(st, ca, fa, (int)m->nmodes, (int)R, S, d.nspans, d.span_off, pieces,
-                            block_of(o)));
+    CTC_HIP(launch_als_gram(st, ca, fa, (int)m->nmodes, (int)R, S, d.nspans, d.span_off,
+                            thin ? d.tile_thin : nullptr, pieces, block_of(o)));
   }
   // rows absent from the directory become 0 (SG/als.cu:699 zeroes the factor);
   // the solve writes every other row
@@ -619,7 +659,21 @@ static ctc_status als_mode_plain(ctc_model *m, uint32_t mode, const ctc_options 
   {
     Prof p(m->ctx, "als_solve");
     CTC_HIP(launch_als_solve(st, pieces, d.slot_pb, d.ngroups ? gsum : nullptr, d.slot_gb, d.directory,
-                             d.dlength, (int)R, o->lambda, o->refine != 0, m->F[mode], m->dflag));
+                             thin ? d.long_slot : nullptr, thin ? d.nlong_slot : d.dlength, (int)R, o->lambda, o->refine != 0, m->F[mode], m->dflag));
+  }
+  if (thin) {
+    Prof p(m->ctx, "als_thin");
+    MixedArgs a{};
+    a.prec = kPrecF64;
+    for (uint32_t s = 0; s + 1 < m->nmodes; ++s) a.oidx[s] = d.oidx[s], a.fr[s] = fa.f[1 + s];
+    a.vals = d.vals;
+    a.directory = d.directory;
+    a.out = m->F[mode];
+    a.thin = d.thin_items;
+    a.nthin = a.nthin16 = d.nthin;
+    a.lam = o->lambda;
+    a.flag = m->dflag;
+    CTC_HIP(launch_rows_thin(st, a, (int)m->nmodes, (int)R));
   }
   m->resid_valid = false;
   return CTC_OK;

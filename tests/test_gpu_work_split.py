@@ -202,3 +202,48 @@ def test_als_row_lengths(ctx, rest, mixed, R):
     got = m.factor(0).astype(np.float64)
     for r, n in enumerate(lens):
         assert np.linalg.norm(got[r] - want[r]) <= (1e-4 if mixed else 1e-5) * np.linalg.norm(want[r]), (r, n)
+
+
+@pytest.mark.parametrize("rest", [(47, 39), (23, 19, 17)], ids=["3way", "4way"])
+@pytest.mark.parametrize("longer", [(), (17, 40, 700)], ids=["all_short", "short_and_long"])
+def test_als_short_rows_of_rank_32(ctx, rest, longer):
+    """The default rank-32 ALS update of 5000 rows, of 1 to 16 nonzeros (their dual
+    form; runs of them over tiles and spans) and longer ones between them, eagerly
+    and in a batch's captured graph, against the span kernels alone: both solve
+    in 64 bits, so row by row they agree to a few FP32 roundings (1e-6), and to the
+    ridge solution at the parity tests' bar (1e-5).  Without lambda such rows stay refused."""
+    say(f"[als short rows] rest={rest} longer={longer}")
+    rng = np.random.default_rng(41)
+    lens = rng.integers(1, 17, 5000)
+    for k, n in enumerate(longer):
+        lens[rng.choice(5000, 40, replace=False)] = n
+    lens[[7, 4999]] = 0
+    flat = np.concatenate([rng.choice(int(np.prod(rest)), size=n, replace=False) for n in lens])
+    ind = [np.repeat(np.arange(5000), lens).astype(np.uint32),
+           *(a.astype(np.uint32) for a in np.unravel_index(flat, rest))]
+    vals = rng.uniform(1.0, 5.0, len(flat))
+    dims = (5000, *rest)
+    F = [rng.uniform(-1, 1, (d, 32)).astype(np.float32) for d in dims]
+    t = ct.Coo.from_arrays(ind, vals, dims)
+    m = ct.Model(ctx, t, None, None, rank=32)
+    got = {}
+    for kernel in (ct.ALS_AUTO, ct.ALS_SPANS):
+        m.set_factors(F)
+        m.als_mode_update(0, ct.Options(algorithm=ct.ALS, rank=32, lambda_=0.5, als_kernel=kernel))
+        got[kernel] = m.factor(0).astype(np.float64)
+    want = ridge(ind, vals, F, 0, 0.5)
+    size = np.linalg.norm(want, axis=1)
+    assert np.all(np.linalg.norm(got[ct.ALS_AUTO] - got[ct.ALS_SPANS], axis=1) <= 1e-6 * size)
+    assert np.all(np.linalg.norm(got[ct.ALS_AUTO] - want, axis=1) <= 1e-5 * size)
+    b = ct.Batch(ctx, [t], [None], [32])
+    for k, f in enumerate(F):
+        b.set_factor(0, k, f)
+    b.als(ct.Options(algorithm=ct.ALS, rank=32, lambda_=0.5), iters=1, graph=True)
+    m.set_factors(F)
+    for k in range(len(dims)):
+        m.als_mode_update(k, ct.Options(algorithm=ct.ALS, rank=32, lambda_=0.5))
+    for k in range(len(dims)):
+        np.testing.assert_array_equal(b.factor(0, k), m.factor(k))
+    with pytest.raises(ct.CtcError) as e:
+        m.als_mode_update(0, ct.Options(algorithm=ct.ALS, rank=32, lambda_=0.0))
+    assert e.value.status == 7
