@@ -18,15 +18,14 @@
 // number of gather instructions, not their width, sets its time.
 //
 // Reductions.  One wave walks a span of tiles, one lane per nonzero.  Row
-// sums inside a tile use a segmented inclusive scan (DPP row shifts and
-// broadcasts) that takes each lane's distance to its row's start from the tile
-// mask; the row still open at the end of a tile is carried in a wave-uniform
+// sums inside a tile use a segmented inclusive scan that takes each lane's
+// distance to its row's start from the tile mask; the row still open at the end of a tile is carried in a wave-uniform
 // value into the next tile.  Completed rows are written as (num, den) pieces
 // with the same piece numbering as the ALS Gram pieces, so the per-row sums
 // have a fixed order (deterministic, no atomics).
 //
-// The three passes of a column over 20M nonzeros (480K x 18K x 2K): 135 / 172 /
-// 195 us (169 / 182 / 219 us with the scan on the LDS pipe and no tile in
+// The three passes of a column over 20M nonzeros (480K x 18K x 2K): 137 / 173 /
+// 196 us (169 / 182 / 219 us with the whole scan on the LDS pipe and no tile in
 // flight); the 16 bytes per nonzero that a pass streams take 68 us.
 #include <hip/hip_runtime.h>
 
@@ -37,27 +36,41 @@
 
 namespace ctc {
 
-// one step of the scan: x + the DPP source where the lane's segment reaches it
-// (a select, not a product: the other segments' sums may be infinite)
-template <int CTRL, int ROWS>
-__device__ inline float scan_step(float x, bool reach) {
-  const float u = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), CTRL, ROWS, 0xF, false));
-  return x + (reach ? u : 0.f);
+// x of lane - D (what lanes below D get is not used): whole-wave DPP shifts by
+// one for 1 and 2, a swap of the wave's halves for 32, else a shuffle
+template <int D>
+__device__ inline float lane_before(float x) {
+  int v = __float_as_int(x);
+  if constexpr (D <= 2) {
+#pragma unroll
+    for (int i = 0; i < D; ++i) v = __builtin_amdgcn_update_dpp(0, v, 0x138, 0xF, 0xF, false);
+  } else if constexpr (D == 32) {
+    v = (int)__builtin_amdgcn_permlane32_swap((unsigned)v, (unsigned)v, false, false)[0];
+  } else {
+    return __shfl_up(x, D, 64);
+  }
+  return __int_as_float(v);
+}
+
+template <int D>
+__device__ inline void scan_step(float &a, float &b, int dist) {
+  const float ua = lane_before<D>(a), ub = lane_before<D>(b);
+  a += dist >= D ? ua : 0.f;
+  b += dist >= D ? ub : 0.f;
 }
 
 // Inclusive segmented scan over the wave; dist = lanes from the start of the
-// lane's segment to it.  Row shifts within 16 lanes, then the row ends
-// broadcast to the next row and the half's end to the upper half: no LDS pipe
-// (18 ds_bpermute per tile before) and no flag to carry along.
+// lane's segment to it, so no flag is carried along (18 shuffles on the LDS pipe
+// per tile before, 6 now; with 12 an epoch of 20M nonzeros took 18.05 ms, now 17.45).
+// The order of the sums is kept: a row of few nonzeros can turn a rounding of its
+// sums into a thousand times that in its value.
 __device__ inline void seg_scan(float &a, float &b, int dist) {
-  const int lane = lane_id();
-  a = scan_step<0x111, 0xF>(a, dist >= 1), b = scan_step<0x111, 0xF>(b, dist >= 1);
-  a = scan_step<0x112, 0xF>(a, dist >= 2), b = scan_step<0x112, 0xF>(b, dist >= 2);
-  a = scan_step<0x114, 0xF>(a, dist >= 4), b = scan_step<0x114, 0xF>(b, dist >= 4);
-  a = scan_step<0x118, 0xF>(a, dist >= 8), b = scan_step<0x118, 0xF>(b, dist >= 8);
-  const bool r1 = dist > (lane & 15), r2 = dist > (lane & 31);
-  a = scan_step<0x142, 0xA>(a, r1), b = scan_step<0x142, 0xA>(b, r1);
-  a = scan_step<0x143, 0xC>(a, r2), b = scan_step<0x143, 0xC>(b, r2);
+  scan_step<1>(a, b, dist);
+  scan_step<2>(a, b, dist);
+  scan_step<4>(a, b, dist);
+  scan_step<8>(a, b, dist);
+  scan_step<16>(a, b, dist);
+  scan_step<32>(a, b, dist);
 }
 
 __device__ inline float lane_value(float x, uint32_t lane) {
@@ -243,7 +256,8 @@ __device__ inline void ccd_finish_wave(uint64_t slot, const double *pieces, cons
 // each, a lane per slot, whose few pieces are added in piece order.  The slots,
 // their rows and their records are consecutive, so the kernel is a stream; with
 // the slots dealt to the blocks in a stride, which kept the long rows (the
-// hottest are numbered first) apart, 480K slots took 25 us; now 9 us.
+// hottest are numbered first) apart, 480K slots took 25 us; the three modes of
+// that tensor now take 5.5 us on average.
 __global__ void __launch_bounds__(256) k_ccd_finish(const double *pieces, const uint32_t *slot_pb,
                                                     const uint32_t *heavy, uint64_t nheavy, uint32_t hb,
                                                     const uint32_t *directory, uint64_t dlength, double lam,
