@@ -1519,14 +1519,28 @@ __global__ void __launch_bounds__(256) k_eval_seg(CissArgs c, CooArgs co, Factor
   block_store_sum(acc, part + (size_t)blockIdx.x * gridDim.y + blockIdx.y);
 }
 
-__global__ void __launch_bounds__(256) k_sumsq(const float *x, uint64_t n, double *part) {
+// blockIdx.y: one of several arrays, n[y] entries
+__global__ void __launch_bounds__(256) k_sumsq(FactorArgs x, RowCounts len, double *part) {
   double acc = 0.0;
+  const float *f = x.f[blockIdx.y];
+  const uint64_t n = len.n[blockIdx.y];
   for (uint64_t p = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; p < n;
        p += (uint64_t)gridDim.x * blockDim.x) {
-    const double v = x[p];
+    const double v = f[p];
     acc += v * v;
   }
-  block_store_sum(acc, part + blockIdx.x);
+  block_store_sum(acc, part + (size_t)blockIdx.y * gridDim.x + blockIdx.x);
+}
+
+// out[0] = sum of first[0 .. nfirst), out[1 + k] = sum of part[k * nb .. k * nb + nb),
+// each in a fixed order
+__global__ void __launch_bounds__(256) k_reduce_stats(const double *first, uint32_t nfirst, const double *part,
+                                                      uint32_t nb, double *out) {
+  const double *p = blockIdx.x ? part + (size_t)(blockIdx.x - 1) * nb : first;
+  const uint32_t n = blockIdx.x ? nb : nfirst;
+  double acc = 0.0;
+  for (uint32_t i = threadIdx.x; i < n; i += 256) acc += p[i];
+  block_store_sum(acc, out + blockIdx.x);
 }
 
 // out[k] = sum of part[k * nb .. k * nb + nb) in a fixed order
@@ -1901,8 +1915,15 @@ hipError_t launch_eval_seg(hipStream_t st, const CissArgs *c, const CooArgs *co,
   return e != hipSuccess ? e : launch_reduce_parts(st, part, kSegBlocks, nseg, out);
 }
 
-hipError_t launch_sumsq(hipStream_t st, const float *x, uint64_t n, unsigned nblocks, double *part) {
-  hipLaunchKernelGGL(k_sumsq, dim3(nblocks), dim3(256), 0, st, x, n, part);
+hipError_t launch_sumsq(hipStream_t st, const FactorArgs &x, const RowCounts &len, int count, unsigned nblocks,
+                        double *part) {
+  hipLaunchKernelGGL(k_sumsq, dim3(nblocks, (unsigned)count), dim3(256), 0, st, x, len, part);
+  return hipGetLastError();
+}
+
+hipError_t launch_reduce_stats(hipStream_t st, const double *first, uint32_t nfirst, const double *part, uint32_t nb,
+                               uint32_t groups, double *out) {
+  hipLaunchKernelGGL(k_reduce_stats, dim3(1 + groups), dim3(256), 0, st, first, nfirst, part, nb, out);
   return hipGetLastError();
 }
 

@@ -55,7 +55,14 @@ hipError_t launch_eval_coo(hipStream_t st, const CooArgs &c, const FactorArgs &f
 constexpr unsigned kSegBlocks = 64;
 hipError_t launch_eval_seg(hipStream_t st, const CissArgs *c, const CooArgs *co, const FactorArgs &f,
                            int nmodes, int R, const uint64_t *seg, uint32_t nseg, double *part, double *out);
-hipError_t launch_sumsq(hipStream_t st, const float *x, uint64_t n, unsigned nblocks, double *part);
+// sums of squares of `count` arrays, nblocks partials each
+struct RowCounts {
+  uint64_t n[4];
+};
+hipError_t launch_sumsq(hipStream_t st, const FactorArgs &x, const RowCounts &len, int count, unsigned nblocks,
+                        double *part);
+hipError_t launch_reduce_stats(hipStream_t st, const double *first, uint32_t nfirst, const double *part, uint32_t nb,
+                               uint32_t groups, double *out);
 hipError_t launch_reduce_parts(hipStream_t st, const double *part, uint32_t nb, uint32_t groups,
                                double *out);
 hipError_t launch_fill(hipStream_t st, float *x, uint64_t n, float v);
