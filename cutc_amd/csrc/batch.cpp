@@ -264,7 +264,7 @@ static ctc_options class_options(const RankClass &c, const ctc_options *o) {
 // that the sweep itself only launches kernels
 static ctc_status prepare_class(RankClass &c, const ctc_options *t) {
   ctc_model *m = c.model;
-  if (als_uses_rows(t, c.rank)) return als_rows_prepare(m, t, t->precision == CTC_PREC_MIXED);
+  if (als_uses_rows(t, c.rank, m->train_nnz)) return als_rows_prepare(m, t, t->precision == CTC_PREC_MIXED);
   size_t need = 0;
   for (uint32_t md = 0; md < m->nmodes; ++md) {
     CTC_TRY(ensure_ciss(m, md));

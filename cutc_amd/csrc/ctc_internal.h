@@ -246,14 +246,22 @@ ctc_status als_mode_rows(ctc_model *m, uint32_t mode, const ctc_options *o, bool
 // everything als_mode_rows allocates or uploads, for all modes
 ctc_status als_rows_prepare(ctc_model *m, const ctc_options *o, bool bf16);
 // which FP32 ALS kernels a model of rank R uses under these options
-inline bool als_uses_rows(const ctc_options *o, uint32_t R) {
-  return o->precision == CTC_PREC_MIXED || o->als_kernel == CTC_ALS_ROWS || (o->als_kernel == CTC_ALS_AUTO && R >= 64);
+//
+// By default rank 32 takes them from kRowsNnz nonzeros on, where the workgroups'
+// chunks of 1024 nonzeros fill the chip: a sweep of 20M nonzeros 3.36 ms (spans
+// 3.87), 3.7M 0.81 (0.89), but 0.86M 0.48 (0.40), 0.1M 0.41 (0.29).  lambda > 0
+// and no refinement or tile length asked for, as in als_uses_thin below.
+constexpr uint64_t kRowsNnz = 4000000;
+inline bool als_uses_rows(const ctc_options *o, uint32_t R, uint64_t nnz) {
+  if (o->precision == CTC_PREC_MIXED || o->als_kernel == CTC_ALS_ROWS) return true;
+  if (o->als_kernel != CTC_ALS_AUTO) return false;
+  return R >= 64 || (R == 32 && nnz >= kRowsNnz && !o->tile_len && !o->refine && o->lambda > 0.0);
 }
 // Whether the span ALS may solve its short rows in their dual form: at rank 32 a
 // row of at most 16 nonzeros is an n x n system in place of the 32 x 32 one and of
 // its 8 KB piece.  Only with lambda > 0 (without it such a row is singular, and
-// is reported), the default kernel choice and no refinement.  Sweep of 20M nonzeros
-// with 375K such rows 3.74 ms, without this 5.82 ms.
+// is reported), the default kernel choice and no refinement.  Span sweep of 20M
+// nonzeros with 375K such rows 3.74 ms, without this 5.82 ms.
 inline bool als_uses_thin(const ctc_options *o, uint32_t R) {
   return R == 32 && o->precision == CTC_PREC_FP32 && o->als_kernel == CTC_ALS_AUTO && !o->refine && o->lambda > 0.0;
 }

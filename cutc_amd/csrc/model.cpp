@@ -611,7 +611,7 @@ extern "C" ctc_status ctc_model_prepare(ctc_model *m, const ctc_options *o) {
   if (!m || !o) return fail(CTC_ERR_INVALID_ARG, "ctc_model_prepare");
   CTC_HIP(hipSetDevice(m->ctx->device));
   if (o->algorithm == CTC_SGD) return ensure_ciss(m, 0);
-  if (o->algorithm == CTC_ALS && als_uses_rows(o, m->rank))
+  if (o->algorithm == CTC_ALS && als_uses_rows(o, m->rank, m->train_nnz))
     return als_rows_prepare(m, o, o->precision == CTC_PREC_MIXED);
   for (uint32_t md = 0; md < m->nmodes; ++md) {
     CTC_TRY(ensure_ciss(m, md));
@@ -628,7 +628,7 @@ extern "C" ctc_status ctc_model_prepare(ctc_model *m, const ctc_options *o) {
 // =========================================================================
 static ctc_status als_mode_plain(ctc_model *m, uint32_t mode, const ctc_options *o) {
   const uint32_t R = m->rank;
-  if (als_uses_rows(o, R)) return als_mode_rows(m, mode, o, o->precision == CTC_PREC_MIXED);
+  if (als_uses_rows(o, R, m->train_nnz)) return als_mode_rows(m, mode, o, o->precision == CTC_PREC_MIXED);
   if (R > 64) return fail(CTC_ERR_UNSUPPORTED, "the span ALS kernels support ranks up to 64 (got %u)", R);
   CTC_TRY(ensure_ciss(m, mode));
   const uint32_t S = als_span_tiles(o, m->ciss[mode].nnz);

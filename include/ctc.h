@@ -246,8 +246,9 @@ typedef enum ctc_ref_quirk {
  * per-(span, row) FP64 Gram pieces, a second kernel sums a row's pieces and
  * solves (ranks 8-64).  ROWS: one workgroup per row forms its Gram on FP64
  * matrix cores and solves it in place with a blocked FP64 Cholesky, long
- * rows cut into chunks (ranks 32-128).  AUTO: ROWS for rank >= 64 (at rank 32
- * SPANS measured faster on the 100M-nonzero benchmark tensor). */
+ * rows cut into chunks (ranks 32-128).  AUTO: ROWS for rank >= 64 and, with
+ * lambda > 0, no refinement and no tile_len, for rank 32 from 4M training
+ * nonzeros on; below that, SPANS with the short rows in their dual form. */
 typedef enum ctc_als_kernel { CTC_ALS_AUTO = 0, CTC_ALS_SPANS = 1, CTC_ALS_ROWS = 2 } ctc_als_kernel;
 
 typedef enum ctc_sgd_update {

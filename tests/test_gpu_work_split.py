@@ -247,3 +247,22 @@ def test_als_short_rows_of_rank_32(ctx, rest, longer):
     with pytest.raises(ct.CtcError) as e:
         m.als_mode_update(0, ct.Options(algorithm=ct.ALS, rank=32, lambda_=0.0))
     assert e.value.status == 7
+
+
+def test_als_rank_32_kernel_by_size(ctx):
+    """The default rank-32 ALS update on both sides of the size from which it runs
+    the row-fused kernels, against the span kernels: both sum and solve in 64 bits, so
+    the factors agree to a few FP32 roundings (1e-6)."""
+    for nnz in (3_990_000, 4_010_000):
+        say(f"[als rank 32 by size] nnz={nnz}")
+        t, _ = ct.synth((3000, 400, 300), nnz, zipf=(1.0, 0.5, 0.0), test_fraction=0.0, seed=9)
+        rng = np.random.default_rng(51)
+        F = [rng.uniform(-1, 1, (d, 32)).astype(np.float32) for d in t.dims]
+        m = ct.Model(ctx, t, None, None, rank=32)
+        for mode in range(3):
+            got = []
+            for kernel in (ct.ALS_AUTO, ct.ALS_SPANS):
+                m.set_factors(F)
+                m.als_mode_update(mode, ct.Options(algorithm=ct.ALS, rank=32, lambda_=0.05, als_kernel=kernel))
+                got.append(m.factor(mode).astype(np.float64))
+            assert np.linalg.norm(got[0] - got[1]) <= 1e-6 * np.linalg.norm(got[1]), (nnz, mode)
