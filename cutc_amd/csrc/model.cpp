@@ -1471,6 +1471,10 @@ extern "C" ctc_status ctc_autotune(ctc_model *m, const ctc_options *o, ctc_tune_
     subs = {16, 32, 64};
     blocks = {64, 256};
   }
+  // ALS's default is not one of the lengths: its spans are sized by each mode, and
+  // at rank 32 it may be the row-fused kernels (als_uses_rows), which no other
+  // trial reaches
+  if (o->algorithm == CTC_ALS) tiles.insert(tiles.begin(), 0u);
   hipEvent_t e0, e1;
   CTC_HIP(hipEventCreate(&e0));
   CTC_HIP(hipEventCreate(&e1));

@@ -458,8 +458,9 @@ typedef struct ctc_tune_result {
 /* Measured search over the work-unit shape of opt->algorithm's sweep, the
  * GA's fitness (mean epoch time over (blocksize, tile length),
  * GA/fitness.c:31-100): ALS / CCD++ / lock-free SGD over tile_len 64..4096 and
- * block 64..256; the default SGD schedule over walker spans 1024..8192,
- * sub-steps 16..64 and blocks 64 / 256 (span and sub-step define that
+ * block 64..256, ALS also over its default (tile_len 0 in the result: what an
+ * update without a tile_len runs); the default SGD schedule over walker spans
+ * 1024..8192, sub-steps 16..64 and blocks 64 / 256 (span and sub-step define that
  * schedule, so the tuned shape is what later solves with it compute).  The
  * factors and the best-model copy are restored afterwards. */
 

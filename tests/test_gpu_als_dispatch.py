@@ -1,0 +1,40 @@
+"""Which kernels a call runs, read from the context's kernel statistics."""
+import sys
+
+import numpy as np
+import pytest
+
+import cutc_amd as ct
+
+pytestmark = pytest.mark.gpu
+
+
+def say(*a):
+    print(*a, flush=True)
+    sys.stdout.flush()
+
+
+def launches(ctx, *names):
+    return {n: ctx.kernel_stats(n)[0] for n in names}
+
+
+def test_autotune_times_the_default_als_kernels():
+    """Autotuning rank-32 ALS from the size on from which the row-fused kernels are
+    the default times them as well as the spans, and the shape it returns runs."""
+    say("[autotune default als]")
+    ctx = ct.Context(0)
+    t, _ = ct.synth((3000, 400, 300), 4_010_000, zipf=(1.0, 0.5, 0.0), test_fraction=0.0, seed=9)
+    m = ct.Model(ctx, t, None, None, rank=32)
+    rng = np.random.default_rng(61)
+    m.set_factors([rng.uniform(-1, 1, (d, 32)).astype(np.float32) for d in t.dims])
+    ctx.set_profiling(True)
+    ctx.reset_stats()
+    r = m.autotune(ct.Options(algorithm=ct.ALS, rank=32, lambda_=0.05))
+    n = launches(ctx, "als_gram", "als_rows_items", "als_rows_chunks")
+    say(f"  {r} {n}")
+    assert n["als_gram"] > 0 and n["als_rows_items"] + n["als_rows_chunks"] > 0
+    ctx.reset_stats()
+    m.als_mode_update(0, ct.Options(algorithm=ct.ALS, rank=32, lambda_=0.05, tile_len=r["tile_len"], block=r["block"]))
+    n = launches(ctx, "als_gram", "als_rows_items", "als_rows_chunks")
+    rows = n["als_rows_items"] + n["als_rows_chunks"] > 0
+    assert rows == (r["tile_len"] == 0) and rows != (n["als_gram"] > 0)
