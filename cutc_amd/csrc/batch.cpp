@@ -32,7 +32,8 @@ struct RankClass {
   ctc_model *model = nullptr;
   uint64_t *seg_train = nullptr, *seg_test = nullptr;  // device, nprob + 1 each
   double *dsum = nullptr;                              // device, 2 * nprob
-  double *dpart = nullptr;                             // device, nprob * kSegBlocks
+  unsigned seg_blocks = 1;                             // blocks that share a problem's RMSE
+  double *dpart = nullptr;                             // device, 2 * nprob * seg_blocks where those are several
   bool tuned = false;
   uint32_t tile_len = 0, block = 0;
   hipEvent_t join = nullptr;
@@ -181,10 +182,13 @@ extern "C" ctc_status ctc_batch_create(ctc_context *ctx, uint32_t nproblems, con
     ctc_coo_free(cte);
     if (s != CTC_OK) break;
     b->total_train += seg_tr[np];
+    uint64_t longest = 0;
+    for (const uint32_t p : c.problems) longest = std::max({longest, b->place[p].ntrain, b->place[p].ntest});
+    c.seg_blocks = eval_seg_blocks((int)c.rank, (uint32_t)np, longest);
     if (hipMalloc(&c.seg_train, (np + 1) * sizeof(uint64_t)) != hipSuccess ||
         hipMalloc(&c.seg_test, (np + 1) * sizeof(uint64_t)) != hipSuccess ||
         hipMalloc(&c.dsum, 2 * np * sizeof(double)) != hipSuccess ||
-        hipMalloc(&c.dpart, np * kSegBlocks * sizeof(double)) != hipSuccess) {
+        (c.seg_blocks > 1 && hipMalloc(&c.dpart, 2 * np * c.seg_blocks * sizeof(double)) != hipSuccess)) {
       s = fail(CTC_ERR_NOMEM, "batch segment tables");
       break;
     }
@@ -417,11 +421,13 @@ extern "C" ctc_status ctc_batch_rmse(ctc_batch *b, double *rmse_tr, double *rmse
     ct.nnz = m->test.nnz;
     FactorArgs fa{};
     for (uint32_t md = 0; md < m->nmodes; ++md) fa.f[md] = m->F[md];
-    CTC_HIP(launch_eval_seg(st, &ca, nullptr, fa, (int)m->nmodes, (int)c.rank, c.seg_train, np, c.dpart,
-                            c.dsum));
+    const unsigned nb = c.seg_blocks;
+    double *part = nb > 1 ? c.dpart : c.dsum;  // train, then test
+    CTC_HIP(launch_eval_seg(st, &ca, nullptr, fa, (int)m->nmodes, (int)c.rank, c.seg_train, np, nb, part));
     if (m->test.nnz)
-      CTC_HIP(launch_eval_seg(st, nullptr, &ct, fa, (int)m->nmodes, (int)c.rank, c.seg_test, np, c.dpart,
-                              c.dsum + np));
+      CTC_HIP(launch_eval_seg(st, nullptr, &ct, fa, (int)m->nmodes, (int)c.rank, c.seg_test, np, nb,
+                              part + (size_t)np * nb));
+    if (nb > 1) CTC_HIP(launch_reduce_parts(st, part, nb, (m->test.nnz ? 2 : 1) * np, c.dsum));
     sums[ci].assign(2 * (size_t)np, 0.0);
   }
   for (size_t ci = 0; ci < b->cls.size(); ++ci) {

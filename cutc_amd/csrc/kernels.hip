@@ -16,6 +16,7 @@
 //     walker's first nonzero is the tile header's first slot.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdint>
 
 #include "kernels_common.h"
@@ -1478,10 +1479,10 @@ __global__ void __launch_bounds__(256) k_eval_coo(CooArgs c, FactorArgs fa, int 
 // part[b * gridDim.y + y].  CISS=true reads mode-0 CISS order, false a COO.
 // Bound by the row gathers.  Walkers of R / 4 lanes move a row as one 16-byte
 // load per lane, the walkers of a segment's blocks take its nonzeros in turn,
-// and the FP32 prediction is summed over the walker's lanes.  Few segments are the
-// common case, so a segment is shared by kSegBlocks blocks: with one block per
-// segment and a lane per nonzero, 24 problems of 0.3M nonzeros (six per rank)
-// took 24 ms of an 80 ms pass of ten iterations; this way the pass takes 56 ms.
+// and the FP32 prediction is summed over the walker's lanes.  A long segment is
+// shared by several blocks (eval_seg_blocks): with one block per segment and a
+// lane per nonzero, 24 problems of 0.3M nonzeros (six per rank) took 24 ms of an
+// 80 ms pass of ten iterations, which 64 blocks per segment made 56 ms.
 template <int R, int N, bool CISS>
 __global__ void __launch_bounds__(256) k_eval_seg(CissArgs c, CooArgs co, FactorArgs fa, const uint64_t *seg,
                                                   double *part) {
@@ -1889,20 +1890,32 @@ hipError_t launch_eval_coo(hipStream_t st, const CooArgs &c, const FactorArgs &f
   return hipGetLastError();
 }
 
+// Blocks that share a segment: eight nonzeros for each walker of the longest
+// segment's blocks, and no more than 8192 blocks for all segments, 32 a CU, since a
+// block costs more than a short segment's nonzeros.  RMSE of a batch of 2000 problems
+// of 300 nonzeros 127 us, 400 of 4000 137 us, 4 of 5000 115 us; with 64 blocks for
+// every segment 243 / 154 / 124 us, with one 145 / 281 / 272 us; 4, 16 and 32 nonzeros
+// a walker differ by up to 2, 7 and 25 percent.
+unsigned eval_seg_blocks(int R, uint32_t nseg, uint64_t longest) {
+  const uint64_t share = 8 * 1024 / (uint64_t)R;  // a block has 256 / (R / 4) walkers
+  const uint64_t most = std::min<uint64_t>(kSegBlocks, std::max<uint64_t>(1, 8192 / nseg));
+  return (unsigned)std::min(most, std::max<uint64_t>(1, (longest + share - 1) / share));
+}
+
 hipError_t launch_eval_seg(hipStream_t st, const CissArgs *c, const CooArgs *co, const FactorArgs &f,
-                           int nmodes, int R, const uint64_t *seg, uint32_t nseg, double *part, double *out) {
+                           int nmodes, int R, const uint64_t *seg, uint32_t nseg, unsigned blocks, double *part) {
   if (nseg == 0) return hipSuccess;
   const CissArgs ca = c ? *c : CissArgs{};
   const CooArgs cb = co ? *co : CooArgs{};
-#define CTC_SEG(NN)                                                                                        \
-  do {                                                                                                     \
-    if (c) {                                                                                               \
-      CTC_R_SWITCH(R, hipLaunchKernelGGL((k_eval_seg<RR, NN, true>), dim3(nseg, kSegBlocks), dim3(256), 0, \
-                                         st, ca, cb, f, seg, part));                                       \
-    } else {                                                                                               \
-      CTC_R_SWITCH(R, hipLaunchKernelGGL((k_eval_seg<RR, NN, false>), dim3(nseg, kSegBlocks), dim3(256), 0, \
-                                         st, ca, cb, f, seg, part));                                       \
-    }                                                                                                      \
+#define CTC_SEG(NN)                                                                                                  \
+  do {                                                                                                               \
+    if (c) {                                                                                                         \
+      CTC_R_SWITCH(R, hipLaunchKernelGGL((k_eval_seg<RR, NN, true>), dim3(nseg, blocks), dim3(256), 0, st, ca, cb, \
+                                         f, seg, part));                                                             \
+    } else {                                                                                                         \
+      CTC_R_SWITCH(R, hipLaunchKernelGGL((k_eval_seg<RR, NN, false>), dim3(nseg, blocks), dim3(256), 0, st, ca, cb, \
+                                         f, seg, part));                                                             \
+    }                                                                                                                \
   } while (0)
   if (nmodes == 3)
     CTC_SEG(3);
@@ -1911,8 +1924,7 @@ hipError_t launch_eval_seg(hipStream_t st, const CissArgs *c, const CooArgs *co,
   else
     return hipErrorInvalidValue;
 #undef CTC_SEG
-  const hipError_t e = hipGetLastError();
-  return e != hipSuccess ? e : launch_reduce_parts(st, part, kSegBlocks, nseg, out);
+  return hipGetLastError();
 }
 
 hipError_t launch_sumsq(hipStream_t st, const FactorArgs &x, const RowCounts &len, int count, unsigned nblocks,

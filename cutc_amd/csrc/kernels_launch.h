@@ -50,11 +50,12 @@ hipError_t launch_als_solve(hipStream_t st, const double *pieces, const uint32_t
 hipError_t launch_eval_coo(hipStream_t st, const CooArgs &c, const FactorArgs &f, int nmodes, int R,
                            unsigned nblocks, double *part);
 // per-segment squared error: exactly one of c (mode-0 CISS order) / co (COO) is
-// non-null.  Each segment is shared by kSegBlocks blocks, whose partials
-// (part: nseg x kSegBlocks) are added in order into out[segment].
+// non-null.  Each segment is shared by `blocks` blocks, whose partials are part
+// (nseg x blocks), to be added in order; with one block, part is the result.
 constexpr unsigned kSegBlocks = 64;
+unsigned eval_seg_blocks(int R, uint32_t nseg, uint64_t longest);
 hipError_t launch_eval_seg(hipStream_t st, const CissArgs *c, const CooArgs *co, const FactorArgs &f,
-                           int nmodes, int R, const uint64_t *seg, uint32_t nseg, double *part, double *out);
+                           int nmodes, int R, const uint64_t *seg, uint32_t nseg, unsigned blocks, double *part);
 // sums of squares of `count` arrays, nblocks partials each
 struct RowCounts {
   uint64_t n[4];

@@ -266,3 +266,31 @@ def test_als_rank_32_kernel_by_size(ctx):
                 m.als_mode_update(mode, ct.Options(algorithm=ct.ALS, rank=32, lambda_=0.05, als_kernel=kernel))
                 got.append(m.factor(mode).astype(np.float64))
             assert np.linalg.norm(got[0] - got[1]) <= 1e-6 * np.linalg.norm(got[1]), (nnz, mode)
+
+
+@pytest.mark.parametrize("R,count,longest", [(8, 3, 1024), (8, 3, 1025), (64, 140, 20_000), (8, 5000, 3000)],
+                         ids=["one_block", "two_blocks", "shared_by_58", "one_block_each"])
+def test_batch_rmse_of_many_problems(ctx, R, count, longest):
+    """Per-problem RMSE where the blocks that share a problem are set by the longest
+    one and by the number of problems, with and without test entries.  The bound is
+    that of test_batch_rmse_of_segments."""
+    say(f"[batch rmse many] R={R} count={count} longest={longest}")
+    dims, rng = (40, 35, 30), np.random.default_rng(71)
+    sizes = rng.integers(1, 20, count)
+    sizes[count // 2] = longest
+    probs, tests, wt, we = [], [], [], []
+    F = [rng.uniform(-1, 1, (d, R)).astype(np.float32) for d in dims]
+    for k, n in enumerate(sizes):
+        t, ind, vals = coo(dims, n, 1000 + k)
+        e, eind, evals = coo(dims, 3, 90_000 + k)
+        probs.append(t), tests.append(e if k % 3 else None)
+        wt.append(np.sqrt(np.mean((vals - predict(ind, F)) ** 2)))
+        we.append(np.sqrt(np.mean((evals - predict(eind, F)) ** 2)) if k % 3 else 0.0)
+    b = ct.Batch(ctx, probs, tests, [R] * count)
+    for p in range(count):
+        for m, f in enumerate(F):
+            b.set_factor(p, m, f)
+    for _ in range(2):
+        tr, te = b.rmse()
+        np.testing.assert_allclose(tr, wt, rtol=1e-6, atol=4e-6)
+        np.testing.assert_allclose(te, we, rtol=1e-6, atol=4e-6)
