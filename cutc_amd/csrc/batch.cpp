@@ -272,10 +272,10 @@ static ctc_status prepare_class(RankClass &c, const ctc_options *t) {
   size_t need = 0;
   for (uint32_t md = 0; md < m->nmodes; ++md) {
     CTC_TRY(ensure_ciss(m, md));
-    CTC_TRY(ensure_pieces(m, md, als_span_tiles(t, m->ciss[md].nnz)));
+    const PieceTables *pt = nullptr;
+    CTC_TRY(ensure_pieces(m, md, als_span_tiles(t, m->ciss[md].nnz), &pt));
     if (als_uses_thin(t, c.rank)) CTC_TRY(ensure_thin(m, md));
-    const DevCiss &d = m->ciss[md];
-    need = std::max(need, (size_t)(d.npieces + d.ngroups) * ((size_t)c.rank * c.rank + c.rank) * sizeof(double));
+    need = std::max(need, (size_t)(pt->npieces + pt->ngroups) * ((size_t)c.rank * c.rank + c.rank) * sizeof(double));
   }
   return ensure_scratch(m, need);
 }
@@ -337,9 +337,10 @@ static std::vector<uintptr_t> graph_key_of(ctc_batch *b, const ctc_options *o, u
     k.push_back((uintptr_t)c.model->scratch);
     for (uint32_t md = 0; md < b->nmodes; ++md) {
       const DevCiss &d = c.model->ciss[md];
-      k.push_back((uintptr_t)d.slot_pb);
-      k.push_back((uintptr_t)d.span_off);
-      k.push_back((uintptr_t)d.slot_gb);
+      const PieceTables &pt = d.pieces[d.pieces_last];  // prepare_class asked for the ones in use
+      k.push_back((uintptr_t)pt.slot_pb);
+      k.push_back((uintptr_t)pt.span_off);
+      k.push_back((uintptr_t)pt.slot_gb);
       k.push_back((uintptr_t)(als_uses_thin(&t, c.rank) ? d.thin_items : nullptr));
       k.push_back((uintptr_t)d.mix_items);
       k.push_back((uintptr_t)d.mix_chunk);

@@ -27,10 +27,11 @@ ctc_status ccd_epoch_impl(ctc_model *m, const ctc_options *o) {
   const uint32_t inner = o->inner_iters ? o->inner_iters : 1;
   hipStream_t st = m->ctx->stream;
   size_t max_pieces = 0;
+  const PieceTables *pt[CTC_MAX_MODES] = {nullptr, nullptr, nullptr, nullptr};
   for (uint32_t md = 0; md < N; ++md) {
     CTC_TRY(ensure_ciss(m, md));
-    CTC_TRY(ensure_pieces(m, md, S));
-    max_pieces = std::max<size_t>(max_pieces, m->ciss[md].npieces);
+    CTC_TRY(ensure_pieces(m, md, S, &pt[md]));
+    max_pieces = std::max<size_t>(max_pieces, pt[md]->npieces);
     if (!m->FT[md]) CTC_HIP(hipMalloc(&m->FT[md], m->dims[md] * R * sizeof(float)));
     if (!m->ccdx[md]) CTC_HIP(hipMalloc(&m->ccdx[md], std::max<uint64_t>(1, m->dims[md]) * 4 * sizeof(float)));
     if (!m->resid[md]) {
@@ -72,8 +73,8 @@ ctc_status ccd_epoch_impl(ctc_model *m, const ctc_options *o) {
         a.add_back = it == 0 ? 1 : 0;
         a.resid = m->resid[md];
         a.span_tiles = S;
-        a.nspans = d.nspans;
-        a.span_off = d.span_off;
+        a.nspans = pt[md]->nspans;
+        a.span_off = pt[md]->span_off;
         a.pieces = pieces;
         a.lds_s = -1;  // a small other mode's records are read from LDS (3-way tensors)
         if (N == 3)
@@ -90,8 +91,8 @@ ctc_status ccd_epoch_impl(ctc_model *m, const ctc_options *o) {
         }
         {
           Prof p(m->ctx, "ccd_finish");
-          CTC_HIP(launch_ccd_finish(st, pieces, d.slot_pb, d.heavy_slot, d.nheavy_slot, d.directory, d.dlength,
-                                    o->lambda, col, (float4 *)m->ccdx[md]));
+          CTC_HIP(launch_ccd_finish(st, pieces, pt[md]->slot_pb, pt[md]->heavy_slot, pt[md]->nheavy_slot, d.directory,
+                                    d.dlength, o->lambda, col, (float4 *)m->ccdx[md]));
         }
       }
     }

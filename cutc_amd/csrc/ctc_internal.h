@@ -59,19 +59,10 @@ ctc_status build_host_ciss(const ctc_coo *t, uint32_t mode, HostCiss &out);
 ctc_status quirk_multiset(const ctc_coo *t, uint32_t mode, uint32_t flags, ctc_coo **out);
 
 // ----------------------------------------------------------- device CISS --
-// Device copy of one mode's CISS plus the per-span piece tables used by the
-// deterministic segmented reductions (see kernels.hip).
-struct DevCiss {
-  uint32_t nmodes = 0, mode = 0;
-  uint64_t nnz = 0, ntiles = 0, dlength = 0;
-  uint32_t *oidx[CTC_MAX_MODES - 1] = {nullptr, nullptr, nullptr};
-  float *vals = nullptr;
-  uint32_t *tile_slot = nullptr;
-  uint64_t *tile_mask = nullptr;
-  uint32_t *directory = nullptr;
-  uint32_t *rowptr = nullptr;
-  // piece tables for span_tiles tiles per span
-  uint32_t span_tiles = 0;
+// The pieces (span, row) of a mode's CISS for spans of span_tiles tiles, which the
+// deterministic segmented reductions write and add (see kernels.hip)
+struct PieceTables {
+  uint32_t span_tiles = 0;  // 0: not built
   uint64_t nspans = 0, npieces = 0;
   uint32_t *span_off = nullptr;  // nspans: piece id = slot + span_off[span]
   uint32_t *slot_pb = nullptr;   // dlength + 1: pieces of slot s
@@ -83,6 +74,22 @@ struct DevCiss {
   uint32_t *grp_piece = nullptr;  // ngroups: first piece of group g
   uint32_t *grp_n = nullptr;      // ngroups: pieces in group g
   uint32_t *slot_gb = nullptr;    // dlength + 1: groups of slot s (empty for light slots)
+};
+
+// Device copy of one mode's CISS and the tables built over it
+struct DevCiss {
+  uint32_t nmodes = 0, mode = 0;
+  uint64_t nnz = 0, ntiles = 0, dlength = 0;
+  uint32_t *oidx[CTC_MAX_MODES - 1] = {nullptr, nullptr, nullptr};
+  float *vals = nullptr;
+  uint32_t *tile_slot = nullptr;
+  uint64_t *tile_mask = nullptr;
+  uint32_t *directory = nullptr;
+  uint32_t *rowptr = nullptr;
+  // piece tables of two span lengths: ALS and CCD++ have each their own, and a
+  // program may run both in turn (ensure_pieces)
+  PieceTables pieces[2];
+  uint32_t pieces_last = 0;  // the one asked for last
   // short rows that the FP32 span ALS solves in their dual form (ensure_thin):
   // their items, the nonzeros they cover (a bit per nonzero of a tile) and the other rows' slots
   bool thin_ready = false;
@@ -227,7 +234,8 @@ namespace ctc {
 ctc_status ensure_scratch(ctc_model *m, size_t bytes);
 ctc_status ensure_ciss(ctc_model *m, uint32_t mode);
 ctc_status ensure_thin(ctc_model *m, uint32_t mode);
-ctc_status ensure_pieces(ctc_model *m, uint32_t mode, uint32_t span_tiles);
+// *out stays valid until tables of two other span lengths have been asked for
+ctc_status ensure_pieces(ctc_model *m, uint32_t mode, uint32_t span_tiles, const PieceTables **out);
 // every ctc_ref_quirk bit
 constexpr uint32_t kQuirkAll = CTC_QUIRK_TILE_HEAD | CTC_QUIRK_LAST_LANE | CTC_QUIRK_TRUNC_VALUES |
                                CTC_QUIRK_NO_ADDBACK | CTC_QUIRK_CCD_GRID;

@@ -139,7 +139,6 @@ static ctc_status upload_ciss(ctc_model *m, HostCiss &h, DevCiss &d, uint32_t mo
   d.h_tile_slot.swap(h.tile_slot);
   d.h_tile_mask.swap(h.tile_mask);
   d.h_rowptr.swap(h.rowptr);
-  d.span_tiles = 0;
   return CTC_OK;
 }
 
@@ -153,11 +152,16 @@ ctc_status ensure_ciss(ctc_model *m, uint32_t mode) {
   return CTC_OK;
 }
 
+static void free_pieces(PieceTables &t) {
+  for (uint32_t *p : {t.span_off, t.slot_pb, t.heavy_slot, t.grp_piece, t.grp_n, t.slot_gb}) dev_free(p);
+  t = PieceTables();
+}
+
 static void free_dev_ciss(DevCiss &d) {
+  for (PieceTables &t : d.pieces) free_pieces(t);
   for (int s = 0; s < 3; ++s) dev_free(d.oidx[s]);
   for (void *p : {(void *)d.vals, (void *)d.tile_slot, (void *)d.tile_mask, (void *)d.directory, (void *)d.rowptr,
-                  (void *)d.span_off, (void *)d.slot_pb, (void *)d.grp_piece, (void *)d.grp_n, (void *)d.slot_gb,
-                  (void *)d.heavy_slot, (void *)d.thin_items, (void *)d.tile_thin, (void *)d.long_slot,
+                  (void *)d.thin_items, (void *)d.tile_thin, (void *)d.long_slot,
                   (void *)d.mix_items, (void *)d.mix_heavy_slot, (void *)d.mix_heavy_pb, (void *)d.mix_grp,
                   (void *)d.mix_heavy_gb})
     dev_free(p);
@@ -189,9 +193,19 @@ ctc_status ensure_quirk_ciss(ctc_model *m, uint32_t mode, uint32_t flags) {
 // Piece tables for spans of `span_tiles` tiles (see k_als_gram).  Piece ids
 // run over (span, slot) pairs in order, so piece(span, slot) = slot +
 // span_off[span] with span_off[span] = pieces before the span - its first slot.
-ctc_status ensure_pieces(ctc_model *m, uint32_t mode, uint32_t span_tiles) {
+// The tables of two span lengths are kept: below 8.4M nonzeros ALS's default is
+// shorter than CCD++'s, and with one set a program that ran both in turn built and
+// uploaded it at every switch (an ALS sweep and a CCD++ epoch of 1M nonzeros, R = 16,
+// in turn: 2.92 ms, now 2.11; alone the two take 0.42 and 1.65).
+ctc_status ensure_pieces(ctc_model *m, uint32_t mode, uint32_t span_tiles, const PieceTables **out) {
   DevCiss &d = m->ciss[mode];
-  if (d.span_tiles == span_tiles && d.span_off) return CTC_OK;
+  for (uint32_t i = 0; i < 2; ++i)
+    if (d.pieces[i].span_tiles == span_tiles) {
+      d.pieces_last = i;
+      *out = &d.pieces[i];
+      return CTC_OK;
+    }
+  Prof built(m->ctx, "piece_tables");
   const uint64_t nspans = (d.ntiles + span_tiles - 1) / span_tiles;
   std::vector<uint32_t> off(nspans), pb(d.dlength + 1);
   uint64_t base = 0;
@@ -227,28 +241,25 @@ ctc_status ensure_pieces(ctc_model *m, uint32_t mode, uint32_t span_tiles) {
     }
   }
   gb[d.dlength] = (uint32_t)gpiece.size();
-  dev_free(d.span_off);
-  dev_free(d.slot_pb);
-  dev_free(d.grp_piece);
-  dev_free(d.grp_n);
-  dev_free(d.slot_gb);
-  dev_free(d.heavy_slot);
-  d.span_off = d.slot_pb = d.grp_piece = d.grp_n = d.slot_gb = d.heavy_slot = nullptr;
+  PieceTables &t = d.pieces[d.pieces[d.pieces_last].span_tiles ? 1 - d.pieces_last : d.pieces_last];
+  free_pieces(t);
   hipStream_t st = m->ctx->stream;
-  CTC_TRY(upload(&d.span_off, off.data(), nspans, st));
-  CTC_TRY(upload(&d.slot_pb, pb.data(), d.dlength + 1, st));
-  d.nheavy_slot = heavy.size();
-  CTC_TRY(upload(&d.heavy_slot, heavy.data(), heavy.size(), st));
-  d.ngroups = gpiece.size();
-  if (d.ngroups) {
-    CTC_TRY(upload(&d.grp_piece, gpiece.data(), d.ngroups, st));
-    CTC_TRY(upload(&d.grp_n, gn.data(), d.ngroups, st));
-    CTC_TRY(upload(&d.slot_gb, gb.data(), d.dlength + 1, st));
+  CTC_TRY(upload(&t.span_off, off.data(), nspans, st));
+  CTC_TRY(upload(&t.slot_pb, pb.data(), d.dlength + 1, st));
+  t.nheavy_slot = heavy.size();
+  CTC_TRY(upload(&t.heavy_slot, heavy.data(), heavy.size(), st));
+  t.ngroups = gpiece.size();
+  if (t.ngroups) {
+    CTC_TRY(upload(&t.grp_piece, gpiece.data(), t.ngroups, st));
+    CTC_TRY(upload(&t.grp_n, gn.data(), t.ngroups, st));
+    CTC_TRY(upload(&t.slot_gb, gb.data(), d.dlength + 1, st));
   }
   CTC_HIP(hipStreamSynchronize(st));
-  d.span_tiles = span_tiles;
-  d.nspans = nspans;
-  d.npieces = base;
+  t.span_tiles = span_tiles;  // from here on it is found
+  t.nspans = nspans;
+  t.npieces = base;
+  d.pieces_last = (uint32_t)(&t - d.pieces);
+  *out = &t;
   return CTC_OK;
 }
 
@@ -616,7 +627,8 @@ extern "C" ctc_status ctc_model_prepare(ctc_model *m, const ctc_options *o) {
   for (uint32_t md = 0; md < m->nmodes; ++md) {
     CTC_TRY(ensure_ciss(m, md));
     if (o->algorithm == CTC_ALS) {
-      CTC_TRY(ensure_pieces(m, md, als_span_tiles(o, m->ciss[md].nnz)));
+      const PieceTables *t = nullptr;
+      CTC_TRY(ensure_pieces(m, md, als_span_tiles(o, m->ciss[md].nnz), &t));
       if (als_uses_thin(o, m->rank)) CTC_TRY(ensure_thin(m, md));
     }
   }
@@ -632,34 +644,36 @@ static ctc_status als_mode_plain(ctc_model *m, uint32_t mode, const ctc_options 
   if (R > 64) return fail(CTC_ERR_UNSUPPORTED, "the span ALS kernels support ranks up to 64 (got %u)", R);
   CTC_TRY(ensure_ciss(m, mode));
   const uint32_t S = als_span_tiles(o, m->ciss[mode].nnz);
-  CTC_TRY(ensure_pieces(m, mode, S));
+  const PieceTables *t = nullptr;
+  CTC_TRY(ensure_pieces(m, mode, S, &t));
   const bool use_thin = als_uses_thin(o, R);
   if (use_thin) CTC_TRY(ensure_thin(m, mode));
   DevCiss &d = m->ciss[mode];
   const bool thin = use_thin && d.nthin > 0;
   const size_t psz = (size_t)R * R + R;
-  CTC_TRY(ensure_scratch(m, (d.npieces + d.ngroups) * psz * sizeof(double)));
+  CTC_TRY(ensure_scratch(m, (t->npieces + t->ngroups) * psz * sizeof(double)));
   hipStream_t st = m->ctx->stream;
   double *pieces = (double *)m->scratch;
-  double *gsum = pieces + d.npieces * psz;
+  double *gsum = pieces + t->npieces * psz;
   CissArgs ca = ciss_args(d);
   FactorArgs fa = rel_factors(m->F, m->nmodes, mode);
   {
     Prof p(m->ctx, "als_gram");
-    CTC_HIP(launch_als_gram(st, ca, fa, (int)m->nmodes, (int)R, S, d.nspans, d.span_off,
+    CTC_HIP(launch_als_gram(st, ca, fa, (int)m->nmodes, (int)R, S, t->nspans, t->span_off,
                             thin ? d.tile_thin : nullptr, pieces, block_of(o)));
   }
   // rows absent from the directory become 0 (SG/als.cu:699 zeroes the factor);
   // the solve writes every other row
   if (d.dlength < m->dims[mode]) CTC_HIP(launch_fill(st, m->F[mode], m->dims[mode] * R, 0.f));
-  if (d.ngroups) {
+  if (t->ngroups) {
     Prof p(m->ctx, "als_reduce");
-    CTC_HIP(launch_piece_reduce(st, pieces, d.grp_piece, d.grp_n, d.ngroups, (int)R, gsum));
+    CTC_HIP(launch_piece_reduce(st, pieces, t->grp_piece, t->grp_n, t->ngroups, (int)R, gsum));
   }
   {
     Prof p(m->ctx, "als_solve");
-    CTC_HIP(launch_als_solve(st, pieces, d.slot_pb, d.ngroups ? gsum : nullptr, d.slot_gb, d.directory,
-                             thin ? d.long_slot : nullptr, thin ? d.nlong_slot : d.dlength, (int)R, o->lambda, o->refine != 0, m->F[mode], m->dflag));
+    CTC_HIP(launch_als_solve(st, pieces, t->slot_pb, t->ngroups ? gsum : nullptr, t->slot_gb, d.directory,
+                             thin ? d.long_slot : nullptr, thin ? d.nlong_slot : d.dlength, (int)R, o->lambda,
+                             o->refine != 0, m->F[mode], m->dflag));
   }
   if (thin) {
     Prof p(m->ctx, "als_thin");

@@ -38,3 +38,40 @@ def test_autotune_times_the_default_als_kernels():
     n = launches(ctx, "als_gram", "als_rows_items", "als_rows_chunks")
     rows = n["als_rows_items"] + n["als_rows_chunks"] > 0
     assert rows == (r["tile_len"] == 0) and rows != (n["als_gram"] > 0)
+
+
+def test_als_and_ccd_keep_their_piece_tables():
+    """ALS and CCD++ run in turn on one model, whose default spans differ, build
+    their tables once each; a third span length replaces one of the two, and every
+    update gives what a model of its own gives."""
+    say("[piece tables]")
+    ctx = ct.Context(0)
+    dims, R = (4000, 300, 60), 16
+    t, _ = ct.synth(dims, 200_000, zipf=(1.0, 0.5, 0.0), test_fraction=0.0, seed=4)
+    rng = np.random.default_rng(62)
+    F = [rng.uniform(-1, 1, (d, R)).astype(np.float32) for d in t.dims]
+    als, ccd = (ct.Options(algorithm=a, rank=R, lambda_=0.05) for a in (ct.ALS, ct.CCD))
+    wide = ct.Options(algorithm=ct.ALS, rank=R, lambda_=0.05, tile_len=512)
+
+    def step(m, opt):
+        m.set_factors(F)
+        if opt is ccd:
+            m.ccd_epoch(opt)
+        else:
+            for k in range(3):
+                m.als_mode_update(k, opt)
+        return m.factors()
+
+    alone = {}
+    for opt in (als, ccd, wide):
+        alone[id(opt)] = step(ct.Model(ctx, t, None, None, rank=R), opt)
+    m = ct.Model(ctx, t, None, None, rank=R)
+    ctx.set_profiling(True)
+    built = []
+    for opt in (als, ccd, als, ccd, wide, ccd, wide, als, ccd, als):
+        ctx.reset_stats()
+        for a, b in zip(step(m, opt), alone[id(opt)]):
+            np.testing.assert_array_equal(a, b)
+        built.append(ctx.kernel_stats("piece_tables")[0])
+    say(f"  built {built}")
+    assert built == [3, 3, 0, 0, 3, 0, 0, 3, 3, 0]
