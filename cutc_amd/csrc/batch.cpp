@@ -342,8 +342,8 @@ static std::vector<uintptr_t> graph_key_of(ctc_batch *b, const ctc_options *o, u
       k.push_back((uintptr_t)pt.span_off);
       k.push_back((uintptr_t)pt.slot_gb);
       k.push_back((uintptr_t)(als_uses_thin(&t, c.rank) ? d.thin_items : nullptr));
-      k.push_back((uintptr_t)d.mix_items);
-      k.push_back((uintptr_t)d.mix_chunk);
+      k.push_back((uintptr_t)d.rows[d.rows_last].items);
+      k.push_back((uintptr_t)d.rows[d.rows_last].chunk);
       k.push_back((uintptr_t)c.model->F[md]);
       k.push_back((uintptr_t)c.model->Fbf[md]);
     }

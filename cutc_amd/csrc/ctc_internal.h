@@ -76,6 +76,15 @@ struct PieceTables {
   uint32_t *slot_gb = nullptr;    // dlength + 1: groups of slot s (empty for light slots)
 };
 
+// Work items of the row-fused ALS (see kernels_mixed.h) for rows cut at chunk nonzeros
+struct RowItems {
+  uint32_t chunk = 0;  // 0: not built
+  uint64_t nitems = 0, nheavy = 0, nparts = 0, nthin = 0, nthin16 = 0, ndual = 0, ndual48 = 0, ngroups = 0;
+  uint4 *items = nullptr;
+  uint32_t *heavy_slot = nullptr, *heavy_pb = nullptr, *heavy_gb = nullptr;
+  uint2 *grp = nullptr;  // long rows' partial groups {first partial, count}
+};
+
 // Device copy of one mode's CISS and the tables built over it
 struct DevCiss {
   uint32_t nmodes = 0, mode = 0;
@@ -97,13 +106,9 @@ struct DevCiss {
   uint4 *thin_items = nullptr;
   uint64_t *tile_thin = nullptr;
   uint32_t *long_slot = nullptr;
-  // BF16-operand ALS work items (see kernels_mixed.h) for rows cut at mix_chunk nonzeros
-  uint32_t mix_chunk = 0;
-  uint64_t mix_nitems = 0, mix_nheavy = 0, mix_nparts = 0, mix_nthin = 0, mix_nthin16 = 0, mix_ndual = 0, mix_ndual48 = 0,
-           mix_ngroups = 0;
-  uint4 *mix_items = nullptr;
-  uint32_t *mix_heavy_slot = nullptr, *mix_heavy_pb = nullptr, *mix_heavy_gb = nullptr;
-  uint2 *mix_grp = nullptr;  // long rows' partial groups {first partial, count}
+  // work items of two chunk lengths: FP32 and mixed updates have each their own
+  RowItems rows[2];
+  uint32_t rows_last = 0;  // the one asked for last
   // host copies needed by the piece-table builder
   std::vector<uint32_t> h_tile_slot;
   std::vector<uint64_t> h_tile_mask;
@@ -251,6 +256,7 @@ ctc_status ccd_epoch_jacobi(ctc_model *m, const ctc_options *o, uint32_t start);
 // one row-fused ALS mode update (ranks 32, 64, 128), enqueued on the model's
 // stream: BF16-operand Gram (bf16) or FP64-accumulated Gram from FP32 factors
 ctc_status als_mode_rows(ctc_model *m, uint32_t mode, const ctc_options *o, bool bf16);
+void free_row_items(RowItems &t);
 // everything als_mode_rows allocates or uploads, for all modes
 ctc_status als_rows_prepare(ctc_model *m, const ctc_options *o, bool bf16);
 // which FP32 ALS kernels a model of rank R uses under these options

@@ -160,10 +160,9 @@ static void free_pieces(PieceTables &t) {
 static void free_dev_ciss(DevCiss &d) {
   for (PieceTables &t : d.pieces) free_pieces(t);
   for (int s = 0; s < 3; ++s) dev_free(d.oidx[s]);
+  for (RowItems &t : d.rows) free_row_items(t);
   for (void *p : {(void *)d.vals, (void *)d.tile_slot, (void *)d.tile_mask, (void *)d.directory, (void *)d.rowptr,
-                  (void *)d.thin_items, (void *)d.tile_thin, (void *)d.long_slot,
-                  (void *)d.mix_items, (void *)d.mix_heavy_slot, (void *)d.mix_heavy_pb, (void *)d.mix_grp,
-                  (void *)d.mix_heavy_gb})
+                  (void *)d.thin_items, (void *)d.tile_thin, (void *)d.long_slot})
     dev_free(p);
   d = DevCiss();
 }

@@ -75,3 +75,35 @@ def test_als_and_ccd_keep_their_piece_tables():
         built.append(ctx.kernel_stats("piece_tables")[0])
     say(f"  built {built}")
     assert built == [3, 3, 0, 0, 3, 0, 0, 3, 3, 0]
+
+
+def test_fp32_and_mixed_keep_their_row_items():
+    """FP32 and mixed row-fused updates run in turn on one model, whose chunks of long
+    rows differ, list their rows once each; a third chunk length replaces one of the
+    two, and every update gives what a model of its own gives."""
+    say("[row items]")
+    ctx = ct.Context(0)
+    R = 64
+    t, _ = ct.synth((3000, 20, 600), 150_000, zipf=(1.0, 0.5, 0.0), test_fraction=0.0, seed=4)
+    rng = np.random.default_rng(63)
+    F = [rng.uniform(-1, 1, (d, R)).astype(np.float32) for d in t.dims]
+    full, mixed, short = (ct.Options(algorithm=ct.ALS, rank=R, lambda_=0.05, **k)
+                          for k in ({}, {"precision": ct.PREC_MIXED}, {"tile_len": 96}))
+
+    def step(m, opt):
+        m.set_factors(F)
+        for k in range(3):
+            m.als_mode_update(k, opt)
+        return m.factors()
+
+    alone = {id(opt): step(ct.Model(ctx, t, None, None, rank=R), opt) for opt in (full, mixed, short)}
+    m = ct.Model(ctx, t, None, None, rank=R)
+    ctx.set_profiling(True)
+    built = []
+    for opt in (full, mixed, full, mixed, short, mixed, short, full, mixed, full):
+        ctx.reset_stats()
+        for a, b in zip(step(m, opt), alone[id(opt)]):
+            np.testing.assert_array_equal(a, b)
+        built.append(ctx.kernel_stats("row_items")[0])
+    say(f"  built {built}")
+    assert built == [3, 3, 0, 0, 3, 0, 0, 3, 3, 0]
