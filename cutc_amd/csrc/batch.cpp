@@ -17,6 +17,7 @@
 // one block per range.
 #include <algorithm>
 #include <cmath>
+#include <cstring>
 #include <vector>
 
 #include "ctc_internal.h"
@@ -327,8 +328,9 @@ static ctc_status enqueue_run(ctc_batch *b, const ctc_options *o, uint32_t iters
 }
 
 static std::vector<uintptr_t> graph_key_of(ctc_batch *b, const ctc_options *o, uint32_t iters) {
-  std::vector<uintptr_t> k{iters, (uintptr_t)std::llround(o->lambda * 1e12), (uintptr_t)o->refine,
-                           (uintptr_t)o->precision};
+  uint64_t lambda;  // as it is: rounded, two values could share a graph
+  std::memcpy(&lambda, &o->lambda, sizeof lambda);
+  std::vector<uintptr_t> k{iters, (uintptr_t)lambda, (uintptr_t)o->refine, (uintptr_t)o->precision};
   for (auto &c : b->cls) {
     const ctc_options t = class_options(c, o);
     k.push_back(t.tile_len);

@@ -107,3 +107,33 @@ def test_fp32_and_mixed_keep_their_row_items():
         built.append(ctx.kernel_stats("row_items")[0])
     say(f"  built {built}")
     assert built == [3, 3, 0, 0, 3, 0, 0, 3, 3, 0]
+
+
+@pytest.mark.parametrize("first,then", [(1e7, 4e7), (1e-13, 0.0)], ids=["large", "tiny_then_none"])
+def test_batch_graph_of_another_lambda(first, then):
+    """A batch's captured run is not replayed for another ridge weight, however large or
+    small the two are; without one, short rows stay refused."""
+    say(f"[batch graph lambda] {first} then {then}")
+    ctx = ct.Context(0)
+    R = 32
+    t, _ = ct.synth((6000, 300, 200), 40_000, test_fraction=0.0, seed=5)
+    rng = np.random.default_rng(64)
+    F = [rng.uniform(-1, 1, (d, R)).astype(np.float32) for d in t.dims]
+    b = ct.Batch(ctx, [t], [None], [R])
+
+    def run(lam, graph):
+        for k, f in enumerate(F):
+            b.set_factor(0, k, f)
+        try:
+            b.als(ct.Options(algorithm=ct.ALS, rank=R, lambda_=lam), iters=1, graph=graph)
+        except ct.CtcError as e:
+            return e.status
+        return [b.factor(0, k) for k in range(3)]
+
+    run(first, True)
+    got, want = run(then, True), run(then, False)
+    if then == 0.0:
+        assert got == want == 7
+    else:
+        for a, e in zip(got, want):
+            np.testing.assert_array_equal(a, e)
