@@ -137,3 +137,25 @@ def test_batch_graph_of_another_lambda(first, then):
     else:
         for a, e in zip(got, want):
             np.testing.assert_array_equal(a, e)
+
+
+@pytest.mark.parametrize("nnz,kw,rows", [(3_990_000, {}, False), (4_010_000, {}, True), (4_010_000, {"refine": 1}, False),
+                                         (4_010_000, {"tile_len": 1024}, False), (4_010_000, {"lambda_": 0.0}, False),
+                                         (30_000, {"als_kernel": ct.ALS_ROWS}, True),
+                                         (4_010_000, {"als_kernel": ct.ALS_SPANS}, False)],
+                         ids=["below", "above", "refined", "tile_len", "no_lambda", "rows_asked", "spans_asked"])
+def test_als_rank_32_family(nnz, kw, rows):
+    """Which kernels the rank-32 ALS update runs on either side of the size rule and
+    where an option decides."""
+    say(f"[als rank 32 family] nnz={nnz} {kw}")
+    ctx = ct.Context(0)
+    t, _ = ct.synth((300, 250, 200), nnz, test_fraction=0.0, seed=9)
+    m = ct.Model(ctx, t, None, None, rank=32)
+    rng = np.random.default_rng(65)
+    m.set_factors([rng.uniform(-1, 1, (d, 32)).astype(np.float32) for d in t.dims])
+    ctx.set_profiling(True)
+    ctx.reset_stats()
+    m.als_mode_update(0, ct.Options(**{**dict(algorithm=ct.ALS, rank=32, lambda_=0.05), **kw}))
+    n = launches(ctx, "als_gram", "als_rows_items", "als_rows_chunks")
+    say(f"  {n}")
+    assert (n["als_rows_items"] + n["als_rows_chunks"] > 0) == rows and (n["als_gram"] == 0) == rows

@@ -294,3 +294,83 @@ def test_batch_rmse_of_many_problems(ctx, R, count, longest):
         tr, te = b.rmse()
         np.testing.assert_allclose(tr, wt, rtol=1e-6, atol=4e-6)
         np.testing.assert_allclose(te, we, rtol=1e-6, atol=4e-6)
+
+
+@pytest.mark.parametrize("R,modes,above", [(8, 3, False), (8, 3, True), (16, 3, True), (32, 3, False), (32, 3, True), (32, 4, True)])
+def test_sgd_walk_lane_shapes(ctx, R, modes, above):
+    """The FP32 SGD walk just below and just above the number of walkers from which a
+    lane holds four elements of a row, with spans of 4 nonzeros, against the oracle's
+    schedule in 64 bits at the parity tests' bar (1e-5)."""
+    import oracle as O
+    walkers = 2048 * 256 // R + (1 if above else -1)
+    nnz = 4 * walkers - 3
+    dims = (9001, 120, 70) if modes == 3 else (9001, 60, 40, 9)
+    say(f"[sgd lane shapes] R={R} dims={dims} walkers={walkers}")
+    t, ind, vals = coo(dims, nnz, 81)
+    rng = np.random.default_rng(82)
+    F = [(0.5 * rng.uniform(-1, 1, (d, R))).astype(np.float32) for d in dims]
+    F64 = [f.astype(np.float64) for f in F]
+    oc = O.Coo(ind, vals, dims)
+    O.sgd_sync_epoch(oc, F64, 1e-3, 0.05, 4, 2, 60_000, order=O.mode_order(oc, 0)[0], nthreads=4)
+    m = ct.Model(ctx, t, None, None, rank=R)
+    m.set_factors(F)
+    m.sgd_epoch(ct.Options(algorithm=ct.SGD, rank=R, lambda_=0.05, sgd_scale=1.0, tile_len=4, sgd_substep=2,
+                           sgd_hot_rows=60_000), lr=1e-3)
+    for k, f in enumerate(F64):
+        assert np.linalg.norm(m.factor(k) - f) < 1e-5 * np.linalg.norm(f), k
+
+
+@pytest.mark.parametrize("R,dims,nnz", [(128, (700, 300, 60), 4096 * 2 * 64 + 5000), (128, (2, 900, 600), 4096 * 2 * 96 + 77),
+                                        (64, (900, 120, 40, 9), 4096 * 4 * 64 + 1), (32, (1500, 300, 60), 4096 * 8 * 96 + 33)],
+                         ids=["r128_span64", "r128_span96_long", "r64_4way_span64", "r32_span96"])
+def test_walk_spans_of_several_chunks(ctx, R, dims, nnz):
+    """MTTKRP, the gradient with both regularisers and the training loss where the
+    spans are longer than the 32 nonzeros of a small tensor (64 and 96: several chunks
+    even at R = 128, where a chunk is 32), with rows inside a span, over its chunks,
+    over walkers and over workgroups, against 64 bits at the parity tests' bars
+    (1e-5, loss 1e-6)."""
+    import torch
+    say(f"[walk chunks] R={R} dims={dims} nnz={nnz}")
+    t, ind, vals = coo(dims, nnz, 91)
+    rng = np.random.default_rng(92)
+    F = [rng.uniform(-1, 1, (d, R)).astype(np.float32) for d in dims]
+    m = ct.Model(ctx, t, None, None, rank=R)
+    m.set_factors(F)
+    di, dv = [torch.from_numpy(i.astype(np.int64)).cuda() for i in ind], torch.from_numpy(vals.astype(np.float32)).cuda().double()
+    D = [torch.from_numpy(f).cuda() for f in F]
+    D64 = [f.double() for f in D]
+
+    def others(mode):
+        h = torch.ones(nnz, R, dtype=torch.float64, device="cuda")
+        for k, f in enumerate(D64):
+            if k != mode:
+                h *= f[di[k]]
+        return h
+
+    e = dv - (others(0) * D64[0][di[0]]).sum(1)
+    sq = float((e * e).sum())
+    assert m.evaluate(0.0)["loss"] == pytest.approx(sq, rel=1e-6)
+    grads = {}
+    for per_occ in (False, True):
+        G = [torch.full_like(f, 7.0) for f in D]
+        torch.cuda.synchronize()
+        loss = m.grad_device([f.data_ptr() for f in D], [g.data_ptr() for g in G], 0.3, per_occ)
+        cnt = [torch.bincount(i, minlength=f.shape[0]).double()[:, None] if per_occ else 1.0 for i, f in zip(di, D64)]
+        want = 0.5 * sq + sum(0.15 * float((c * f * f).sum()) for c, f in zip(cnt, D64))
+        assert loss == pytest.approx(want, rel=1e-6)
+        grads[per_occ] = [(g.double(), 0.3 * c * f) for g, c, f in zip(G, cnt, D64)]
+    for mode in range(len(dims)):
+        h = others(mode)
+        order = torch.argsort(di[mode], stable=True)
+        lens = torch.bincount(di[mode], minlength=dims[mode])
+
+        def row_sums(w):
+            return torch.segment_reduce((h * w[:, None])[order], "sum", lengths=lens, unsafe=True)
+
+        want = row_sums(dv)
+        got = torch.from_numpy(m.mttkrp(mode)).cuda().double()
+        assert float((got - want).norm()) < 1e-5 * float(want.norm()), mode
+        adjoint = row_sums(e)
+        for per_occ, g in grads.items():
+            got, want = g[mode][0], g[mode][1] - adjoint
+            assert float((got - want).norm()) < 1e-5 * float(want.norm()), (mode, per_occ)
