@@ -259,12 +259,17 @@ ctc_status als_mode_rows(ctc_model *m, uint32_t mode, const ctc_options *o, bool
 void free_row_items(RowItems &t);
 // everything als_mode_rows allocates or uploads, for all modes
 ctc_status als_rows_prepare(ctc_model *m, const ctc_options *o, bool bf16);
-// which FP32 ALS kernels a model of rank R uses under these options
+// Whether a model of rank R takes the row-fused ALS kernels under these options.
 //
-// By default rank 32 takes them from kRowsNnz nonzeros on, where the workgroups'
-// chunks of 1024 nonzeros fill the chip: a sweep of 20M nonzeros 3.36 ms (spans
-// 3.87), 3.7M 0.81 (0.89), but 0.86M 0.48 (0.40), 0.1M 0.41 (0.29).  lambda > 0
-// and no refinement or tile length asked for, as in als_uses_thin below.
+// By default rank 32 takes them from kRowsNnz nonzeros on: a workgroup's chunk of a
+// long row is 1024 nonzeros, and below about 4M there are too few of them for the
+// chip.  Sweeps of ratings (480K x 18K x 2K, Zipf), spans with the short rows in
+// dual form against row-fused, ms: 1.5M nonzeros 0.66 / 0.84, 3M 1.02 / 1.13, 3.9M
+// 1.20 / 1.24, 4.2M 1.31 / 1.26, 20M 3.73 / 3.29.  Other shapes cross elsewhere:
+// uniform rows of 33, 2M nonzeros 1.50 / 1.39, two million rows of 3, 6M nonzeros
+// 37 / 4.0 (spans without the dual form), rows of 40 alike, one workgroup's solve
+// each, level: 6M 3.56 / 3.61, 12M 6.96 / 7.05, 20M 11.8 / 11.6.  lambda > 0 and no
+// refinement or tile length asked for, as in als_uses_thin below.
 constexpr uint64_t kRowsNnz = 4000000;
 inline bool als_uses_rows(const ctc_options *o, uint32_t R, uint64_t nnz) {
   if (o->precision == CTC_PREC_MIXED || o->als_kernel == CTC_ALS_ROWS) return true;
@@ -275,7 +280,7 @@ inline bool als_uses_rows(const ctc_options *o, uint32_t R, uint64_t nnz) {
 // row of at most 16 nonzeros is an n x n system in place of the 32 x 32 one and of
 // its 8 KB piece.  Only with lambda > 0 (without it such a row is singular, and
 // is reported), the default kernel choice and no refinement.  Span sweep of 20M
-// nonzeros with 375K such rows 3.74 ms, without this 5.82 ms.
+// nonzeros with 375K such rows 3.73 ms, without this 5.87 ms.
 inline bool als_uses_thin(const ctc_options *o, uint32_t R) {
   return R == 32 && o->precision == CTC_PREC_FP32 && o->als_kernel == CTC_ALS_AUTO && !o->refine && o->lambda > 0.0;
 }

@@ -788,11 +788,11 @@ __global__ void __launch_bounds__(256) k_sgd_fold(SettleArgs a) {
 // loss_part (the training loss of tc_loss_sq, SG/completion.c:166-189).
 // Bound by the gathers of the other modes' rows: the rows of four nonzeros are
 // gathered together, the next chunk's indices one chunk ahead (44 registers at
-// N = 3).  MTTKRP of 8M nonzeros at R = 32 117 us per mode, 2.1 times the
-// indices, values and rows a CU can take from its cache at 64 B per clock; with
-// an atomic row per walker and row 260 us, 283 us with the gathers in fours
-// alone.  Two or eight nonzeros at a time: 123 / 134 us.  The adjoint of 20M
-// nonzeros of a 4-way tensor: 510 us per mode (1100 us).
+// N = 3).  MTTKRP of 8M nonzeros at R = 32 132 us per mode (117 us with spans of
+// 256, see walk_span: 2.1 times the indices, values and rows a CU can take from
+// its cache at 64 B per clock); with an atomic row per walker and row 258 us.  The
+// adjoint of 20M nonzeros of a 4-way tensor 495 us per mode (1087 us).  Two or
+// eight nonzeros at a time: 128 / 145 us and 525 / 504 us.
 // ==========================================================================
 enum : int { kWalkMttkrp = 0, kWalkAdjoint = 1, kWalkJacobi = 2, kWalkLoss = 3 };
 
@@ -1004,12 +1004,12 @@ __global__ void __launch_bounds__(256) k_mttkrp(CissArgs c, FactorArgs fa, uint3
 // registers; block (bi, bj) of G (bi >= bj) takes A = h[bi], B = h[bj].
 // FP64 accumulation keeps the normal equations within 1e-5 of an FP64
 // reference even when (G + lambda I) is poorly conditioned.
-// ==========================================================================
-typedef double doublex4 __attribute__((ext_vector_type(4)));
-
 //
 // tile_thin (null: none) marks the nonzeros of rows that are solved in their
 // dual form: the walk passes over them and writes no piece for their rows.
+// ==========================================================================
+typedef double doublex4 __attribute__((ext_vector_type(4)));
+
 template <int R, int N>
 __device__ __forceinline__ void als_gram_walk(const CissArgs &c, const FactorArgs &fa, uint32_t span_tiles,
                                               uint64_t nspans, const uint32_t *span_off, const uint64_t *tile_thin,
@@ -1154,9 +1154,10 @@ __device__ __forceinline__ void als_gram_walk(const CissArgs &c, const FactorArg
 
 // Occupancy: at R <= 32 the walk (with its one-step gather lookahead) is held
 // to 6 waves per SIMD, about 80 registers; at R = 64, and at R = 32 with four
-// modes (which would spill at 80), it keeps the compiler's default.  Measured on the 100M-nonzero tensor at R = 32: 4.56 ms per mode
-// without lookahead at the default occupancy, 4.27 ms without lookahead at 7
-// waves, 4.00 ms with lookahead at 6.
+// modes (which would spill at 80), it keeps the compiler's default.  Measured on
+// the 100M-nonzero tensor at R = 32: 4.56 ms per mode without lookahead at the
+// default occupancy, 4.27 ms without lookahead at 7 waves, 4.00 ms with lookahead
+// at 6.
 template <int R, int N>
 __global__ void __launch_bounds__(256, 6) k_als_gram(CissArgs c, FactorArgs fa, uint32_t span_tiles,
                                                      uint64_t nspans, const uint32_t *span_off,
@@ -1166,7 +1167,7 @@ __global__ void __launch_bounds__(256, 6) k_als_gram(CissArgs c, FactorArgs fa, 
 template <int R, int N>
 __global__ void __launch_bounds__(256) k_als_gram_wide(CissArgs c, FactorArgs fa, uint32_t span_tiles,
                                                        uint64_t nspans, const uint32_t *span_off,
-                                                     const uint64_t *tile_thin, double *pieces) {
+                                                       const uint64_t *tile_thin, double *pieces) {
   als_gram_walk<R, N>(c, fa, span_tiles, nspans, span_off, tile_thin, pieces);
 }
 
@@ -1188,8 +1189,9 @@ __device__ inline int tri_row(int t) {
 // Heavy slots (more pieces than the solve's serial sum should take) are first
 // reduced in fixed groups of consecutive pieces.  A thread owns one element of
 // a group's sum (blockIdx.y: 256 elements of the piece), eight pieces' loads in
-// flight, added in piece order: 20M nonzeros at R = 32, 32 us
-// per mode (218 us with one 64-thread workgroup per group and a load at a time).
+// flight, added in piece order: the rank-32 class of a batch (1.8M nonzeros) 41 us per
+// mode, 1M nonzeros at R = 16 7 us; on the span kernels 20M nonzeros at R = 32 take 32 us
+// (218 us with one 64-thread workgroup per group and a load at a time).
 template <int R>
 __global__ void __launch_bounds__(256) k_piece_reduce(const double *pieces, const uint32_t *grp_piece,
                                                       const uint32_t *grp_n, double *gsum) {
@@ -1481,8 +1483,9 @@ __global__ void __launch_bounds__(256) k_eval_coo(CooArgs c, FactorArgs fa, int 
 // load per lane, the walkers of a segment's blocks take its nonzeros in turn,
 // and the FP32 prediction is summed over the walker's lanes.  A long segment is
 // shared by several blocks (eval_seg_blocks): with one block per segment and a
-// lane per nonzero, 24 problems of 0.3M nonzeros (six per rank) took 24 ms of an
-// 80 ms pass of ten iterations, which 64 blocks per segment made 56 ms.
+// lane per nonzero, the RMSE of 24 problems of 0.3M nonzeros (six per rank) took
+// 24 ms; with 64 blocks per segment its longest kernel, of the six at rank 64, takes
+// 0.53 ms.
 template <int R, int N, bool CISS>
 __global__ void __launch_bounds__(256) k_eval_seg(CissArgs c, CooArgs co, FactorArgs fa, const uint64_t *seg,
                                                   double *part) {
@@ -1770,9 +1773,13 @@ hipError_t launch_loss_walk(hipStream_t st, const CissArgs &c, const FactorArgs 
 
 uint64_t mttkrp_walkers_per_block(int R, unsigned block) { return (uint64_t)(block / 64) * (64 / (R / 4)); }
 
-// Spans of 256 where they fill the chip (MTTKRP of 8M nonzeros at R = 32: 117 us,
-// 125 / 131 / 131 us with 128 / 64 / 32), down to 32 for smaller tensors: about
-// 4096 waves (the loss of 1M nonzeros at R = 16: 14 us, 89 us with 256).
+// Spans of 256 where they fill the chip, down to 32 for smaller tensors: about 4096
+// waves (the loss of 1M nonzeros at R = 16: 14 us, 89 us with 256).  A span between
+// two powers of two costs: MTTKRP of 8M nonzeros at R = 32 132 us with the 224 it
+// gets, 117 / 124 / 123 / 133 us with 256 / 128 / 64 / 32, the adjoint of 4M
+// nonzeros 92 us with 96, 79 us with 64.  Rounding down to the power of two would take
+// that back but leaves more partial sums of a hot row to the FP32 atomics: at one
+// size the error of the sums against 64 bits grew from 9e-8 to 1.2e-7 of their norm.
 uint32_t walk_span(uint64_t nnz, int R) {
   const uint64_t per = nnz / (4096 * (uint64_t)(256 / R)) / 32 * 32;
   return (uint32_t)(per < 32 ? 32 : per > 256 ? 256 : per);
@@ -1794,10 +1801,10 @@ hipError_t launch_als_gram(hipStream_t st, const CissArgs &c, const FactorArgs &
   do {                                                                                                    \
     if (nmodes == 3)                                                                                      \
       hipLaunchKernelGGL((k_als_gram<RR, 3>), dim3(grid), dim3(block), 0, st, c, f, span_tiles, nspans, \
-                         span_off, tile_thin, pieces);                                                               \
+                         span_off, tile_thin, pieces);                                                    \
     else                                                                                                  \
       hipLaunchKernelGGL((k_als_gram<RR, 4>), dim3(grid), dim3(block), 0, st, c, f, span_tiles, nspans, \
-                         span_off, tile_thin, pieces);                                                               \
+                         span_off, tile_thin, pieces);                                                    \
   } while (0)
   switch (R) {
     case 8: CTC_GRAM(8); break;

@@ -19,10 +19,10 @@
 //
 // Reductions.  One wave walks a span of tiles, one lane per nonzero.  Row
 // sums inside a tile use a segmented inclusive scan that takes each lane's
-// distance to its row's start from the tile mask; the row still open at the end of a tile is carried in a wave-uniform
-// value into the next tile.  Completed rows are written as (num, den) pieces
-// with the same piece numbering as the ALS Gram pieces, so the per-row sums
-// have a fixed order (deterministic, no atomics).
+// distance to its row's start from the tile mask; the row still open at the end
+// of a tile is carried in a wave-uniform value into the next tile.  Completed
+// rows are written as (num, den) pieces with the same piece numbering as the ALS
+// Gram pieces, so the per-row sums have a fixed order (deterministic, no atomics).
 //
 // The three passes of a column over 20M nonzeros (480K x 18K x 2K): 137 / 173 /
 // 196 us (169 / 182 / 219 us with the whole scan on the LDS pipe and no tile in

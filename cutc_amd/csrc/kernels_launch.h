@@ -16,7 +16,7 @@ hipError_t launch_sgd(hipStream_t st, const CissArgs &c, const FactorArgs &f, co
 hipError_t launch_sgd_sync(hipStream_t st, const CissArgs &c, const FactorArgs &f, const SyncArgs &sy, int nmodes,
                            int R, uint32_t span, uint32_t sub, uint32_t s, uint32_t long_min, float step, float lam,
                            unsigned block, bool mixed);
-// nb_merge is set here; pb / fb must be prefix sums with pb[0..1] = fb[0..1] = 0
+// nb_light is set here; pb, lb and fb must be prefix sums whose first two entries are 0
 hipError_t launch_sgd_settle(hipStream_t st, SettleArgs a, int R, bool mixed);
 // out: zeros, or for the adjoint what launch_reg_rows left (lam, per_occ: its arguments)
 hipError_t launch_mttkrp(hipStream_t st, const CissArgs &c, const FactorArgs &f, int nmodes, int R,

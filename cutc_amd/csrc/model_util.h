@@ -41,6 +41,8 @@ inline uint32_t span_tiles_of(const ctc_options *o) {
 // kSpanWaves waves, because a span is one wave's serial chain.
 // k_als_gram at R = 16 with spans of 1024 nonzeros and by this rule: 20K
 // nonzeros 78 -> 8 us, 1M nonzeros 74 -> 28 us; from 8.4M nonzeros on the span is 1024.
+// A span adds a piece to the scratch: at most 16383, 138 MB at R = 32 (1M nonzeros
+// 132 MB beside their rows' own pieces, 8 MB with spans of 1024).
 constexpr uint64_t kSpanWaves = 8192;
 inline uint32_t als_span_tiles(const ctc_options *o, uint64_t nnz) {
   const uint32_t most = span_tiles_of(o);
